@@ -395,6 +395,7 @@ struct SplitPlan {
 // under `slot` (one slot per decode kernel).
 enum ResidentSlot {
   kSlotGeneric = 0, kSlotMfmaPow2, kSlotMfma, kSlotPlain, kSlotG4, kSlotPrefill, kSlotFp16G4,
+  kSlotG4One,
   kSlotCount
 };
 int64_t resident_workgroups(const void *kernel, int threads, int slot);
@@ -538,6 +539,7 @@ bool mfma_supported(const DecodeArgs &a);
 bool g4_shape(const DecodeArgs &a);
 bool g4_supported(const DecodeArgs &a);
 int64_t g4_resident();
+int64_t g4_one_chunk_resident();
 int launch_decode_g4(DecodeArgs &a, void *workspace, size_t ws_bytes, hipStream_t stream);
 // the uncompressed fp16 baseline at head_dim 128, GQA <= 4, fp16 queries
 bool fp16_g4_supported(const DecodeArgs &a);

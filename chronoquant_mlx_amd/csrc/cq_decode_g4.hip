@@ -191,6 +191,8 @@ __device__ __forceinline__ void merge_partials_g4(const DecodeArgs &a, __amdgpu_
 // folds and writes the outputs, and stores zeros over it.  Data and readiness
 // arrive in one round trip; no flag, no counter, no acknowledgement wait.
 // ---------------------------------------------------------------------------
+constexpr int kMaxFoldSplits = 64;  // one lane of a folding wave per split
+
 __device__ __forceinline__ uint4 load_rec4(__amdgpu_buffer_rsrc_t r, uint32_t off) {
   const i4_t v = __builtin_amdgcn_raw_buffer_load_b128(r, (int)off, 0, kPolicyDevice);
   return uint4{(uint32_t)v[0], (uint32_t)v[1], (uint32_t)v[2], (uint32_t)v[3]};
@@ -229,19 +231,23 @@ __device__ __forceinline__ void note_poll_timeout(const DecodeArgs &a) {
                           __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// Wave 0 of split f's workgroup folds its units; lane = (unit k of the pass,
-// split s), 2^lg >= live lanes per unit.
+// Split f's workgroup folds its units, 64 >> lg of them per wave and pass;
+// lane = (unit k of the pass, split s), 2^lg >= live lanes per unit.  The
+// passes go to the 8 waves: with 33 splits a unit fills a wave and a split
+// has two of them, which one wave polled one after the other (16385 tokens:
+// 15.7 us a call, 13.6 with a wave for each; 4097 tokens, 9 splits of 8 units:
+// 11.3 and 9.8).
 __device__ __forceinline__ void fold_records_g4(const DecodeArgs &a, int b, int h, int gn, int f,
                                                 int live) {
-  if (threadIdx.x >= 64) return;
-  const int lane = threadIdx.x;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
   const int lg = live > 1 ? 32 - __builtin_clz((uint32_t)(live - 1)) : 0;
   const int s = lane & ((1 << lg) - 1), k = lane >> lg;
   const int per_pass = 64 >> lg;
   const int nunits = kD / 8 * gn;
   const __amdgpu_buffer_rsrc_t rr = make_rsrc(a.recs, (uint32_t)kRecBytes);
   const int64_t col = (int64_t)b * a.H + h;
-  for (int j0 = 0; f + live * j0 < nunits; j0 += per_pass) {
+  for (int j0 = wave * per_pass; f + live * j0 < nunits; j0 += kWaves * per_pass) {
     const int u = f + live * (j0 + k);
     const bool valid = s < live && u < nunits;
     const uint32_t off =
@@ -325,7 +331,9 @@ __device__ __forceinline__ void wait_split_flags(const DecodeArgs &a, const uint
 // dim) element over the 8 waves with the log-sum-exp weights, then writes
 // the output (the workgroup holds the whole sequence) or stores its split
 // partial from registers and runs the split tail.
-template <typename OVal>
+// kRecs: the launch may use fold records (grid plans; the balanced instances,
+// which never do and have no registers to spare, leave their code out).
+template <bool kRecs, typename OVal>
 __device__ __forceinline__ void merge_finish_g4(const DecodeArgs &a, G4Merge &M, int b, int h,
                                                 int gn, int slot, int live, float m_run,
                                                 float l_run, OVal o_val) {
@@ -351,7 +359,8 @@ __device__ __forceinline__ void merge_finish_g4(const DecodeArgs &a, G4Merge &M,
   const int64_t bq0 = (int64_t)b * a.nq + h * a.G;
   const bool single = live == kGridLive ? a.nsplit == 1 : live == 1;
   __amdgpu_buffer_rsrc_t racc, rml;
-  if (!single && !a.recs) partial_rsrcs(a, racc, rml);
+  const bool recs = kRecs && a.recs;
+  if (!single && !recs) partial_rsrcs(a, racc, rml);
   if (hh < gn) {
     const float4 m0 = *(const float4 *)&M.m[hh][0], m1 = *(const float4 *)&M.m[hh][4];
     const float4 l0 = *(const float4 *)&M.l[hh][0], l1 = *(const float4 *)&M.l[hh][4];
@@ -369,7 +378,7 @@ __device__ __forceinline__ void merge_finish_g4(const DecodeArgs &a, G4Merge &M,
     }
     if (single) {
       store_any(a.out_dtype, a.out, (bq0 + hh) * kD + d, L > 0.f ? O / L : 0.f);
-    } else if (a.recs) {
+    } else if (recs) {
       const __amdgpu_buffer_rsrc_t rr = make_rsrc(a.recs, (uint32_t)kRecBytes);
       const uint32_t rec = (uint32_t)(((((int64_t)b * a.H + h) * a.nsplit + slot) * kRecUnits +
                                        hh * (kD / 8) + (d >> 3)) * (kRecWords * 4));
@@ -386,7 +395,7 @@ __device__ __forceinline__ void merge_finish_g4(const DecodeArgs &a, G4Merge &M,
   }
   if (single) return;
   if (live == kGridLive) live = grid_live(a, seq_len_of(a, b));
-  if (a.recs) {
+  if (recs) {
     phase_mark(a, 4);  // records stored (issued)
     fold_records_g4(a, b, h, gn, slot, live);
     phase_mark(a, 5);  // fold done, outputs stored (issued)
@@ -1055,7 +1064,7 @@ __global__ __launch_bounds__(kThreadsMfma) void decode_g4_kernel(DecodeArgs a) {
     // merge_finish_g4 reads (m, l) of head col from the lanes col < 4 of kg 0:
     // head col's score lanes of block 0.  Code columns: x = 1032 + c (even nb,
     // weight p s) or 1152 + 16c (odd nb, weight p s / 16).
-    merge_finish_g4(a, lds.mg, b, h, gn, slot, live, m_run, l_run, [&](int nb, int r) {
+    merge_finish_g4<!kBalanced>(a, lds.mg, b, h, gn, slot, live, m_run, l_run, [&](int nb, int r) {
       if constexpr (kDenseV) {
         // field u of dim 8col + nb entered as 2^(10 - pos) + u, code u - 4
         constexpr float kOff[8] = {1028.f, 132.f, 20.f, 516.f, 68.f, 12.f, 260.f, 36.f};
@@ -1217,7 +1226,7 @@ __global__ __launch_bounds__(kThreadsMfma) void decode_fp16_g4_kernel(DecodeArgs
   phase_mark(a, 3);  // wave 0's chunks computed (issued)
   // head hq's weight sum: its lanes col, col + 16, col + 32, col + 48
   l_run = xor32_sum(xor16_sum(l_run));
-  merge_finish_g4(a, lds.mg, b, h, gn, split, kGridLive, m_run, l_run,
+  merge_finish_g4<true>(a, lds.mg, b, h, gn, split, kGridLive, m_run, l_run,
                   [&](int nb, int r) { return acc[nb][r]; });
 }
 
@@ -1236,8 +1245,24 @@ int64_t g4_resident() {
                              kSlotG4);
 }
 
-// Uniform batches (one length bound, or one sequence) take the grid plan
-// unless the balanced partition gives its busiest workgroup fewer units;
+// Residency of the one-chunk instance: with 102 VGPRs and 41 KB of LDS two of
+// its workgroups share a CU (the pipelined instances: one).
+int64_t g4_one_chunk_resident() {
+  return resident_workgroups(reinterpret_cast<const void *>(decode_g4_kernel<false, true>),
+                             kThreadsMfma, kSlotG4One);
+}
+
+// A batch whose 512-token splits are all resident at once under the one-chunk
+// instance takes it, whatever its lengths are.  (Planned for the pipelined
+// instance's residency, 16385 tokens of 8 kv heads, 264 such splits, gave 17
+// splits of 1024 tokens, 136 workgroups for 256 CUs: 17.2 us a call against
+// 13.6.  B=1 T=32768: 17.6 against 16.2; 8 sequences of up to 4096 tokens,
+// which took the balanced partition: 22.5 against 14.5.)  Only up to 64 splits
+// per sequence, what a fold record's reader holds: 128 splits of one 65536-token
+// sequence, merged through the split-ready flags, took 28.7 us against 17.9.
+//
+// Otherwise: uniform batches (one length bound, or one sequence) take the grid
+// plan unless the balanced partition gives its busiest workgroup fewer units;
 // per-sequence lengths always take the balanced partition.  Both plan one
 // resident generation of workgroups.  Balanced: P workgroups per kv head
 // (never more than the batch has units), and a sequence spans at most
@@ -1249,8 +1274,15 @@ int launch_decode_g4(DecodeArgs &a, void *workspace, size_t ws_bytes, hipStream_
   const int64_t n_max = units_of(a.max_T);
   int64_t P = std::max((int64_t)1, resident / a.H);
   P = std::min(P, (int64_t)a.B * n_max);
-  bool balanced = a.seq_lens && a.B > 1;
-  if (!balanced) {
+  const bool dense_v = a.fbits[1] == 3;  // (K rows are INT4: mfma_supported)
+  const bool one_chunk = !dense_v && !split_tokens_override() &&
+                         n_max <= kMaxFoldSplits &&
+                         (int64_t)a.B * a.H * n_max <= g4_one_chunk_resident();
+  bool balanced = !one_chunk && a.seq_lens && a.B > 1;
+  if (one_chunk) {
+    a.nsplit = (int)n_max;
+    a.split_len = kUnit;
+  } else if (!balanced) {
     const SplitPlan g = plan_splits((int64_t)a.B * a.H, a.max_T, resident);
     const int64_t grid_units = g.split_len / kUnit;
     const int64_t bal_units = ((int64_t)a.B * n_max + P - 1) / P;
@@ -1272,9 +1304,9 @@ int launch_decode_g4(DecodeArgs &a, void *workspace, size_t ws_bytes, hipStream_
   // Fold records: every split waits for the others, so the grid must be one
   // resident generation; a folder's lanes hold up to 64 splits.
   const int64_t slots = (int64_t)a.B * a.H * a.nsplit;
-  if (!balanced && a.nsplit > 1 && a.nsplit <= 64 && slots <= kMaxRecSplits && slots <= resident)
+  if (!balanced && a.nsplit > 1 && a.nsplit <= kMaxFoldSplits && slots <= kMaxRecSplits &&
+      (one_chunk || slots <= resident))
     a.recs = records_of(workspace);
-  const bool dense_v = a.fbits[1] == 3;  // (K rows are INT4: mfma_supported)
   if (balanced) {
     const dim3 grid((unsigned)P, (unsigned)a.H, 1u);
     if (dense_v) decode_g4_kernel<true, false, true><<<grid, dim3(kThreadsMfma), 0, stream>>>(a);
@@ -1314,7 +1346,7 @@ int launch_decode_fp16_g4(DecodeArgs &a, void *workspace, size_t ws_bytes, hipSt
   int st = setup_workspace(a, workspace, ws_bytes);
   if (st) return st;
   const int64_t slots = (int64_t)a.B * a.H * a.nsplit;
-  if (a.nsplit > 1 && a.nsplit <= 64 && slots <= kMaxRecSplits && slots <= resident)
+  if (a.nsplit > 1 && a.nsplit <= kMaxFoldSplits && slots <= kMaxRecSplits && slots <= resident)
     a.recs = records_of(workspace);
   const dim3 grid((unsigned)a.nsplit, (unsigned)a.H, (unsigned)a.B);
   decode_fp16_g4_kernel<<<grid, dim3(kThreadsMfma), 0, stream>>>(a);

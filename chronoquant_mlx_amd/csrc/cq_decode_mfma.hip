@@ -629,8 +629,8 @@ static int64_t resident_of(int slot) {
 }
 
 int64_t mfma_max_resident() {
-  return std::max(std::max(std::max(resident_of(kSlotPlain), g4_resident()), fp16_g4_resident()),
-                  std::max(resident_of(kSlotMfmaPow2), resident_of(kSlotMfma)));
+  return std::max({resident_of(kSlotPlain), g4_resident(), g4_one_chunk_resident(),
+                   fp16_g4_resident(), resident_of(kSlotMfmaPow2), resident_of(kSlotMfma)});
 }
 
 // The compressed cache takes the balanced partition for per-sequence lengths
