@@ -81,6 +81,8 @@ SIGNATURES = {
                              _P, _I32, _P, _SZ, _P], _I32),
     "cq_prefill_attn": ([_DESC, _P, _I32, _I32, _I64, _F, _I32, _I64, _P, _P, _SZ, _P], _I32),
     "cq_prefill_workspace_size": ([_I32, _I32, _I32, _I64, _I64], _SZ),
+    "cq_flash_attn": ([_DESC, _P, _I32, _I32, _I64, _F, _I32, _P, _P, _I64, _P, _P, _SZ, _P], _I32),
+    "cq_flash_scratch_size": ([_DESC, _I32, _I64, _I64], _SZ),
     "cq_gemv": ([_P, _P, _P, _I64, _I32, _I32, _P], _I32),
     "cq_gemv_rms_norm": ([_P, _P, _P, _P, _F, _P, _P, _I64, _I32, _I32, _P], _I32),
     "cq_gemv_silu": ([_P, _P, _P, _I64, _I32, _I32, _P], _I32),

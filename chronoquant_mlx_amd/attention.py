@@ -9,7 +9,11 @@ Prefill (q_len > 1, mask None or "causal", head_dim 128, fp16): the gfx950
 chunked-prefill kernel (cq_prefill_attn), which computes the fallback's
 semantics from the compressed cache without materialising K/V.
 
-Fallback (array masks, other shapes): reconstruct fp16 K/V on the GPU
+Flash kernel (cq_flash_attn; fp16 / bf16 queries, head_dim a multiple of 8):
+the other head dims, boolean masks and dense residual rows, with the fallback's
+semantics.
+
+Fallback (additive masks, fp32 queries, other head dims): reconstruct fp16 K/V on the GPU
 (cq_reconstruct) and run dense GQA attention with the reference's rounding
 points: q' = fp16(q * fp16(scale)), fp16 scores, mask, softmax in fp32
 rounded to the query dtype, fp16 weights @ V.
@@ -18,12 +22,12 @@ from __future__ import annotations
 
 import torch
 
-from .kernels import (MAX_FUSED_HEAD_DIM, chronoquant_prefill_kernel, chronoquant_sdpa_cache_kernel,
-                      prefill_supported)
+from .kernels import (MAX_FUSED_HEAD_DIM, chronoquant_flash_kernel, chronoquant_prefill_kernel,
+                      chronoquant_sdpa_cache_kernel, prefill_supported)
 
-# q_len > 1 with mask None / "causal" runs the gfx950 chunked-prefill kernel
-# (same semantics as the reconstruct fallback below); False forces the
-# fallback, which the tests use as a second implementation.
+# q_len > 1 runs the gfx950 chunked-prefill kernel or the flash kernel (same
+# semantics as the reconstruct fallback below); False forces the fallback,
+# which the tests use as a second implementation.
 PREFILL_KERNEL = True
 
 
@@ -71,6 +75,10 @@ def chronoquant_sdpa(queries: torch.Tensor, keys, values, cache, scale: float, m
 
     if PREFILL_KERNEL and prefill_supported(queries, cache, mask):
         return chronoquant_prefill_kernel(queries, cache, scale, causal=mask is not None)
+    if PREFILL_KERNEL and cache.offset > 0 and queries.is_cuda:
+        out = chronoquant_flash_kernel(queries, cache, scale, mask)
+        if out is not None:
+            return out
 
     full_k, full_v = cache.reconstruct_history()
     n_kv_heads = full_k.shape[1]

@@ -611,8 +611,64 @@ __global__ __launch_bounds__(256) void rope_append_kernel(RopeAppendArgs a) {
 }
 
 // ---------------------------------------------------------------------------
-// cq_reconstruct: one thread per (b, h, t, word) — reference cache.py:131-156
+// cq_reconstruct (reference cache.py:131-156) and the rebuild of both components
+// for cq_flash_attn: fp16 rows [B * H][T][row_dims], dims past D zero.
 // ---------------------------------------------------------------------------
+struct RebuildArgs {
+  cq_component comp[2];  // by blockIdx.z
+  uint16_t *out[2];
+  float inv_stride[2];
+  int BH, D, T, row_dims;
+};
+
+// head_dim a multiple of 8, 16-byte aligned rows, T < 2^24: one thread per 8
+// dims, one 16-byte anchor load and one 16-byte store.  PR: row_dims / 8, 0 for
+// a value known at run time only.  Bound: the stores (HBM / Infinity Cache).
+// (One thread per 8 dims with eight 2-byte loads and stores and 64-bit
+// divisions took 17-18.5 us for one component of 8192 tokens, 4 heads x 256
+// dims; both take 11 together now, 3.7 TB/s.)
+template <int PR>
+__global__ __launch_bounds__(256) void rebuild_kernel(RebuildArgs a) {
+  const int ci = blockIdx.z;
+  const cq_component &c = a.comp[ci];
+  const int pr = PR ? PR : a.row_dims / 8;
+  const int i = (int)(blockIdx.x * 256 + threadIdx.x);
+  const int t = i / pr, w = i - t * pr;
+  if (t >= a.T) return;
+  const int stride = c.stride;
+  int g = (int)((float)t * a.inv_stride[ci]);  // off by at most one
+  int r = t - g * stride;
+  if (r < 0) --g, r += stride;
+  else if (r >= stride) ++g, r -= stride;
+  const int fb = field_bits(c), rw = row_words_of(a.D, fb);
+  uint32_t magic;  // fp16 1024 in both halves
+  asm volatile("v_mov_b32 %0, 0x64006400" : "=v"(magic));
+  for (int bh = blockIdx.y; bh < a.BH; bh += gridDim.y) {
+    uint4 x = uint4{0u, 0u, 0u, 0u};
+    if (8 * w < a.D) {
+      x = *(const uint4 *)(c.keyframes + ((int64_t)bh * c.cap_keyframes + g) * a.D + 8 * w);
+      uint32_t word = 0x88888888u, s = 0u;  // an I-frame: + 0
+      if (r != 0) {
+        const int64_t slot = (int64_t)bh * c.cap_pframes + (t - g - 1);
+        const uint32_t *row = c.packed + slot * rw;
+        s = c.scales[slot];
+        if (fb == 4) {
+          word = row[w];
+        } else {  // dense fields to nibbles of the same codes
+          const uint32_t f8 = stream_bits(row, rw, 8 * fb * w, 8 * fb);
+          const uint32_t m = (1u << fb) - 1u, up = 8u - (1u << (fb - 1));
+          word = 0;
+#pragma unroll
+          for (int k = 0; k < 8; ++k) word |= (((f8 >> (fb * k)) & m) + up) << (4 * k);
+        }
+      }
+      x = rebuild8(word, x, s, magic);
+    }
+    *(uint4 *)(a.out[ci] + ((int64_t)bh * a.T + t) * (8 * pr) + 8 * w) = x;
+  }
+}
+
+// Any head_dim: one thread per (b, h, t, word).
 __global__ __launch_bounds__(256) void reconstruct_kernel(cq_component c, int B, int H,
                                                           int D, int W, int64_t T,
                                                           uint16_t *__restrict__ out) {
@@ -676,6 +732,33 @@ int validate_cache(const cq_cache_desc *c) {
 
 int64_t num_keyframes(int64_t n, int stride) { return n <= 0 ? 0 : (n - 1) / stride + 1; }
 int64_t num_pframes(int64_t n, int stride) { return n - num_keyframes(n, stride); }
+
+// Whether rebuild_kernel serves these operands.
+static bool rebuild_ok(const cq_component &c, int D, int64_t T, const void *out) {
+  return D % 8 == 0 && T < (1 << 24) && (((uintptr_t)c.keyframes | (uintptr_t)out) & 15) == 0;
+}
+
+static void launch_rebuild(RebuildArgs &a, int components, hipStream_t s) {
+  for (int i = 0; i < components; ++i) a.inv_stride[i] = 1.0f / (float)a.comp[i].stride;
+  const int pr = a.row_dims / 8;
+  const dim3 grid((unsigned)(((int64_t)a.T * pr + 255) / 256), (unsigned)std::min(a.BH, 65535),
+                  (unsigned)components), blk(256);
+  switch (pr) {
+    case 8: rebuild_kernel<8><<<grid, blk, 0, s>>>(a); break;
+    case 12: rebuild_kernel<12><<<grid, blk, 0, s>>>(a); break;
+    case 16: rebuild_kernel<16><<<grid, blk, 0, s>>>(a); break;
+    case 32: rebuild_kernel<32><<<grid, blk, 0, s>>>(a); break;
+    default: rebuild_kernel<0><<<grid, blk, 0, s>>>(a); break;
+  }
+}
+
+int launch_rebuild(const cq_cache_desc &c, int64_t T, int row_dims, uint16_t *k, uint16_t *v,
+                   hipStream_t s) {
+  if (!rebuild_ok(c.k, c.head_dim, T, k) || !rebuild_ok(c.v, c.head_dim, T, v)) return CQ_ERR_ALIGN;
+  RebuildArgs a{{c.k, c.v}, {k, v}, {}, c.batch * c.n_kv_heads, c.head_dim, (int)T, row_dims};
+  launch_rebuild(a, 2, s);
+  return launch_status();
+}
 
 }  // namespace cq
 
@@ -884,6 +967,11 @@ int cq_reconstruct(const cq_cache_desc *cache, int32_t component, int64_t seq_le
       num_pframes(seq_len, c.stride) > c.cap_pframes)
     return CQ_ERR_CAPACITY;
   const int D = cache->head_dim, W = (D + 7) / 8;
+  if (rebuild_ok(c, D, seq_len, out)) {
+    RebuildArgs a{{c, c}, {out, out}, {}, cache->batch * cache->n_kv_heads, D, (int)seq_len, D};
+    launch_rebuild(a, 1, (hipStream_t)stream);
+    return launch_status();
+  }
   const int64_t total = (int64_t)cache->batch * cache->n_kv_heads * seq_len * W;
   reconstruct_kernel<<<dim3((unsigned)((total + 255) / 256)), dim3(256), 0,
                        (hipStream_t)stream>>>(c, cache->batch, cache->n_kv_heads, D, W,

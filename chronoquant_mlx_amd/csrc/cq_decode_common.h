@@ -17,6 +17,9 @@ namespace cq {
 int validate_cache(const cq_cache_desc *c);
 int64_t num_keyframes(int64_t n, int stride);
 int64_t num_pframes(int64_t n, int stride);
+// K and V of T tokens as fp16 rows of row_dims dims (cq_codec.hip)
+int launch_rebuild(const cq_cache_desc &c, int64_t T, int row_dims, uint16_t *k, uint16_t *v,
+                   hipStream_t s);
 
 constexpr int kMaxSplits = 1024;
 constexpr int kThreadsMfma = 512;   // 8 waves per MFMA workgroup
@@ -395,7 +398,7 @@ struct SplitPlan {
 // under `slot` (one slot per decode kernel).
 enum ResidentSlot {
   kSlotGeneric = 0, kSlotMfmaPow2, kSlotMfma, kSlotPlain, kSlotG4, kSlotPrefill, kSlotFp16G4,
-  kSlotG4One,
+  kSlotG4One, kSlotFlash,
   kSlotCount
 };
 int64_t resident_workgroups(const void *kernel, int threads, int slot);

@@ -41,6 +41,32 @@ __device__ __forceinline__ uint32_t code_field(int code, int fb) {
 }
 
 // ---------------------------------------------------------------------------
+// Rebuilt rows
+// ---------------------------------------------------------------------------
+// One code word (8 nibbles, dims 0..7 of a group) and the group's fp16
+// anchor (a01, a23, a45, a67) -> the rebuilt fp16 values in dim order:
+// fp16(a + fp16(fp16(n - 8) * s)).  The low and high nibbles of the bytes
+// are interleaved into bytes n0 n1 n2 n3 / n4 n5 n6 n7, then a byte permute
+// against the magic constant makes each nibble fp16 1024 + n; subtracting
+// 1032 is exact.  Codes past the end of the cache read as 0 and the scale as
+// 0, so c * s = -0 and an I-frame row is its anchor exactly.
+typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ uint4 rebuild8(uint32_t cw, uint4 a, uint32_t scale, uint32_t magic) {
+  const half2_t s2 = __builtin_bit_cast(half2_t, scale * 0x10001u);  // the fp16 scale in both halves
+  const uint32_t lo = cw & 0x0F0F0F0Fu, hi = (cw >> 4) & 0x0F0F0F0Fu;
+  const uint32_t x0 = __builtin_amdgcn_perm(hi, lo, 0x05010400u);  // bytes n0 n1 n2 n3
+  const uint32_t x1 = __builtin_amdgcn_perm(hi, lo, 0x07030602u);  // bytes n4 n5 n6 n7
+  const half2_t bias = {(_Float16)-1032.f, (_Float16)-1032.f};
+  const uint32_t sel_a = 0x07010500u, sel_b = 0x07030502u;  // bytes (0,1) / (2,3) of x
+  const half2_t c01 = __builtin_bit_cast(half2_t, __builtin_amdgcn_perm(magic, x0, sel_a)) + bias;
+  const half2_t c23 = __builtin_bit_cast(half2_t, __builtin_amdgcn_perm(magic, x0, sel_b)) + bias;
+  const half2_t c45 = __builtin_bit_cast(half2_t, __builtin_amdgcn_perm(magic, x1, sel_a)) + bias;
+  const half2_t c67 = __builtin_bit_cast(half2_t, __builtin_amdgcn_perm(magic, x1, sel_b)) + bias;
+  return uint4{__builtin_bit_cast(uint32_t, __builtin_bit_cast(half2_t, a.x) + c01 * s2), __builtin_bit_cast(uint32_t, __builtin_bit_cast(half2_t, a.y) + c23 * s2),
+               __builtin_bit_cast(uint32_t, __builtin_bit_cast(half2_t, a.z) + c45 * s2), __builtin_bit_cast(uint32_t, __builtin_bit_cast(half2_t, a.w) + c67 * s2)};
+}
+
+// ---------------------------------------------------------------------------
 // dtype traits.  round() rounds a binary32 value to the dtype (nearest even)
 // and returns it as binary32; every codec op is "compute in binary32, round"
 // which equals the dtype's own correctly rounded op for + - * / (24 >= 2p+2).

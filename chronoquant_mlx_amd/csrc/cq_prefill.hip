@@ -119,27 +119,6 @@ __device__ __forceinline__ uint32_t bload16(__amdgpu_buffer_rsrc_t r, uint32_t o
   return (uint32_t)__builtin_amdgcn_raw_buffer_load_b16(r, (int)off, 0, 0);
 }
 
-// One code word (8 nibbles, dims 0..7 of a group) and the group's fp16
-// anchor (a01, a23, a45, a67) -> the rebuilt fp16 values in dim order:
-// fp16(a + fp16(fp16(n - 8) * s)).  The low and high nibbles of the bytes
-// are interleaved into bytes n0 n1 n2 n3 / n4 n5 n6 n7, then a byte permute
-// against the magic constant makes each nibble fp16 1024 + n; subtracting
-// 1032 is exact.  Codes past the end of the cache read as 0 and the scale as
-// 0, so c * s = -0 and an I-frame row is its anchor exactly.
-__device__ __forceinline__ uint4 rebuild8(uint32_t cw, uint4 a, h2_t s2, uint32_t magic) {
-  const uint32_t lo = cw & 0x0F0F0F0Fu, hi = (cw >> 4) & 0x0F0F0F0Fu;
-  const uint32_t x0 = __builtin_amdgcn_perm(hi, lo, 0x05010400u);  // bytes n0 n1 n2 n3
-  const uint32_t x1 = __builtin_amdgcn_perm(hi, lo, 0x07030602u);  // bytes n4 n5 n6 n7
-  const h2_t bias = {(_Float16)-1032.f, (_Float16)-1032.f};
-  const uint32_t sel_a = 0x07010500u, sel_b = 0x07030502u;  // bytes (0,1) / (2,3) of x
-  const h2_t c01 = as_h2(__builtin_amdgcn_perm(magic, x0, sel_a)) + bias;
-  const h2_t c23 = as_h2(__builtin_amdgcn_perm(magic, x0, sel_b)) + bias;
-  const h2_t c45 = as_h2(__builtin_amdgcn_perm(magic, x1, sel_a)) + bias;
-  const h2_t c67 = as_h2(__builtin_amdgcn_perm(magic, x1, sel_b)) + bias;
-  return uint4{as_u(as_h2(a.x) + c01 * s2), as_u(as_h2(a.y) + c23 * s2),
-               as_u(as_h2(a.z) + c45 * s2), as_u(as_h2(a.w) + c67 * s2)};
-}
-
 // LDS transpose read (gfx950 ds_read_b64_tr_b16): within each group of 16
 // lanes, lane 4j + c addresses 4 fp16 (c: a 4-column slice of row j) and
 // lane r of the group receives element r % 4 of lanes r / 4, r / 4 + 4,
@@ -412,10 +391,9 @@ void prefill_mfma_kernel(PrefillArgs a) {
   // ---- 1. rebuild the staged block: K (waves 0-7) or V (waves 8-15) into
   // LDS buffer `buf` --------------------------------------------------------------
   auto rebuild = [&](int buf) {
-    const h2_t s2 = as_h2(r_s * 0x10001u);
     uint4 *dst = (uint4 *)(c == 0 ? &lds.k[buf][kkey][16 * ke] : &lds.v[buf][kkey][16 * ke]);
 #pragma unroll
-    for (int j = 0; j < 2; ++j) dst[j] = rebuild8(r_cw[j], r_an[j], s2, magic);
+    for (int j = 0; j < 2; ++j) dst[j] = rebuild8(r_cw[j], r_an[j], r_s, magic);
   };
 
   // Pipeline: while block kb's products read one LDS buffer, the waves

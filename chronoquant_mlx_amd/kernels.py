@@ -228,3 +228,55 @@ def prefill_supported(queries: torch.Tensor, cache, mask) -> bool:
             and (mask is None or (isinstance(mask, str) and mask == "causal"))
             and cache.offset >= L and nq % cache._shape[1] == 0
             and 256 % (nq // cache._shape[1]) == 0)
+
+
+def _differentiated(t: torch.Tensor) -> bool:
+    """Whether autograd, forward-mode AD or a functorch transform follows t:
+    what is computed from it then has to stay torch ops."""
+    return ((torch.is_grad_enabled() and t.requires_grad) or type(t) is not torch.Tensor
+            or torch._C._functorch.is_functorch_wrapped_tensor(t)
+            or torch.autograd.forward_ad.unpack_dual(t).tangent is not None)
+
+
+def chronoquant_flash_kernel(q: torch.Tensor, cache, scale: float, mask) -> torch.Tensor | None:
+    """Attention of q [B, nq, L, D] (fp16 or bf16, UNSCALED) over the cache
+    with mask None, "causal" or a boolean tensor that broadcasts to [B, kv
+    heads, q heads per kv head, L, cache.offset] (cq_flash_attn).  The result
+    semantics of the reconstruct fallback of chronoquant_sdpa.  None for a call
+    the kernel does not serve (the caller then runs the fallback)."""
+    B, nq, L, D = q.shape
+    T = cache.offset
+    if cache._shape is None or q.dtype not in (torch.float16, torch.bfloat16) or _differentiated(q):
+        return None
+    H = cache._shape[1]
+    if q.device != cache._device or cache._shape[0] != B or cache._shape[2] != D or nq % H:
+        return None
+    strides, mask_ptr = None, None
+    if mask is None:
+        kind = 0
+    elif isinstance(mask, str):
+        if T < L:
+            return None
+        kind = 1
+    else:
+        if mask.dtype != torch.bool:
+            return None
+        mask = mask.to(q.device)
+        try:
+            mask = mask.expand(B, H, nq // H, L, T)
+        except RuntimeError:
+            return None
+        kind, strides, mask_ptr = 2, (ctypes.c_int64 * 5)(*mask.stride()), mask.data_ptr()
+    desc = cache._descriptor()
+    need = _lib.load().cq_flash_scratch_size(desc, nq, L, T)
+    if not need:
+        return None
+    q = q.contiguous()
+    if q.data_ptr() % 16:
+        q = q.clone()
+    out = torch.empty_like(q)
+    scratch = torch.empty(need, dtype=torch.uint8, device=q.device)
+    _lib.call("cq_flash_attn", desc, q.data_ptr(), _lib.dtype_code(q.dtype), nq, L, float(scale),
+              kind, mask_ptr, strides, T, out.data_ptr(), scratch.data_ptr(), need,
+              _lib.stream_of(q))
+    return out

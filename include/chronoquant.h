@@ -257,6 +257,28 @@ int cq_prefill_attn(const cq_cache_desc *cache, const void *q, int32_t q_dtype,
 size_t cq_prefill_workspace_size(int32_t batch, int32_t n_kv_heads, int32_t n_q_heads,
                                  int64_t n_q, int64_t seq_len);
 
+/* Attention of n_q query rows per sequence over the compressed cache, for the
+ * calls cq_prefill_attn declines: any head_dim that is a multiple of 8, dense
+ * residual rows, and boolean masks.  The same semantics (the reconstruct
+ * fallback of chronoquant_sdpa, reference attention.py:8-20, 61-74 over
+ * cache.py:131-160), with bf16 queries' weights kept in 32 bits, as the
+ * reference's promotion keeps them.
+ * mask_kind: 0 none; 1 causal (query i sees keys <= seq_len - n_q + i, n_q <=
+ * seq_len); 2 a boolean mask, one byte per element (0: hidden), element
+ * (sequence, kv head, q head of the group, query, key) at the element strides
+ * mask_strides[5] (0: broadcast).  A hidden key's score is the lowest finite
+ * value, so a row that sees no key weighs all keys alike.
+ * q, out: [B][n_q_heads][n_q][head_dim], CQ_F16 or CQ_BF16, 16-byte aligned.
+ * scratch: caller-owned device memory of cq_flash_scratch_size(...) bytes (0
+ * for a shape it does not serve), 256-byte aligned, any contents: K and V
+ * rebuilt as fp16 rows, and the key splits' partials. */
+int cq_flash_attn(const cq_cache_desc *cache, const void *q, int32_t q_dtype, int32_t n_q_heads,
+                  int64_t n_q, float scale, int32_t mask_kind, const uint8_t *mask,
+                  const int64_t *mask_strides, int64_t seq_len, void *out, void *scratch,
+                  size_t scratch_bytes, cq_stream_t stream);
+size_t cq_flash_scratch_size(const cq_cache_desc *cache, int32_t n_q_heads, int64_t n_q,
+                             int64_t seq_len);
+
 /* ---- Fused elementwise ops of the end-to-end decoder ------------------
  * No counterpart in the reference's own files: these are the roles of
  * mlx's mx.fast.rms_norm / mx.fast.rope and mlx_lm's SwiGLU inside the

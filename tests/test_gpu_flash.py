@@ -1,0 +1,137 @@
+"""cq_flash_attn against the oracle's restatement of the reconstruct fallback
+(attention.py:8-20, 61-74): head dims on both sides of the padded sizes, row
+tiles and key blocks with remainders, split keys, boolean masks of every
+broadcast form (rows that see no key among them), dense rows, fp16 and bf16
+queries, and the calls it leaves to the fallback."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import oracle as O
+from tests.cqtest import assert_close, build_gpu_cache, build_oracle, to_gpu
+
+pytestmark = pytest.mark.gpu
+
+
+def _stream(rng, B, H, T, D):
+    return np.cumsum(rng.standard_normal((B, H, T, D)) * 0.1, axis=2).astype(np.float16)
+
+
+def _mask(kind, rng, L, T):
+    """(mask as [L, T] booleans or None, what the call takes)."""
+    if kind in ("causal", None):
+        return None, kind
+    if kind == "window":
+        q, k = np.arange(T - L, T)[:, None], np.arange(T)[None]
+        m = (q >= k) & (q < k + max(1, T // 4))
+    elif kind == "rows":  # one column for every key: broadcast over the keys
+        return np.broadcast_to(rng.random((L, 1)) > 0.5, (L, T)), None
+    else:
+        m = rng.random((L, T)) > 0.5
+        m[0] = False  # a row that sees nothing weighs every key alike
+    return m, torch.from_numpy(m).cuda()
+
+
+# (H, G, D, T, L, mask, params): 64-, 96-, 128- and 256-wide rows and their edges
+# (8, 72, 80, 136), key blocks of 32 and 64 with one key more or less, 256-row
+# tiles with one row more (G L = 256, 257), and enough keys to split
+CASES = [
+    (2, 4, 64, 65, 64, "causal", {}), (2, 3, 72, 300, 77, "causal", {}), (1, 2, 80, 127, 128 - 1, None, {}),
+    (2, 1, 8, 40, 3, "causal", {}), (1, 4, 136, 33, 33, "causal", {}), (2, 4, 256, 1000, 64, "causal", {}),
+    (1, 1, 256, 32, 1, None, {}), (1, 1, 256, 2049, 257, "random", {}), (2, 4, 128, 1000, 65, "window", {}),
+    (1, 4, 128, 129, 129, "random", {}), (1, 2, 96, 64, 20, "rows", {}), (1, 4, 256, 500, 100, "window", {}),
+    (2, 4, 128, 600, 50, "causal", dict(stride_k=64, stride_v=32, bits_v=3, dz_v=0.05, dense=True)),
+    (1, 2, 80, 200, 30, "causal", dict(stride_k=5, stride_v=1, bits_k=2, dense=True)),
+]
+
+
+@pytest.mark.parametrize("dtype", ["f16", "bf16"])
+@pytest.mark.parametrize("H,G,D,T,L,mask,params", CASES)
+def test_flash_matches_fallback(H, G, D, T, L, mask, params, dtype):
+    from chronoquant_mlx_amd import ChronoQuantCache, kernels
+    rng = np.random.default_rng(D * 7 + T + L)
+    k, v = _stream(rng, 1, H, T, D), _stream(rng, 1, H, T, D)
+    p = dict(dict(stride_k=32, stride_v=8), **params)
+    dense = p.pop("dense", False)
+    cache = ChronoQuantCache(stride_k=p["stride_k"], stride_v=p["stride_v"], delta_bits_k=p.get("bits_k", 4),
+                             delta_bits_v=p.get("bits_v", 4), dead_zone_v=p.get("dz_v", 0.0),
+                             dense_residuals=dense)
+    cache.update_and_fetch(to_gpu(k), to_gpu(v))
+    q32 = rng.standard_normal((1, G * H, L, D)).astype(np.float32)
+    scale = D ** -0.5
+    m, arg = _mask(mask, rng, L, T)
+    if m is not None and arg is None:
+        arg = torch.from_numpy(m[:, :1].copy()).cuda()
+    ck, cv = build_oracle(k[0], v[0], **p)
+    rk, rv = ck.reconstruct(), cv.reconstruct()
+    dt = torch.float16 if dtype == "f16" else torch.bfloat16
+    qt = to_gpu(q32, dt)
+    out = kernels.chronoquant_flash_kernel(qt, cache, scale, arg)
+    assert out is not None and out.dtype == dt
+    if dtype == "f16":
+        ref = O.sdpa_fallback(qt.cpu().numpy()[0], rk, rv, scale, causal=mask == "causal", mask=m)
+    else:
+        bits = qt.cpu().view(torch.int16).numpy().view(np.uint16)[0]
+        ref = O.bf16_to_f32(O.sdpa_fallback_bf16q(bits, rk, rv, scale, causal=mask == "causal", mask=m))
+    assert_close(out.float().cpu().numpy()[0], ref.astype(np.float64), what=f"{dtype} {mask}")
+
+
+def test_flash_bf16_weights_keep_32_bits():
+    # One dominant and many small weights: with the weights rounded to fp16 the
+    # small ones (2^-16 of the top one) would be off by up to 2^-9 each; the
+    # split pair holds them to 2^-20.  V rows of the small ones share a sign, so
+    # their errors add up.  Bar: one bf16 rounding of the output (2^-9) on the
+    # part the small ones make, which the fallback in fp32 meets too.
+    from chronoquant_mlx_amd import ChronoQuantCache, kernels
+    T, D = 4096, 64
+    rng = np.random.default_rng(3)
+    k = np.zeros((1, 1, T, D), np.float16)
+    k[..., 0] = rng.uniform(-0.25, 0.25, T)
+    v = np.ones((1, 1, T, D), np.float16)
+    k[0, 0, 0, 0], v[0, 0, 0] = 11, 0
+    cache = ChronoQuantCache(stride_k=1, stride_v=1)
+    cache.update_and_fetch(to_gpu(k), to_gpu(v))
+    q = torch.zeros(1, 1, 2, D, dtype=torch.bfloat16, device="cuda")
+    q[..., 0] = 1.0
+    out = kernels.chronoquant_flash_kernel(q, cache, 1.0, None).double().cpu().numpy()
+    w = np.exp(k[0, 0, :, 0].astype(np.float64))
+    exact = w[1:].sum() / w.sum()
+    assert np.all(np.abs(out - exact) <= 2.0 ** -9 * exact), (out.ravel()[0], exact)
+
+
+@pytest.mark.parametrize("shape", [(1, 1, 1, 9, 70), (1, 2, 1, 9, 70), (2, 2, 3, 9, 70), (9, 1), (70,)])
+def test_flash_mask_broadcasts_like_the_fallback(shape):
+    from chronoquant_mlx_amd import attention as A
+    B, H, G, L, T, D = 2, 2, 3, 9, 70, 128
+    rng = np.random.default_rng(len(shape))
+    cache = build_gpu_cache(_stream(rng, B, H, T, D), _stream(rng, B, H, T, D), stride_k=32, stride_v=8)
+    q = to_gpu(rng.standard_normal((B, G * H, L, D)))
+    mask = torch.from_numpy(rng.random(shape) > 0.4).cuda()
+    got = A.chronoquant_sdpa(q, None, None, cache, D ** -0.5, mask)
+    A.PREFILL_KERNEL = False
+    try:
+        ref = A.chronoquant_sdpa(q, None, None, cache, D ** -0.5, mask)
+    finally:
+        A.PREFILL_KERNEL = True
+    assert_close(got.float().cpu().numpy(), ref.float().cpu().numpy())
+
+
+def test_flash_leaves_to_the_fallback():
+    # additive masks, fp32 queries, head dims that are no multiple of 8, causal
+    # chunks longer than the cache, and queries that autograd follows
+    from chronoquant_mlx_amd import chronoquant_sdpa, kernels
+    rng = np.random.default_rng(1)
+    H, L, T = 2, 5, 40
+    for D, dt, mask in ((64, torch.float16, torch.zeros(L, T, device="cuda")), (64, torch.float32, None),
+                        (12, torch.float16, None), (64, torch.float16, "grad")):
+        cache = build_gpu_cache(_stream(rng, 1, H, T, D), _stream(rng, 1, H, T, D), stride_k=32, stride_v=8)
+        q = to_gpu(rng.standard_normal((1, H, L, D)), dt)
+        if isinstance(mask, str):
+            q.requires_grad_(True)
+            mask = torch.ones(L, T, dtype=torch.bool, device="cuda")
+        assert kernels.chronoquant_flash_kernel(q, cache, 1.0, mask) is None
+        out = chronoquant_sdpa(q, None, None, cache, D ** -0.5, mask)
+        assert out.shape == q.shape and bool(torch.isfinite(out).all())
+        assert out.requires_grad == q.requires_grad
+    q = to_gpu(rng.standard_normal((1, H, T + 1, 12)))
+    assert kernels.chronoquant_flash_kernel(q, cache, 1.0, "causal") is None
