@@ -265,7 +265,9 @@ static int64_t generic_resident() {
                              kSlotGeneric);
 }
 
-int64_t decode_max_resident() { return std::max(generic_resident(), mfma_max_resident()); }
+int64_t decode_max_resident() {
+  return std::max({generic_resident(), mfma_max_resident(), wide_max_resident()});
+}
 
 static int launch_generic(DecodeArgs &a, void *workspace, size_t ws_bytes, hipStream_t stream) {
   int st = prepare_launch(a, kGenericGroup, generic_resident(), workspace, ws_bytes);
@@ -328,6 +330,8 @@ static int decode_entry(const cq_cache_desc *cache, const void *q, int32_t q_dty
   if (st) return st;
   if (allow_mfma && mfma_supported(a))
     return launch_decode_mfma(a, workspace, workspace_bytes, (hipStream_t)stream);
+  if (allow_mfma && wide_supported(a))
+    return launch_decode_wide(a, workspace, workspace_bytes, (hipStream_t)stream);
   return launch_generic(a, workspace, workspace_bytes, (hipStream_t)stream);
 }
 

@@ -398,7 +398,7 @@ struct SplitPlan {
 // under `slot` (one slot per decode kernel).
 enum ResidentSlot {
   kSlotGeneric = 0, kSlotMfmaPow2, kSlotMfma, kSlotPlain, kSlotG4, kSlotPrefill, kSlotFp16G4,
-  kSlotG4One, kSlotFlash,
+  kSlotG4One, kSlotFlash, kSlotWide,
   kSlotCount
 };
 int64_t resident_workgroups(const void *kernel, int threads, int slot);
@@ -537,6 +537,10 @@ inline int64_t balanced_slots(int64_t P, int64_t max_T) {
 
 int launch_decode_mfma(DecodeArgs &a, void *workspace, size_t ws_bytes, hipStream_t stream);
 bool mfma_supported(const DecodeArgs &a);
+// other head dims and dense rows (cq_decode_wide.hip)
+bool wide_supported(const DecodeArgs &a);
+int64_t wide_max_resident();
+int launch_decode_wide(DecodeArgs &a, void *workspace, size_t ws_bytes, hipStream_t stream);
 // GQA groups of at most 4 q heads (cq_decode_g4.hip): the shape conditions
 // alone, and together with mfma_supported's
 bool g4_shape(const DecodeArgs &a);

@@ -1,0 +1,598 @@
+// cq_decode_wide.hip — gfx950 MFMA split-K decode over the ChronoQuant cache for
+// the shapes the head_dim-128 kernels do not take: any head_dim that is a
+// multiple of 8, dense 2- and 3-bit rows, fp16 or bf16 queries, strides >= 4,
+// any GQA ratio in chunks of 16 q heads.
+//
+// Reference semantics: the fused Metal kernel (kernels.py:79-228), in the
+// factoring of the 16-head kernel (cq_decode_mfma.hip):
+//   score_t = q'.a_g(t) + s_t * (q'.c_t)
+//   out     = sum_g P_g a_g + sum_t (p_t s_t) c_t,   P_g = sum_{t in g} p_t
+// These shapes ran on the portable kernel, whose weights and products are fp32,
+// so no operand here holds less than fp32 needs:
+// * q' is exact in fp16 (bf16 rows scaled by a power of two first), code fields
+//   enter as fp16 denormals n * 2^-24 (exact), anchors are fp16: the scores are
+//   exact products summed in fp32;
+// * P and p*s enter as fp16 pairs hi + lo (22 bits), two products each, scaled by
+//   powers of two so that the pairs stay clear of fp16's subnormals and range;
+// * the fields are not offset by a magic constant (1024 + n would leave the
+//   accumulator 14 bits for n): a chunk's code product starts at zero and is
+//   scaled into the fp32 accumulator, and the sum of the same weights times the
+//   fields' offset comes off at the end.
+//
+// Layout (NS K-steps of 32 dims, 32 NS >= D; W = D / 8 words of a row): lane (c,
+// kg) of a score operand holds words NS kg .. NS kg + NS - 1 of token c (one or
+// two wide loads), K-step j taking word NS kg + j; lane c of a V operand words
+// NU c .. NU c + NU - 1 (NU = 2 beyond 128 dims) of 16 tokens.  Work: the balanced
+// partition of cq_plan.h, 512-token units over one resident generation.
+//
+// Bound: the chain of a chunk (loads, two products, softmax) with two waves per
+// SIMD in flight.  4 sequences of 16001 tokens, 16/4 heads x 256 dims (82 MB): 34 us,
+// 2.4 TB/s, against 370 on the portable kernel (fp32 VALU products, 8 head slots for
+// 4 heads); 16 ragged sequences of up to 4096, 32/8 x 64: 30 against 177; one of
+// 1000, 16/4 x 256: 19 against 304.  Error of the fp32 output against binary64:
+// 0.8 to 1.4e-7 relative, the portable kernel 0.6 to 1.4e-7.
+#include <hip/hip_runtime.h>
+#include <math.h>
+
+#include <algorithm>
+
+#include "cq_mfma_common.h"
+
+namespace cq {
+
+namespace {
+
+constexpr float kTauW = 2.f;                // lazy-rescale threshold: p <= 4
+constexpr float kPScale = 16.f;             // P_g operand scale (P_g <= 64 * 4)
+constexpr float kWScale = 512.f;            // p*s operand scale (p*s <= 4 * 16, see emax)
+constexpr int kScaleExp = 4;                // log2 of the largest scale that needs no care
+
+template <int NS>
+struct WideDims {
+  static constexpr int kDP = 32 * NS;
+  static constexpr int kNU = NS > 4 ? 2 : 1;  // V words per lane
+  static constexpr int kTiles = 8 * kNU;      // 16-column V tiles
+};
+
+struct alignas(16) WideWave {
+  int slot_k[kChunk], slot_v[kChunk];  // P-frame slot (-1: I-frame / padding)
+  int gkl[kChunk], gvl[kChunk];        // anchor index relative to the chunk's first
+  uint32_t s16[kChunk];                // fp16 K scale | fp16 V scale << 16 (0: none)
+  float qa[16][kHeads];                // q'.anchor_k by (local anchor, head)
+};
+
+template <int NS>
+struct alignas(16) WideMerge {
+  static constexpr int kO = 16 * 8 * WideDims<NS>::kNU;  // dims the V tiles cover
+  float t[kWaves][kMergeHeads][kO];
+  float m[kWaves][kHeads], l[kWaves][kHeads];
+  float wm[kHeads], wl[kHeads];
+  float o[kHeads][kO];
+};
+
+template <int NS>
+struct WideLds {
+  h8_t qn[NS][64], qc[NS][64];  // q' of K-step j, lane (head, kg): natural order, field order
+  float cs[kHeads], qsum[kHeads];
+  union {
+    WideWave w[kWaves];
+    WideMerge<NS> mg;
+  };
+};
+
+// n consecutive dwords at a dword-aligned offset
+template <int N>
+__device__ __forceinline__ void bload_words(__amdgpu_buffer_rsrc_t r, uint32_t off, uint32_t (&w)[N]) {
+  int i = 0;
+#pragma unroll
+  for (; i + 4 <= N; i += 4) {
+    const uint4 v = bload128(r, off + 4u * i);
+    w[i] = v.x, w[i + 1] = v.y, w[i + 2] = v.z, w[i + 3] = v.w;
+  }
+#pragma unroll
+  for (; i + 2 <= N; i += 2) {
+    const auto v = __builtin_amdgcn_raw_buffer_load_b64(r, (int)(off + 4u * i), 0, kPolicyStream);
+    w[i] = (uint32_t)v[0], w[i + 1] = (uint32_t)v[1];
+  }
+  if (i < N) w[i] = bload32(r, off + 4u * i);
+}
+
+// Dense rows: the fields of dims 8 word .. 8 word + 7 (8 fb stream bits at bit 8 fb word),
+// spread to nibbles.
+__device__ __forceinline__ uint32_t bload_dense(__amdgpu_buffer_rsrc_t r, uint32_t row, int word, int fb) {
+  const uint32_t bit = 8u * fb * word;
+  const uint32_t a = bload32(r, row + 4u * (bit >> 5)), b = bload32(r, row + 4u * (bit >> 5) + 4u);
+  const uint32_t f = __builtin_amdgcn_alignbit(b, a, bit & 31u);
+  const uint32_t m = (1u << fb) - 1u;
+  uint32_t w = 0;
+#pragma unroll
+  for (int k = 0; k < 8; ++k) w |= ((f >> (fb * k)) & m) << (4 * k);
+  return w;
+}
+
+// hi + lo fp16 pair of x0, x1
+__device__ __forceinline__ void split2(float x0, float x1, h2_t &hi, h2_t &lo) {
+  hi = h2_t{(_Float16)x0, (_Float16)x1};
+  lo = h2_t{(_Float16)(x0 - (float)hi.x), (_Float16)(x1 - (float)hi.y)};
+}
+__device__ __forceinline__ h8_t h8_of2(h2_t a, h2_t b, h2_t c, h2_t d) {
+  return h8_t{a.x, a.y, b.x, b.y, c.x, c.y, d.x, d.y};
+}
+
+template <int NS, bool Dense>
+__global__ __launch_bounds__(kThreadsMfma) __attribute__((amdgpu_waves_per_eu(2, 2)))
+void decode_wide_kernel(DecodeArgs a) {
+  using Dm = WideDims<NS>;
+  constexpr int NU = Dm::kNU, NT = Dm::kTiles;
+  __shared__ WideLds<NS> lds;
+  __shared__ int32_t s_units[kMaxTableSeqs + 1];
+  __shared__ int32_t s_loop[8];  // cursor unit [2], cursor sequence [2], end unit, P, n
+  prefetch_args();
+  const int h = blockIdx.y / a.n_chunks;
+  const int chunk = blockIdx.y - h * a.n_chunks;
+  const bool table = a.seq_lens && a.B > 1 && a.B <= kMaxTableSeqs;
+  {
+    if (table) build_unit_table(a, s_units);
+    UnitSpace us;
+    us.start = table ? s_units : nullptr;
+    us.n = units_of(a.max_T);
+    us.B = a.B;
+    const int64_t U = us.total();
+    const int64_t P = min((int64_t)gridDim.x, U);  // every workgroup below P has units
+    if ((int64_t)blockIdx.x >= P) return;
+    if (threadIdx.x == 0) {
+      const int64_t u0 = unit_begin(blockIdx.x, U, P);
+      s_loop[0] = (int32_t)u0;
+      s_loop[2] = us.seq_of(u0);
+      s_loop[4] = (int32_t)unit_begin(blockIdx.x + 1, U, P);
+      s_loop[5] = (int32_t)P;
+      s_loop[6] = (int32_t)us.n;
+    }
+    __syncthreads();
+  }
+  const int D = a.D, W = a.W;
+  const int j0 = chunk * kHeads;
+  const int gn = min(kHeads, a.G - j0);
+  const int sk = a.stride[0], sv = a.stride[1];
+  const float isk = a.inv_stride[0], isv = a.inv_stride[1];
+  const int fbk = Dense ? a.fbits[0] : 4, fbv = Dense ? a.fbits[1] : 4;
+  const uint32_t krow = 4u * row_words_of(D, fbk), vrow = 4u * row_words_of(D, fbv);
+  const float biask = (float)(1 << (fbk - 1)), biasv = (float)(1 << (fbv - 1));
+
+  for (int it = 0;; ++it) {
+    const int tid = thread_id();
+    __builtin_assume(tid >= 0 && tid < kThreadsMfma);
+    const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int col = lane & 15, kg = lane >> 4;
+    const volatile int32_t *sl = s_loop;
+    const int32_t u = __builtin_amdgcn_readfirstlane(sl[it & 1]);
+    if (u >= __builtin_amdgcn_readfirstlane(sl[4])) break;
+    const int b = __builtin_amdgcn_readfirstlane(sl[2 + (it & 1)]);
+    Segment sg;
+    {
+      UnitSpace us;
+      us.start = table ? s_units : nullptr;
+      us.n = __builtin_amdgcn_readfirstlane(sl[6]);
+      us.B = a.B;
+      const int64_t u_next = segment_at(us, blockIdx.x, __builtin_amdgcn_readfirstlane(sl[5]), u, b,
+                                        seq_len_of(a, b), sg);
+      if (tid == 0) {
+        s_loop[(it + 1) & 1] = (int32_t)u_next;
+        s_loop[2 + ((it + 1) & 1)] = b + 1;
+      }
+    }
+    if (sg.live == 0) {  // past the sequence's end
+      __syncthreads();
+      continue;
+    }
+    const int64_t t0 = sg.t0, t1 = sg.t1;
+    const int64_t bh = (int64_t)b * a.H + h;
+    const __amdgpu_buffer_rsrc_t r_kfk =
+        make_rsrc(a.kf[0] + bh * a.cap_kf[0] * D, (uint32_t)(a.cap_kf[0] * D * 2));
+    const __amdgpu_buffer_rsrc_t r_kfv =
+        make_rsrc(a.kf[1] + bh * a.cap_kf[1] * D, (uint32_t)(a.cap_kf[1] * D * 2));
+    const __amdgpu_buffer_rsrc_t r_pkk =
+        make_rsrc((const char *)a.pk[0] + bh * a.cap_pf[0] * krow, (uint32_t)(a.cap_pf[0] * krow));
+    const __amdgpu_buffer_rsrc_t r_pkv =
+        make_rsrc((const char *)a.pk[1] + bh * a.cap_pf[1] * vrow, (uint32_t)(a.cap_pf[1] * vrow));
+    const __amdgpu_buffer_rsrc_t r_sck = make_rsrc(a.sc[0] + bh * a.cap_pf[0], (uint32_t)(a.cap_pf[0] * 2));
+    const __amdgpu_buffer_rsrc_t r_scv = make_rsrc(a.sc[1] + bh * a.cap_pf[1], (uint32_t)(a.cap_pf[1] * 2));
+
+    // ---- q' tables: half-wave tid / 32 = head, its lane = word ----------------------
+    {
+      const int hh = tid >> 5, w = tid & 31;
+      float v[8];
+      float top = 0.f, sum = 0.f;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[e] = 0.f;
+      if (hh < gn && w < W) {
+        const uint4 raw = *(const uint4 *)((const uint16_t *)a.q +
+                                           ((int64_t)b * a.nq + h * a.G + j0 + hh) * D + 8 * w);
+        const uint32_t x[4] = {raw.x, raw.y, raw.z, raw.w};
+        if (a.q_dtype == CQ_BF16) {
+          const float scb = bf2f(f2bf(a.scale));
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            v[2 * i] = bf2f(f2bf(__uint_as_float(x[i] << 16) * scb));
+            v[2 * i + 1] = bf2f(f2bf(__uint_as_float(x[i] & 0xffff0000u) * scb));
+          }
+        } else {
+          const float sch = h2f(f2h(a.scale));
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            v[2 * i] = h2f(f2h(h2f((uint16_t)(x[i] & 0xffffu)) * sch));
+            v[2 * i + 1] = h2f(f2h(h2f((uint16_t)(x[i] >> 16)) * sch));
+          }
+        }
+      }
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        top = fmaxf(top, fabsf(v[e]));
+        sum += v[e];
+      }
+#pragma unroll
+      for (int x = 1; x < 32; x *= 2) {
+        top = fmaxf(top, __shfl_xor(top, x, 64));
+        sum += __shfl_xor(sum, x, 64);
+      }
+      // bf16: a power of two brings the row's top to [2^13, 2^14), so that the
+      // fp16 form is exact down to 2^-27 of it (0, infinities, NaN: as they are)
+      const int ex = (int)(__float_as_uint(top) >> 23);
+      const int up = (a.q_dtype != CQ_BF16 || ex == 0 || ex == 255) ? 0 : min(127 + 13 - ex, 100);
+      const float f = __uint_as_float((uint32_t)(127 + up) << 23);
+      if (w == 0) {
+        lds.cs[hh] = kLog2e * __uint_as_float((uint32_t)(127 - up) << 23);
+        lds.qsum[hh] = sum * f;
+      }
+      if (w < 4 * NS) {
+        h8_t q;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) q[e] = (_Float16)(v[e] * f);
+        const int qkg = w / NS, qj = w - qkg * NS;
+        lds.qn[qj][16 * qkg + hh] = q;
+        lds.qc[qj][16 * qkg + hh] = h8_t{q[0], q[4], q[1], q[5], q[2], q[6], q[3], q[7]};
+      }
+    }
+    __syncthreads();
+    const float cs = lds.cs[col], sbias = biask * lds.qsum[col];
+
+    float m_run = -INFINITY;  // per head col, log2 units
+    float l_run = 0.f;        // sum of p over this lane's tokens
+    float w_run = 0.f;        // sum of the p*s operands (kWScale)
+    f4_t acc[NT];             // kPScale units
+#pragma unroll
+    for (int n = 0; n < NT; ++n) acc[n] = f4_t{0.f, 0.f, 0.f, 0.f};
+    const h2_t ones = {(_Float16)1.f, (_Float16)1.f};
+    WideWave &Ws = lds.w[wave];
+
+    for (int64_t c0l = t0 + (int64_t)wave * kChunk; c0l < t1; c0l += kWaves * kChunk) {
+      const int c0 = (int)c0l;
+      const int nt = (int)min((int64_t)kChunk, t1 - c0l);
+      const int gk_base = div_stride(c0, sk, isk), gk_last = div_stride(c0 + nt - 1, sk, isk);
+      const int gv_base = div_stride(c0, sv, isv), gv_last = div_stride(c0 + nt - 1, sv, isv);
+      // ---- token phase: one token per lane ------------------------------------------
+      uint32_t s16;
+      {
+        const bool valid = lane < nt;
+        const int t = c0 + (valid ? lane : nt - 1);
+        const int gk = div_stride(t, sk, isk), gv = div_stride(t, sv, isv);
+        const int slk = (valid && t != gk * sk) ? t - gk - 1 : -1;
+        const int slv = (valid && t != gv * sv) ? t - gv - 1 : -1;
+        const uint32_t sk16 = bload16(r_sck, (uint32_t)slk * 2u);  // slot -1: past the buffer, 0
+        const uint32_t sv16 = bload16(r_scv, (uint32_t)slv * 2u);
+        Ws.slot_k[lane] = slk;
+        Ws.slot_v[lane] = slv;
+        Ws.gkl[lane] = gk - gk_base;
+        Ws.gvl[lane] = gv - gv_base;
+        s16 = sk16 | (sv16 << 16);
+      }
+      wave_lds_sync();
+      // ---- the chunk's loads ------------------------------------------------------------
+      // (slot -1 wraps past the buffer, or to bytes of row 0: the token's scale is 0)
+      uint32_t kw[4][NS];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const uint32_t row = (uint32_t)Ws.slot_k[16 * i + col] * krow;
+        if constexpr (Dense) {
+#pragma unroll
+          for (int j = 0; j < NS; ++j)
+            kw[i][j] = fbk == 4 ? bload32(r_pkk, row + 4u * (NS * kg + j))
+                                : bload_dense(r_pkk, row, NS * kg + j, fbk);
+        } else {
+          bload_words<NS>(r_pkk, row + 4u * NS * kg, kw[i]);
+        }
+      }
+      uint4 ka[NS];
+      {
+        const uint32_t row = (uint32_t)min(gk_base + col, gk_last) * (uint32_t)(2 * D);
+#pragma unroll
+        for (int j = 0; j < NS; ++j)  // dims past D: zeros
+          ka[j] = bload128(r_kfk, NS * kg + j < W ? row + 16u * (NS * kg + j) : 0x80000000u);
+      }
+      uint32_t vw[4][4][NU];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int4 s4 = *(const int4 *)&Ws.slot_v[16 * i + 4 * kg];
+        const int ss[4] = {s4.x, s4.y, s4.z, s4.w};
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const uint32_t row = (uint32_t)ss[r] * vrow;
+          if constexpr (Dense) {
+#pragma unroll
+            for (int x = 0; x < NU; ++x)
+              vw[i][r][x] = fbv == 4 ? bload32(r_pkv, row + 4u * (NU * col + x))
+                                     : bload_dense(r_pkv, row, NU * col + x, fbv);
+          } else {
+            bload_words<NU>(r_pkv, row + 4u * NU * col, vw[i][r]);
+          }
+        }
+      }
+      uint4 va[4][NU];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const uint32_t row = (uint32_t)min(gv_base + 4 * kg + r, gv_last) * (uint32_t)(2 * D);
+#pragma unroll
+        for (int x = 0; x < NU; ++x) va[r][x] = bload128(r_kfv, row + 16u * (NU * col + x));
+      }
+      Ws.s16[lane] = s16;
+      // the chunk's largest V scale, in binary orders above 2^kScaleExp (fp16
+      // exponent field; 0 for every scale below): p is held down by it
+      const int ev = (int)((s16 >> 26) & 31u) - 15 - kScaleExp;
+      const float emax = wave_max((float)max(ev, 0));
+
+      // ---- q'.anchor table -----------------------------------------------------------------
+      {
+        f4_t d = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int j = 0; j < NS; ++j) d = mfma32(__builtin_bit_cast(h8_t, ka[j]), lds.qn[j][lane], d);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) Ws.qa[4 * kg + r][col] = d[r];
+      }
+      wave_lds_sync();
+      // ---- scores of tokens 16i + 4kg + r, head col ------------------------------------------
+      f4_t d[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) d[i] = f4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int j = 0; j < NS; ++j) {
+        const h8_t q = lds.qc[j][lane];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) d[i] = mfma32(unpack_k(kw[i][j]), q, d[i]);
+      }
+      float sc[4][4];
+      float mx = -INFINITY;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int tb = 16 * i + 4 * kg;
+        const int4 g4 = *(const int4 *)&Ws.gkl[tb];
+        const uint4 s4 = *(const uint4 *)&Ws.s16[tb];
+        const int gr[4] = {g4.x, g4.y, g4.z, g4.w};
+        const uint32_t sr[4] = {s4.x, s4.y, s4.z, s4.w};
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const float qc = __builtin_fmaf(d[i][r], kTwo24, -sbias);  // q'.c
+          const float x = __builtin_fmaf((float)as_h2(sr[r]).x, qc, Ws.qa[gr[r]][col]) * cs;
+          sc[i][r] = tb + r < nt ? x : -INFINITY;
+          mx = fmaxf(mx, sc[i][r]);
+        }
+      }
+      // ---- lazy running max ----------------------------------------------------------------------
+      mx = shfl_max_kg(mx) + emax;
+      if (__any(mx > m_run + kTauW)) {
+        const float m_new = fmaxf(m_run, mx);
+        const float f = (m_run == -INFINITY) ? 0.f : fast_exp2(m_run - m_new);
+        l_run *= f;
+        w_run *= f;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const float fr = __shfl(f, 4 * kg + r, 64);  // factor of head 4kg + r
+#pragma unroll
+          for (int n = 0; n < NT; ++n) acc[n][r] *= fr;
+        }
+        m_run = m_new;
+      }
+      const float mref = (m_run == -INFINITY) ? 0.f : m_run;
+
+      // ---- weights as fp16 pairs, P_g --------------------------------------------------------
+      // K index 8kg + e of the products is token 16(2P) + 4kg + e (e < 4) or
+      // 16(2P+1) + 4kg + e - 4
+      f4_t pg = {0.f, 0.f, 0.f, 0.f};  // kPScale * P_g^T: groups 4kg + r, head col
+      h8_t wh[2], wl[2];
+#pragma unroll
+      for (int P = 0; P < 2; ++P) {
+        h2_t ph[2][2], pl[2][2], xh[2][2], xl[2][2];
+        uint32_t ee[2][2];
+#pragma unroll
+        for (int v = 0; v < 2; ++v) {
+          const int i = 2 * P + v, tb = 16 * i + 4 * kg;
+          const uint4 s4 = *(const uint4 *)&Ws.s16[tb];
+          const int4 g4 = *(const int4 *)&Ws.gvl[tb];
+          const uint32_t sr[4] = {s4.x, s4.y, s4.z, s4.w};
+          float p[4], w[4];
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            p[r] = fast_exp2(sc[i][r] - mref);
+            l_run += p[r];
+            w[r] = p[r] * kWScale * (float)as_h2(sr[r]).y;
+            p[r] *= kPScale;
+          }
+          split2(p[0], p[1], ph[v][0], pl[v][0]);
+          split2(p[2], p[3], ph[v][1], pl[v][1]);
+          split2(w[0], w[1], xh[v][0], xl[v][0]);
+          split2(w[2], w[3], xh[v][1], xl[v][1]);
+#pragma unroll
+          for (int x = 0; x < 2; ++x) {
+            w_run = __builtin_amdgcn_fdot2(xh[v][x], ones, w_run, false);
+            w_run = __builtin_amdgcn_fdot2(xl[v][x], ones, w_run, false);
+          }
+          // E^T: group col x these tokens (fp16 1.0 = 0x3c00)
+          ee[v][0] = (g4.x == col ? 0x3c00u : 0u) | (g4.y == col ? 0x3c000000u : 0u);
+          ee[v][1] = (g4.z == col ? 0x3c00u : 0u) | (g4.w == col ? 0x3c000000u : 0u);
+        }
+        const h8_t e8 = h8_of(ee[0][0], ee[0][1], ee[1][0], ee[1][1]);
+        pg = mfma32(e8, h8_of2(ph[0][0], ph[0][1], ph[1][0], ph[1][1]), pg);
+        pg = mfma32(e8, h8_of2(pl[0][0], pl[0][1], pl[1][0], pl[1][1]), pg);
+        wh[P] = h8_of2(xh[0][0], xh[0][1], xh[1][0], xh[1][1]);
+        wl[P] = h8_of2(xl[0][0], xl[0][1], xl[1][0], xl[1][1]);
+      }
+      h8_t pa;  // P_g hi (K index 8kg + e, e < 4: group 4kg + e) and lo (e >= 4)
+      {
+        h2_t h01, l01, h23, l23;
+        split2(pg[0], pg[1], h01, l01);
+        split2(pg[2], pg[3], h23, l23);
+        pa = h8_of2(h01, h23, l01, l23);
+      }
+      // ---- V: fields (from zero, then scaled in) and anchors -------------------------------------
+      // byte k of a word holds fields 2k (low nibble) and 2k + 1; of two tokens'
+      // words a byte permute makes one 16-bit half each, where the low nibble is
+      // the denormal n * 2^-24 and the high one 16 n * 2^-24
+#pragma unroll
+      for (int x = 0; x < NU; ++x) {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          const uint32_t sel = (uint32_t)k | (0x0cu << 8) | ((uint32_t)(4 + k) << 16) | (0x0cu << 24);
+          f4_t lo = {0.f, 0.f, 0.f, 0.f}, hi = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+          for (int P = 0; P < 2; ++P) {
+            const int i0 = 2 * P, i1 = 2 * P + 1;
+            const uint32_t a01 = __builtin_amdgcn_perm(vw[i0][1][x], vw[i0][0][x], sel);
+            const uint32_t a23 = __builtin_amdgcn_perm(vw[i0][3][x], vw[i0][2][x], sel);
+            const uint32_t b01 = __builtin_amdgcn_perm(vw[i1][1][x], vw[i1][0][x], sel);
+            const uint32_t b23 = __builtin_amdgcn_perm(vw[i1][3][x], vw[i1][2][x], sel);
+            const h8_t bl = h8_of(a01 & 0x000F000Fu, a23 & 0x000F000Fu, b01 & 0x000F000Fu, b23 & 0x000F000Fu);
+            const h8_t bh = h8_of(a01 & 0x00F000F0u, a23 & 0x00F000F0u, b01 & 0x00F000F0u, b23 & 0x00F000F0u);
+            lo = mfma32(wh[P], bl, lo);
+            lo = mfma32(wl[P], bl, lo);
+            hi = mfma32(wh[P], bh, hi);
+            hi = mfma32(wl[P], bh, hi);
+          }
+          const int n = 8 * x + 2 * k;
+          constexpr float kUp = kTwo24 * kPScale / kWScale;
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            acc[n][r] = __builtin_fmaf(lo[r], kUp, acc[n][r]);
+            acc[n + 1][r] = __builtin_fmaf(hi[r], kUp / 16.f, acc[n + 1][r]);
+          }
+          const uint4 rows[4] = {va[0][x], va[1][x], va[2][x], va[3][x]};
+          const h4_t ae = rows_operand(rows, k, false), ao = rows_operand(rows, k, true);
+          acc[n] = mfma32(pa, h8_t{ae[0], ae[1], ae[2], ae[3], ae[0], ae[1], ae[2], ae[3]}, acc[n]);
+          acc[n + 1] = mfma32(pa, h8_t{ao[0], ao[1], ao[2], ao[3], ao[0], ao[1], ao[2], ao[3]}, acc[n + 1]);
+        }
+      }
+    }
+
+    // ---- totals, workgroup merge, split epilogue -------------------------------------------------
+    l_run = shfl_sum_kg(l_run);
+    w_run = shfl_sum_kg(w_run) * (biasv / kWScale);
+    float off[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) off[r] = __shfl(w_run, 4 * kg + r, 64);
+    WideMerge<NS> &M = lds.mg;
+    constexpr int kO = WideMerge<NS>::kO;
+    __syncthreads();  // wave scratch becomes the merge area
+    if (kg == 0) {
+      M.m[wave][col] = m_run;
+      M.l[wave][col] = l_run;
+    }
+    for (int p0 = 0; p0 < gn; p0 += kMergeHeads) {
+      const int pn = min(kMergeHeads, gn - p0);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int hp = 4 * kg + r - p0;
+        if (hp >= 0 && hp < pn) {
+          float4 *dst = (float4 *)&M.t[wave][hp][8 * NU * col];
+#pragma unroll
+          for (int n = 0; n < NT; n += 4)
+            dst[n / 4] = make_float4(
+                __builtin_fmaf(acc[n][r], 1.f / kPScale, -off[r]),
+                __builtin_fmaf(acc[n + 1][r], 1.f / kPScale, -off[r]),
+                __builtin_fmaf(acc[n + 2][r], 1.f / kPScale, -off[r]),
+                __builtin_fmaf(acc[n + 3][r], 1.f / kPScale, -off[r]));
+        }
+      }
+      __syncthreads();
+      for (int e = tid; e < pn * (kO / 4); e += kThreadsMfma) {
+        const int hp = e / (kO / 4), d0 = 4 * (e - hp * (kO / 4));
+        const int hh = p0 + hp;
+        float mw[kWaves], mm = -INFINITY;
+#pragma unroll
+        for (int w = 0; w < kWaves; ++w) {
+          mw[w] = M.m[w][hh];
+          mm = fmaxf(mm, mw[w]);
+        }
+        float4 o = make_float4(0.f, 0.f, 0.f, 0.f);
+        float L = 0.f;
+#pragma unroll
+        for (int w = 0; w < kWaves; ++w) {
+          const float f = (mw[w] == -INFINITY) ? 0.f : fast_exp2(mw[w] - mm);
+          const float4 t = *(const float4 *)&M.t[w][hp][d0];
+          o.x += f * t.x;
+          o.y += f * t.y;
+          o.z += f * t.z;
+          o.w += f * t.w;
+          L += f * M.l[w][hh];
+        }
+        *(float4 *)&M.o[hh][d0] = o;
+        if (d0 == 0) {
+          M.wm[hh] = mm;
+          M.wl[hh] = L;
+        }
+      }
+      __syncthreads();
+    }
+    finish_workgroup(a, b, h, chunk, j0, gn, sg.slot, sg.live, M.wm, M.wl, &M.o[0][0], kO);
+    __syncthreads();  // the next segment's staging reuses the merge area
+  }
+}
+
+const void *wide_kernel(int D, bool dense) {
+  auto pick = [dense](const void *plain, const void *d) { return dense ? d : plain; };
+  if (D <= 64) return pick((const void *)decode_wide_kernel<2, false>, (const void *)decode_wide_kernel<2, true>);
+  if (D <= 96) return pick((const void *)decode_wide_kernel<3, false>, (const void *)decode_wide_kernel<3, true>);
+  if (D <= 128) return pick((const void *)decode_wide_kernel<4, false>, (const void *)decode_wide_kernel<4, true>);
+  return pick((const void *)decode_wide_kernel<8, false>, (const void *)decode_wide_kernel<8, true>);
+}
+
+// One 8-wave workgroup per CU (two waves per SIMD of up to 256 registers)
+int64_t wide_resident() {
+  return resident_workgroups((const void *)decode_wide_kernel<8, false>, kThreadsMfma, kSlotWide);
+}
+
+}  // namespace
+
+int64_t wide_max_resident() { return wide_resident(); }
+
+bool wide_supported(const DecodeArgs &a) {
+  if (a.D % 8 || a.D < 32) return false;
+  if (a.q_dtype != CQ_F16 && a.q_dtype != CQ_BF16) return false;
+  if (a.max_T >= (1 << 24) || a.stride[0] < 4 || a.stride[1] < 4) return false;
+  // buffer resources address each (sequence, head) region with 32-bit offsets
+  for (int i = 0; i < 2; ++i)
+    if (a.cap_kf[i] * a.D * 2 >= ((int64_t)1 << 31) ||
+        a.cap_pf[i] * 4 * row_words_of(a.D, a.fbits[i]) >= ((int64_t)1 << 31))
+      return false;
+  if ((int64_t)a.B * units_of(a.max_T) >= ((int64_t)1 << 31)) return false;  // 32-bit unit indices
+  return (((uintptr_t)a.kf[0] | (uintptr_t)a.kf[1] | (uintptr_t)a.q) & 15u) == 0;
+}
+
+int launch_decode_wide(DecodeArgs &a, void *workspace, size_t ws_bytes, hipStream_t stream) {
+  a.chunk_heads = kHeads;
+  a.n_chunks = (a.G + kHeads - 1) / kHeads;
+  const int64_t cols = (int64_t)a.H * a.n_chunks;
+  const int64_t P = std::min(std::max((int64_t)1, wide_resident() / cols),
+                             (int64_t)a.B * units_of(a.max_T));
+  a.nsplit = (int)balanced_slots(P, a.max_T);
+  a.split_len = kUnit;
+  const int st = setup_workspace(a, workspace, ws_bytes);
+  if (st) return st;
+  const dim3 grid((unsigned)P, (unsigned)cols), blk(kThreadsMfma);
+  void *args[] = {&a};
+  const void *k = wide_kernel(a.D, a.fbits[0] != 4 || a.fbits[1] != 4);
+  if (hipLaunchKernel(k, grid, blk, args, 0, stream) != hipSuccess) {
+    (void)hipGetLastError();
+    return CQ_ERR_LAUNCH;
+  }
+  return hipGetLastError() == hipSuccess ? CQ_OK : CQ_ERR_LAUNCH;
+}
+
+}  // namespace cq
