@@ -393,9 +393,20 @@ __device__ __forceinline__ void unpack8_dt(uint4 u, bool f16, float (&f)[8]) {
   }
 }
 
-// codec_row over a 16-lane row, 8 dims per lane (D = 128).
-template <int DT>
-__device__ __forceinline__ float codec_row16(float (&d)[8], int bits, float dz, int (&code)[8]) {
+// fmaxf over the LPR lanes of a row
+template <int LPR>
+__device__ __forceinline__ float lanes_fmax(float v) {
+  v = fmaxf(v, dpp_f<kDppQuadXor1>(v));
+  v = fmaxf(v, dpp_f<kDppQuadXor2>(v));
+  v = fmaxf(v, dpp_f<kDppRowHalfMirror>(v));
+  if (LPR > 8) v = fmaxf(v, dpp_f<kDppRowMirror>(v));
+  if (LPR > 16) v = fmaxf(v, __shfl_xor(v, 16, 64));
+  return v;
+}
+
+// codec_row over a row of LPR lanes, 8 dims per lane.
+template <int DT, int LPR>
+__device__ __forceinline__ float codec_row8(float (&d)[8], int bits, float dz, int (&code)[8]) {
   using T = Dt<DT>;
   const int half = (1 << bits) >> 1;
   const float hm1 = (float)(half - 1);
@@ -403,9 +414,9 @@ __device__ __forceinline__ float codec_row16(float (&d)[8], int bits, float dz, 
   float m = 0.f;
 #pragma unroll
   for (int i = 0; i < 8; ++i) m = fmaxf(m, fabsf(d[i]));
-  const float amax = row16_max(m);
+  const float amax = lanes_fmax<LPR>(m);
   float scale = T::round(amax / hm1);
-  if (dz > 0.f) {  // uniform over the row's 16 lanes
+  if (dz > 0.f) {  // uniform over the row's lanes
     const float thr = T::round(amax * T::round(dz));
     float m2 = 0.f;
 #pragma unroll
@@ -413,7 +424,7 @@ __device__ __forceinline__ float codec_row16(float (&d)[8], int bits, float dz, 
       if (fabsf(d[i]) < thr) d[i] = 0.f;
       m2 = fmaxf(m2, fabsf(d[i]));
     }
-    const float amax_c = row16_max(m2);
+    const float amax_c = lanes_fmax<LPR>(m2);
     const float amax_safe = (amax_c < eps) ? amax : amax_c;
     scale = T::round(amax_safe / hm1);
   }
@@ -500,7 +511,7 @@ __global__ __launch_bounds__(256) void append_row4_kernel(AppendArgs a) {
 #pragma unroll
       for (int i = 0; i < 8; ++i) d[i] = Dt<DT>::round(v[i] - Dt<DT>::round(an[i]));
       int code[8];
-      const float scale = codec_row16<DT>(d, bits, dz, code);
+      const float scale = codec_row8<DT, 16>(d, bits, dz, code);
       const int64_t slot = t - g - 1;
       // this lane's 8 fields (8 fb stream bits from 8 fb j); a dense row's
       // word j takes them from lanes j1 = 32j / 8fb and j1 + 1 of the row
@@ -519,6 +530,217 @@ __global__ __launch_bounds__(256) void append_row4_kernel(AppendArgs a) {
         if (j < rw) pk[(bh * cap_pf + slot) * rw + j] = word;
         if (j == 0) sc[bh * cap_pf + slot] = f2h(scale);
       }
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------
+// cq_append of a prompt or a chunk of one (16-bit tokens, head_dim a multiple of
+// 8, 16-byte aligned rows, at least kBulkTokens new tokens): LPR lanes per row
+// (the power of two >= D / 8), 8 dims per lane, 64 / LPR consecutive tokens of one
+// (component, sequence, kv head) per wave and pass, kBulkPasses passes whose loads
+// are issued together.
+//
+// The codec's results are codec_row's, bit for bit, from fewer operations:
+// * fp16 differences, absolute values and the clip are packed fp16 operations (one
+//   rounding of the exact result, as "fp32, then round" gives);
+// * a quotient R(d / s) is x = d r, x + (d - x s) r with r = 1 / s approximated once
+//   per row: within 2^-24 (1 + 2^-20) of d / s.  Only its place among the points
+//   where rint(R(.)) changes matters; those have at most 12 significant bits, so a
+//   d / s that is not one of them is at least 2^-23 away, and one that is comes out
+//   exactly.  (The same for the scale's quotient by 2^(bits-1) - 1, with room.)
+// * rint and the nibble's + 8 are one addition of 1032 to the clipped quotient;
+// * with a dead zone of at most 1 the row's largest |d| is never below the
+//   threshold, so the second maximum is the first.
+// A row that is zero, underflows the scale to zero, or holds an infinity, a NaN or
+// bf16's largest values takes codec_row8's divisions (a wave-uniform branch).
+//
+// Bound: HBM and VALU issue about alike (bf16: VALU, its roundings are not packed).
+// 16384 tokens x 8 heads x 128: fp16 48 -> 22 us, 3.8 TB/s, bf16 71 -> 30 (the
+// four-rows-per-wave kernel: a division per element and three index divisions
+// per lane); 64 dims 138 -> 13, 4 heads x 256 dims 105 -> 29 (one row per wave);
+// 8 x 32768 x 8 x 128: 693 -> 321 us, 4.3 TB/s.
+// ---------------------------------------------------------------------------
+constexpr int kBulkTokens = 16;
+constexpr int kBulkPasses = 4;
+
+typedef __bf16 bf2v_t __attribute__((ext_vector_type(2)));
+typedef float fl2_t __attribute__((ext_vector_type(2)));
+
+// maximum over the LPR lanes of a row (NaN-propagating)
+template <int LPR>
+__device__ __forceinline__ float lanes_max(float v) {
+  v = max_nn(v, dpp_f<kDppQuadXor1>(v));
+  v = max_nn(v, dpp_f<kDppQuadXor2>(v));
+  v = max_nn(v, dpp_f<kDppRowHalfMirror>(v));
+  if (LPR > 8) v = max_nn(v, dpp_f<kDppRowMirror>(v));
+  if (LPR > 16) v = xor16_max(v);
+  return v;
+}
+__device__ __forceinline__ uint32_t pk_bf16(float a, float b) {
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector(fl2_t{a, b}, bf2v_t));
+}
+__device__ __forceinline__ half2_t as_half2(uint32_t u) { return __builtin_bit_cast(half2_t, u); }
+__device__ __forceinline__ uint32_t half2_bits(half2_t h) { return __builtin_bit_cast(uint32_t, h); }
+
+// The word of 8 nibbles code + 8 of this lane's d = R(x - R(anchor)), as 4 packed
+// pairs of the dtype; scale: the row's, as fp32.  needed: the row's result is used.
+template <int DT, int LPR>
+__device__ __forceinline__ uint32_t encode8(const uint32_t (&d)[4], int bits, float dz, bool needed,
+                                            float &scale) {
+  const float hm1 = (float)((1 << (bits - 1)) - 1);
+  float a;
+  if constexpr (DT == CQ_F16) {
+    half2_t m = as_half2(d[0] & 0x7fff7fffu);
+#pragma unroll
+    for (int i = 1; i < 4; ++i) m = __builtin_elementwise_maximum(m, as_half2(d[i] & 0x7fff7fffu));
+    a = max_nn((float)m.x, (float)m.y);
+  } else {
+    a = 0.f;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      a = max_nn(a, max_nn(__uint_as_float((d[i] & 0x7fffu) << 16), __uint_as_float(d[i] & 0x7fff0000u)));
+  }
+  const float amax = lanes_max<LPR>(a);
+  const float rh = bits == 4 ? 1.f / 7.f : bits == 3 ? 1.f / 3.f : 1.f;
+  const float x0 = amax * rh;
+  const float s = Dt<DT>::round(__builtin_fmaf(__builtin_fmaf(-x0, hm1, amax), rh, x0));
+  const float eps = Dt<DT>::round(1e-10f);
+  constexpr float kTop = 1e36f;  // 1 / s stays a normal number (bf16; fp16 ends far below)
+  if (__any(needed && !(s > eps && amax < kTop && dz <= 1.f))) {
+    // (s == eps > 0 only for bf16, where s < eps alone is special: the general
+    // code is right for every row)
+    float v[8];
+    int code[8];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      v[2 * i] = DT == CQ_BF16 ? __uint_as_float(d[i] << 16) : (float)as_half2(d[i]).x;
+      v[2 * i + 1] = DT == CQ_BF16 ? __uint_as_float(d[i] & 0xffff0000u) : (float)as_half2(d[i]).y;
+    }
+    scale = codec_row8<DT, LPR>(v, bits, dz, code);
+    uint32_t w = 0;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) w |= (uint32_t)(code[i] + 8) << (4 * i);
+    return w;
+  }
+  scale = s;
+  const float thr = dz > 0.f ? Dt<DT>::round(amax * Dt<DT>::round(dz)) : 0.f;
+  const float r = __builtin_amdgcn_rcpf(s);
+  const half2_t lo = {(_Float16)(-hm1 - 1.f), (_Float16)(-hm1 - 1.f)}, hi = {(_Float16)hm1, (_Float16)hm1};
+  const half2_t bias = {(_Float16)1032.f, (_Float16)1032.f};
+  uint32_t p[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    float q[2];
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+      const float v = DT == CQ_BF16 ? __uint_as_float(k ? d[i] & 0xffff0000u : d[i] << 16)
+                                    : (float)(k ? as_half2(d[i]).y : as_half2(d[i]).x);
+      const float x = v * r;
+      q[k] = fabsf(v) < thr ? 0.f : __builtin_fmaf(__builtin_fmaf(-x, s, v), r, x);
+    }
+    half2_t h;
+    if constexpr (DT == CQ_F16) {
+      h = half2_t{(_Float16)q[0], (_Float16)q[1]};
+    } else {  // R to bf16; its values up to 8 and beyond the clip are exact in fp16
+      const uint32_t b = pk_bf16(q[0], q[1]);
+      h = half2_t{(_Float16)__uint_as_float(b << 16), (_Float16)__uint_as_float(b & 0xffff0000u)};
+    }
+    h = __builtin_elementwise_max(__builtin_elementwise_min(h, hi), lo);
+    p[i] = half2_bits(h + bias) & 0x000f000fu;
+  }
+  const uint32_t x = p[0] | (p[1] << 8), y = p[2] | (p[3] << 8);  // nibbles 0 2 1 3 by byte
+  return __builtin_amdgcn_perm(y | (y >> 12), x | (x >> 12), 0x05040100u);
+}
+
+template <int DT, int LPR>
+__global__ __launch_bounds__(256) void append_bulk_kernel(AppendArgs a) {
+  constexpr int R = 64 / LPR;  // tokens per wave and pass
+  const int lane = threadIdx.x & 63, j = lane & (LPR - 1), sub = lane / LPR;
+  const int wave = __builtin_amdgcn_readfirstlane((int)(blockIdx.x * 4 + (threadIdx.x >> 6)));
+  const int ci = (int)blockIdx.y >= a.H ? 1 : 0;
+  const int h = (int)blockIdx.y - ci * a.H, b = blockIdx.z;
+  const cq_component &c = a.comp[ci];
+  const int D = a.D, stride = c.stride, fb = field_bits(c), rw = row_words_of(D, fb);
+  const bool act = 8 * j < D;
+  const int64_t off = a.offsets ? (int64_t)a.offsets[b] : a.offset;
+  const int64_t bh = (int64_t)b * a.H + h;
+  const int64_t xbh = b * a.xs[ci][0] + h * a.xs[ci][1];
+  const uint16_t *x = (const uint16_t *)a.x[ci] + xbh + 8 * j;
+  const float inv = 1.0f / (float)stride;
+  const int s0 = wave * (R * kBulkPasses) + sub;
+  uint4 xv[kBulkPasses], av[kBulkPasses];
+  int gg[kBulkPasses];
+  bool in_new[kBulkPasses];
+#pragma unroll
+  for (int k = 0; k < kBulkPasses; ++k) {
+    const int s = s0 + R * k;
+    const bool live = s < a.S && act;
+    const int64_t t = off + s;
+    // t / stride (t < 2^24, host- or range-checked: rows past it are dropped)
+    int g = (int)((float)(int)t * inv);
+    const int rem = (int)t - g * stride;
+    g += rem < 0 ? -1 : rem >= stride ? 1 : 0;
+    gg[k] = g;
+    const int64_t ta = (int64_t)g * stride;
+    in_new[k] = ta >= off && ta <= t;
+    const int64_t ga = min((int64_t)max(g, 0), c.cap_keyframes - 1);
+    xv[k] = av[k] = uint4{0u, 0u, 0u, 0u};
+    if (live) {
+      xv[k] = *(const uint4 *)(x + (int64_t)s * a.xs[ci][2]);
+      const uint16_t *ar = in_new[k] ? x + (ta - off) * a.xs[ci][2]
+                                     : c.keyframes + (bh * c.cap_keyframes + ga) * D + 8 * j;
+      av[k] = *(const uint4 *)ar;
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < kBulkPasses; ++k) {
+    const int s = s0 + R * k;
+    const int64_t t = off + s;
+    const int g = gg[k];
+    const bool ok = s < a.S && t >= 0 && t < (1 << 24) && g < c.cap_keyframes;
+    const uint32_t xw[4] = {xv[k].x, xv[k].y, xv[k].z, xv[k].w};
+    const uint32_t aw[4] = {av[k].x, av[k].y, av[k].z, av[k].w};
+    uint32_t d[4], kf[4];  // the residual, and the token as fp16
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      if constexpr (DT == CQ_F16) {
+        kf[i] = xw[i];
+        d[i] = half2_bits(as_half2(xw[i]) - as_half2(aw[i]));
+      } else {
+        const float x0 = __uint_as_float(xw[i] << 16), x1 = __uint_as_float(xw[i] & 0xffff0000u);
+        kf[i] = half2_bits(half2_t{(_Float16)x0, (_Float16)x1});
+        // the anchor's fp16 value: rounded from the new token, or the cache's
+        const half2_t ah = in_new[k] ? half2_t{(_Float16)__uint_as_float(aw[i] << 16),
+                                               (_Float16)__uint_as_float(aw[i] & 0xffff0000u)}
+                                     : as_half2(aw[i]);
+        const uint32_t ab = pk_bf16((float)ah.x, (float)ah.y);
+        d[i] = pk_bf16(x0 - __uint_as_float(ab << 16), x1 - __uint_as_float(ab & 0xffff0000u));
+      }
+    }
+    const bool iframe = t == (int64_t)g * stride;
+    float scale;
+    uint32_t word = encode8<DT, LPR>(d, c.delta_bits, c.dead_zone, ok && !iframe, scale);
+    if (iframe) {
+      if (ok && act)
+        *(uint4 *)(c.keyframes + (bh * c.cap_keyframes + g) * D + 8 * j) = uint4{kf[0], kf[1], kf[2], kf[3]};
+    }
+    if (fb != 4) {  // dense rows: 8 fields of fb bits per lane, word j from at most two lanes
+      uint32_t f = 0;
+      const uint32_t down = 8u - (1u << (fb - 1)), m = (1u << fb) - 1u;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) f |= ((((word >> (4 * i)) & 15u) - down) & m) << (fb * i);
+      f = act ? f : 0u;
+      const int j1 = (32 * j) / (8 * fb), o = (32 * j) % (8 * fb);
+      const int row = lane & ~(LPR - 1);
+      const uint32_t lo = (uint32_t)__shfl((int)f, row + min(j1, LPR - 1), 64);
+      const uint32_t hi = (uint32_t)__shfl((int)f, row + min(j1 + 1, LPR - 1), 64);
+      word = (lo >> o) | (hi << (8 * fb - o));
+    }
+    const int64_t slot = t - g - 1;
+    if (!iframe && ok && slot < c.cap_pframes) {
+      if (j < rw) c.packed[(bh * c.cap_pframes + slot) * rw + j] = word;
+      if (j == 0) c.scales[bh * c.cap_pframes + slot] = f2h(scale);
     }
   }
 }
@@ -733,6 +955,16 @@ int validate_cache(const cq_cache_desc *c) {
 int64_t num_keyframes(int64_t n, int stride) { return n <= 0 ? 0 : (n - 1) / stride + 1; }
 int64_t num_pframes(int64_t n, int stride) { return n - num_keyframes(n, stride); }
 
+template <int DT>
+static void launch_bulk(const AppendArgs &a, hipStream_t s) {
+  const int lpr = a.D <= 64 ? 8 : a.D <= 128 ? 16 : 32;
+  const int per_group = 4 * (64 / lpr) * kBulkPasses;  // tokens per workgroup
+  const dim3 grid((unsigned)((a.S + per_group - 1) / per_group), (unsigned)(2 * a.H), (unsigned)a.B), blk(256);
+  if (lpr == 8) append_bulk_kernel<DT, 8><<<grid, blk, 0, s>>>(a);
+  else if (lpr == 16) append_bulk_kernel<DT, 16><<<grid, blk, 0, s>>>(a);
+  else append_bulk_kernel<DT, 32><<<grid, blk, 0, s>>>(a);
+}
+
 // Whether rebuild_kernel serves these operands.
 static bool rebuild_ok(const cq_component &c, int D, int64_t T, const void *out) {
   return D % 8 == 0 && T < (1 << 24) && (((uintptr_t)c.keyframes | (uintptr_t)out) & 15) == 0;
@@ -880,12 +1112,23 @@ int cq_append(const cq_cache_desc *cache, const void *keys, const int64_t *key_s
   hipStream_t s = (hipStream_t)stream;
   // head_dim 128, 16-bit tokens whose rows start 16-byte aligned, 16-byte
   // aligned keyframe rows: four rows per wave
-  const bool row4 = (dtype == CQ_F16 || dtype == CQ_BF16) && a.D == 128 &&
-                    ((key_strides[0] | key_strides[1] | key_strides[2] | value_strides[0] |
-                      value_strides[1] | value_strides[2]) & 7) == 0 &&
-                    key_strides[2] >= 0 && value_strides[2] >= 0 &&
-                    (((uintptr_t)keys | (uintptr_t)values | (uintptr_t)cache->k.keyframes |
-                      (uintptr_t)cache->v.keyframes) & 15) == 0;
+  const bool aligned8 = ((key_strides[0] | key_strides[1] | key_strides[2] | value_strides[0] |
+                          value_strides[1] | value_strides[2]) & 7) == 0 &&
+                        key_strides[2] >= 0 && value_strides[2] >= 0 &&
+                        (((uintptr_t)keys | (uintptr_t)values | (uintptr_t)cache->k.keyframes |
+                          (uintptr_t)cache->v.keyframes) & 15) == 0;
+  const bool row4 = (dtype == CQ_F16 || dtype == CQ_BF16) && a.D == 128 && aligned8;
+  // a chunk of such rows at any head_dim that is a multiple of 8 (positions below
+  // 2^24: known here, or bounded by the capacity, past which rows are dropped)
+  const bool low = offsets ? cache->k.cap_keyframes * cache->k.stride < (1 << 24) &&
+                                 cache->v.cap_keyframes * cache->v.stride < (1 << 24)
+                           : offset + n_new < (1 << 24);
+  if ((dtype == CQ_F16 || dtype == CQ_BF16) && a.D % 8 == 0 && n_new >= kBulkTokens && aligned8 &&
+      low && 2 * a.H <= 65535 && a.B <= 65535) {
+    if (dtype == CQ_F16) launch_bulk<CQ_F16>(a, s);
+    else launch_bulk<CQ_BF16>(a, s);
+    return launch_status();
+  }
   if (row4) {
     const dim3 g4((unsigned)std::min<int64_t>((items + 15) / 16, kAppendGroups));
     if (dtype == CQ_F16) append_row4_kernel<CQ_F16><<<g4, block, 0, s>>>(a);
