@@ -72,6 +72,7 @@ SIGNATURES = {
     "cq_pack_int4": ([_P, _I64, _I32, _P, _P], _I32),
     "cq_unpack_int4": ([_P, _I64, _I32, _P, _P], _I32),
     "cq_append": ([_DESC, _P, _P, _P, _P, _I32, _I64, _P, _I64, _P], _I32),
+    "cq_append_lengths": ([_DESC, _P, _P, _P, _P, _I32, _I64, _P, _I64, _P, _P], _I32),
     "cq_reconstruct": ([_DESC, _I32, _I64, _P, _P], _I32),
     "cq_decode_workspace_size": ([_I32, _I32, _I32, _I32, _I64], _SZ),
     "cq_decode_attn": ([_DESC, _P, _I32, _I32, _F, _P, _I64, _I64, _P, _I32, _P, _SZ, _P], _I32),

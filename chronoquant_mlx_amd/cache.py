@@ -329,11 +329,17 @@ class ChronoQuantCache:
             # device positions: append at pos[b], the fused decode reads
             # pos[b] + S tokens (chronoquant_sdpa serves a bound cache with
             # the fused decode only: its other paths read the host offset)
-            _lib.call("cq_append", self._descriptor(), keys.data_ptr(), ks, values.data_ptr(), vs,
-                      _lib.dtype_code(keys.dtype), S, self._dev_pos.data_ptr(), 0,
-                      _lib.stream_of(keys))
-            if self._len_owner:
-                torch.add(self._dev_pos, S, out=self._dev_len)
+            pos, lens = self._dev_pos, self._dev_len
+            # the append stores the lengths itself unless their tensor is not a
+            # plain vector beside the positions
+            stored = (self._len_owner and lens.numel() == B and lens.is_contiguous()
+                      and lens.device == keys.device
+                      and abs(lens.data_ptr() - pos.data_ptr()) >= 4 * B)
+            _lib.call("cq_append_lengths", self._descriptor(), keys.data_ptr(), ks,
+                      values.data_ptr(), vs, _lib.dtype_code(keys.dtype), S, pos.data_ptr(), 0,
+                      lens.data_ptr() if stored else None, _lib.stream_of(keys))
+            if self._len_owner and not stored:
+                torch.add(pos, S, out=lens)
             return keys, values
         self._ensure_capacity(self.offset + S)
         _lib.call("cq_append", self._descriptor(), keys.data_ptr(), ks, values.data_ptr(), vs,

@@ -173,7 +173,14 @@ struct AppendArgs {
                      // each lane's 2 elements are one aligned 32-bit load
   const int32_t *offsets;
   int64_t offset;
+  int32_t *lengths;  // optional: position + S per sequence
 };
+
+// The lengths after this append, by one thread of each sequence's first key row
+// (instead of a kernel of its own between the append and the decode).
+__device__ __forceinline__ void store_length(const AppendArgs &a, int b, int64_t off) {
+  if (a.lengths) a.lengths[b] = (int32_t)(off + a.S);
+}
 
 // n / d for 0 <= n < 2^31, d >= 1: a float estimate, then the remainder
 // brought into [0, d) (the estimate is off by at most one below 2^24 and by
@@ -309,6 +316,7 @@ __device__ __forceinline__ void load_append_row(const AppendArgs &a, int item, i
   const cq_component &c = a.comp[ci];
   const int D = a.D, E = dims_per_lane(D);
   const int64_t off = a.offsets ? (int64_t)a.offsets[b] : a.offset;
+  if (ci == 0 && h == 0 && s == 0 && lane == 0) store_length(a, b, off);
   const int64_t t = off + s;
   const int stride = c.stride;
   const int64_t g = (t >= 0 && t < 0x7fffffff) ? (int64_t)div_pos((int)t, stride)
@@ -479,6 +487,7 @@ __global__ __launch_bounds__(256) void append_row4_kernel(AppendArgs a) {
                   xs2 = ci ? a.xs[1][2] : a.xs[0][2];
 
     const int64_t off = a.offsets ? (int64_t)a.offsets[b] : a.offset;
+    if (live && ci == 0 && h == 0 && s == 0 && j == 0) store_length(a, b, off);
     const int64_t t = off + s;
     const int64_t g = (t >= 0 && t < 0x7fffffff) ? (int64_t)div_pos((int)t, stride)
                                                  : (t < 0 ? -1 : t / stride);
@@ -664,6 +673,7 @@ __global__ __launch_bounds__(256) void append_bulk_kernel(AppendArgs a) {
   const int D = a.D, stride = c.stride, fb = field_bits(c), rw = row_words_of(D, fb);
   const bool act = 8 * j < D;
   const int64_t off = a.offsets ? (int64_t)a.offsets[b] : a.offset;
+  if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) store_length(a, b, off);
   const int64_t bh = (int64_t)b * a.H + h;
   const int64_t xbh = b * a.xs[ci][0] + h * a.xs[ci][1];
   const uint16_t *x = (const uint16_t *)a.x[ci] + xbh + 8 * j;
@@ -1062,9 +1072,10 @@ int cq_unpack_int4(const uint32_t *packed, int64_t n_rows, int32_t head_dim, int
   return launch_status();
 }
 
-int cq_append(const cq_cache_desc *cache, const void *keys, const int64_t *key_strides,
-              const void *values, const int64_t *value_strides, int32_t dtype,
-              int64_t n_new, const int32_t *offsets, int64_t offset, cq_stream_t stream) {
+int cq_append_lengths(const cq_cache_desc *cache, const void *keys, const int64_t *key_strides,
+                      const void *values, const int64_t *value_strides, int32_t dtype,
+                      int64_t n_new, const int32_t *offsets, int64_t offset, int32_t *lengths,
+                      cq_stream_t stream) {
   int st = validate_cache(cache);
   if (st) return st;
   if (n_new < 0 || offset < 0) return CQ_ERR_ARG;
@@ -1103,6 +1114,7 @@ int cq_append(const cq_cache_desc *cache, const void *keys, const int64_t *key_s
           (((uintptr_t)keys | (uintptr_t)values) & 3) == 0;
   a.offsets = offsets;
   a.offset = offset;
+  a.lengths = lengths;
   // at most kAppendGroups workgroups (8 resident generations of 4-wave
   // groups on 256 CUs); each wave then takes kAppendRowsPerWave rows at a
   // time, every (grid waves)-th row
@@ -1142,6 +1154,13 @@ int cq_append(const cq_cache_desc *cache, const void *keys, const int64_t *key_s
     default: return CQ_ERR_DTYPE;
   }
   return launch_status();
+}
+
+int cq_append(const cq_cache_desc *cache, const void *keys, const int64_t *key_strides,
+              const void *values, const int64_t *value_strides, int32_t dtype,
+              int64_t n_new, const int32_t *offsets, int64_t offset, cq_stream_t stream) {
+  return cq_append_lengths(cache, keys, key_strides, values, value_strides, dtype, n_new, offsets,
+                           offset, nullptr, stream);
 }
 
 int cq_qkv_rope_append(const cq_cache_desc *cache, const void *qkv, const void *q_w,

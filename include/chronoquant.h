@@ -124,6 +124,16 @@ int cq_append(const cq_cache_desc *cache, const void *keys,
               const int64_t *value_strides, int32_t dtype, int64_t n_new,
               const int32_t *offsets, int64_t offset, cq_stream_t stream);
 
+/* cq_append that also stores each sequence's length after it, position + n_new,
+ * to lengths (device int32 [B], not overlapping offsets; NULL: not stored), for the
+ * decode that follows.  n_new == 0 stores nothing.  No counterpart in the reference
+ * (its lengths are host integers). */
+int cq_append_lengths(const cq_cache_desc *cache, const void *keys,
+                      const int64_t *key_strides, const void *values,
+                      const int64_t *value_strides, int32_t dtype, int64_t n_new,
+                      const int32_t *offsets, int64_t offset, int32_t *lengths,
+                      cq_stream_t stream);
+
 /* Full fp16 reconstruction of one component for positions [0, seq_len).
  * Replaces ChronoQuantCache._reconstruct_component (reference
  * cache.py:131-156): r = fp16(anchor + fp16(fp16(code) * scale)) for

@@ -112,3 +112,28 @@ def test_device_positions():
         for i, (x, y) in enumerate(zip(cache.state, ref.state)):
             view = torch.int16 if x.dtype == torch.float16 else torch.int32
             assert torch.equal(x[b].contiguous().view(view), y[0].contiguous().view(view)), (b, i)
+
+
+@pytest.mark.parametrize("D,S,layout", [(128, 1, "plain"), (72, 1, "plain"), (128, 16, "plain"),
+                                        (128, 1, "strided"), (128, 1, "beside"), (128, 1, "longer")])
+def test_lengths_stored_by_the_append(D, S, layout):
+    # one-row kernels, the four-row one and the chunk one; length vectors that the
+    # append cannot store to (strided, longer than the batch) come from a separate sum
+    from chronoquant_mlx_amd import ChronoQuantCache
+    B = 3
+    cache = ChronoQuantCache(stride_k=32, stride_v=8)
+    cache.update_and_fetch(*(torch.randn(B, 2, 64, D, device="cuda").half() for _ in range(2)))
+    n = B + 2 if layout == "longer" else B
+    buf = torch.full((2 * n + 2,), -1, dtype=torch.int32, device="cuda")
+    pos = buf[:n]
+    lens = buf[n:2 * n] if layout != "strided" else torch.zeros(2 * n, dtype=torch.int32, device="cuda")[::2]
+    if layout == "beside":
+        pos, lens = torch.zeros(n, dtype=torch.int32, device="cuda"), torch.zeros(n, dtype=torch.int32, device="cuda")
+    start = torch.tensor([5, 40, 17, 1, 2][:n], dtype=torch.int32, device="cuda")
+    pos.copy_(start)
+    cache.bind_device_position(pos, 128, lengths=lens)
+    new = torch.randn(B, 2, S, D, device="cuda").half()
+    cache.update_and_fetch(new, new)
+    assert torch.equal(lens, start + S) and torch.equal(pos, start)
+    if layout != "strided" and layout != "beside":
+        assert buf[2 * n:].tolist() == [-1, -1]
