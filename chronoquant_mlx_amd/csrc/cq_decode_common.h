@@ -15,6 +15,10 @@
 namespace cq {
 
 int validate_cache(const cq_cache_desc *c);
+// log-sum-exp merge of split partials [row][nsplit] into rows of D fp16 / bf16
+// values (cq_flash.hip)
+void launch_combine(bool bf16, const float *part_ml, const float *part_acc, uint16_t *out,
+                    int64_t rows, int D, int nsplit, hipStream_t s);
 int64_t num_keyframes(int64_t n, int stride);
 int64_t num_pframes(int64_t n, int stride);
 // K and V of T tokens as fp16 rows of row_dims dims (cq_codec.hip)

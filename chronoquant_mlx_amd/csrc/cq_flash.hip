@@ -450,22 +450,23 @@ void flash_kernel(FlashArgs a) {
 // Log-sum-exp merge of the splits: thread = (row, 4 dims).  Bound: reading the
 // partials once.
 template <bool Bf16>
-__global__ __launch_bounds__(256) void combine_kernel(FlashArgs a, int64_t n) {
+__global__ __launch_bounds__(256) void combine_kernel(const float *part_ml, const float *part_acc,
+                                                      uint16_t *out, int D, int nsplit, int64_t n) {
   const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (i >= n) return;
-  const int d4 = a.D / 4;
+  const int d4 = D / 4;
   const int64_t row = i / d4;
   const int d0 = 4 * (int)(i - row * d4);
-  const float2 *ml = (const float2 *)a.part_ml + row * a.nsplit;
-  const float *pa = a.part_acc + row * a.nsplit * a.D + d0;
+  const float2 *ml = (const float2 *)part_ml + row * nsplit;
+  const float *pa = part_acc + row * nsplit * D + d0;
   float M = -INFINITY;
-  for (int s = 0; s < a.nsplit; ++s) M = fmaxf(M, ml[s].x);
+  for (int s = 0; s < nsplit; ++s) M = fmaxf(M, ml[s].x);
   float Ls = 0.f;
   float4 o = make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll 4
-  for (int s = 0; s < a.nsplit; ++s) {
+  for (int s = 0; s < nsplit; ++s) {
     const float2 x = ml[s];
-    const float4 v = *(const float4 *)(pa + (int64_t)s * a.D);
+    const float4 v = *(const float4 *)(pa + (int64_t)s * D);
     const float w = (x.x == -INFINITY) ? 0.f : fast_exp2(x.x - M);
     Ls += w * x.y;
     o.x += w * v.x;
@@ -478,7 +479,7 @@ __global__ __launch_bounds__(256) void combine_kernel(FlashArgs a, int64_t n) {
   uint16_t w[4];
 #pragma unroll
   for (int e = 0; e < 4; ++e) w[e] = Bf16 ? f2bf(ov[e]) : f2h(ov[e]);
-  *(uint2 *)(a.out + row * a.D + d0) =
+  *(uint2 *)(out + row * D + d0) =
       uint2{(uint32_t)w[0] | ((uint32_t)w[1] << 16), (uint32_t)w[2] | ((uint32_t)w[3] << 16)};
 }
 
@@ -548,6 +549,15 @@ void launch_flash(const FlashArgs &a, int dp, bool masked, dim3 grid, hipStream_
 }
 
 }  // namespace
+
+void launch_combine(bool bf16, const float *part_ml, const float *part_acc, uint16_t *out,
+                    int64_t rows, int D, int nsplit, hipStream_t s) {
+  const int64_t n = rows * (D / 4);
+  const dim3 grid((unsigned)((n + 255) / 256)), blk(256);
+  if (bf16) combine_kernel<true><<<grid, blk, 0, s>>>(part_ml, part_acc, out, D, nsplit, n);
+  else combine_kernel<false><<<grid, blk, 0, s>>>(part_ml, part_acc, out, D, nsplit, n);
+}
+
 }  // namespace cq
 
 using namespace cq;
@@ -609,11 +619,8 @@ extern "C" int cq_flash_attn(const cq_cache_desc *cache, const void *q, int32_t 
   const bool masked = mask_kind == kMaskBool;
   if (q_dtype == CQ_BF16) launch_flash<true>(a, p.dp, masked, grid, s);
   else launch_flash<false>(a, p.dp, masked, grid, s);
-  if (p.nsplit > 1) {
-    const int64_t n = (int64_t)a.B * a.nq * a.L * (a.D / 4);
-    const dim3 cg((unsigned)((n + 255) / 256));
-    if (q_dtype == CQ_BF16) combine_kernel<true><<<cg, dim3(256), 0, s>>>(a, n);
-    else combine_kernel<false><<<cg, dim3(256), 0, s>>>(a, n);
-  }
+  if (p.nsplit > 1)
+    launch_combine(q_dtype == CQ_BF16, a.part_ml, a.part_acc, a.out, (int64_t)a.B * a.nq * a.L, a.D,
+                   p.nsplit, s);
   return hipGetLastError() == hipSuccess ? CQ_OK : CQ_ERR_LAUNCH;
 }

@@ -24,9 +24,8 @@
 //   3. online softmax in the log2 domain (lazy rescale beyond 2^8);
 //   4. O += P . V (8 dim tiles x 2 K-steps; two 16-key tiles per K=32 step).
 // With several splits each workgroup writes its rows' unnormalised (m, l, o)
-// to the workspace, and the last of a tile's splits to finish (a ticket on a
-// per-(sequence, kv head, tile) counter) merges them by log-sum-exp, as the
-// decode's split combine does.
+// to the workspace, and a second kernel merges them by log-sum-exp
+// (launch_combine, cq_flash.hip).
 #include <hip/hip_runtime.h>
 #include <math.h>
 
@@ -73,7 +72,6 @@ struct PrefillArgs {
   int nsplit, tiles;
   float *part_ml;      // [B][nq][n_q][nsplit][2]  (m in log2 units, l)
   float *part_acc;     // [B][nq][n_q][nsplit][D]  (real dim order)
-  uint32_t *counters;  // [B][H][tiles]
 };
 
 // bf16 q' = bf16(q * bf16(scale)) (one rounding of the exact fp32 product),
@@ -138,102 +136,34 @@ struct alignas(16) PrefillLds {
   uint16_t v[2][kKeys][kVStride];  // V block, [key][dim]
 };
 
-// Split epilogue: this workgroup's rows' (m, l, o) go to the workspace with
-// device-scope stores; the last of the tile's nsplit workgroups to take a
-// ticket folds every row's partials by log-sum-exp, writes the output and
-// resets the counter.  Row R of the tile is position p0 + R / G, head R % G;
-// lane (col, kg) of wave w holds o of rows 16w + 4kg + r at dims 16dt + col,
-// and m, l of row 16w + col.
-template <bool Bf16>
-__device__ __forceinline__ void split_epilogue(const PrefillArgs &a, int b, int h, int tile,
-                                               int split, int64_t p0, float m_run, float l_run,
+// Split epilogue: this workgroup's rows' (m, l, o) to the workspace.  Row R of the
+// tile is position p0 + R / G, head R % G; lane (col, kg) of wave w holds o of rows
+// 16w + 4kg + r at dims 16dt + col, and m, l of row 16w + col.
+// (The merge is a kernel of its own, over all CUs: the last workgroup of a tile to
+// finish used to read the tile's partials alone, nsplit x 128 KB, which is why more
+// than a few splits did not pay.  8192 keys, 32/8 heads: 64 queries 60 us then, 36
+// now; 128: 64 and 41; 256: 69 and 57; 512: 96-104 and 90-97; 32768 keys, 64: 106 and 58.)
+__device__ __forceinline__ void store_partials(const PrefillArgs &a, int b, int h, int split,
+                                               int64_t p0, float m_run, float l_run,
                                                const f4_t (&acc)[8]) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int col = lane & 15, kg = lane >> 4;
   const int G = a.G, ns = a.nsplit;
   const int64_t L = a.n_q;
-  const int64_t rows = (int64_t)a.B * a.nq * L;  // global rows (host-bounded below 2^31 / (ns D 4))
-  const __amdgpu_buffer_rsrc_t racc = make_rsrc(a.part_acc, (uint32_t)(rows * ns * kD * 4));
-  const __amdgpu_buffer_rsrc_t rml = make_rsrc(a.part_ml, (uint32_t)(rows * ns * 8));
-  auto grow = [&](int R) {  // global row of tile row R (valid position)
-    return (((int64_t)b * a.nq + h * G + R % G) * L + p0 + R / G);
+  auto part = [&](int R) {  // partial of tile row R (valid position)
+    return (((int64_t)b * a.nq + h * G + R % G) * L + p0 + R / G) * ns + split;
   };
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
     const int R = 16 * wave + 4 * kg + r;
     if (p0 + R / G < L) {
-      const uint32_t base = (uint32_t)((grow(R) * ns + split) * kD);
+      float *o = a.part_acc + part(R) * kD + col;
 #pragma unroll
-      for (int dt = 0; dt < 8; ++dt) {
-        store_dev1(racc, 4u * (base + 16 * dt + col), acc[dt][r]);
-      }
+      for (int dt = 0; dt < 8; ++dt) o[16 * dt] = acc[dt][r];
     }
   }
-  {
-    const int R = 16 * wave + col;
-    if (kg == 0 && p0 + R / G < L)
-      store_dev2(rml, (uint32_t)((grow(R) * ns + split) * 8), f2v_t{m_run, l_run});
-  }
-  __shared__ int s_last;
-  __builtin_amdgcn_s_waitcnt(0);  // this thread's partial stores are complete
-  __syncthreads();
-  uint32_t *ctr = a.counters + ((int64_t)b * a.H + h) * a.tiles + tile;
-  if (tid == 0) {
-    const uint32_t prev = __hip_atomic_fetch_add(ctr, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    s_last = (prev == (uint32_t)(ns - 1));
-  }
-  __syncthreads();
-  if (!s_last) return;
-  // fold: thread -> (row R, 4 real dims), all splits' loads issued before use
-  for (int u = tid; u < kRows * (kD / 4); u += kThreads) {
-    const int R = u / (kD / 4), d0 = 4 * (u % (kD / 4));
-    if (p0 + R / G >= L) continue;
-    const int64_t g = grow(R);
-    float M = -INFINITY, Ls = 0.f, o0 = 0.f, o1 = 0.f, o2 = 0.f, o3 = 0.f;
-    for (int s0 = 0; s0 < ns; s0 += 8) {
-      f2v_t ml[8];
-      f4v_t ov[8];
-#pragma unroll
-      for (int k = 0; k < 8; ++k) {
-        const uint32_t sp = (uint32_t)(g * ns + min(s0 + k, ns - 1));
-        ml[k] = load_dev2(rml, sp * 8u);
-        ov[k] = load_dev4(racc, (sp * (uint32_t)kD + (uint32_t)d0) * 4u);
-      }
-      float mb = M;
-#pragma unroll
-      for (int k = 0; k < 8; ++k) {
-        if (s0 + k >= ns) ml[k].x = -INFINITY;
-        mb = fmaxf(mb, ml[k].x);
-      }
-      const float mref = (mb == -INFINITY) ? 0.f : mb;
-      const float f = (M == -INFINITY) ? 0.f : fast_exp2(M - mref);
-      Ls *= f;
-      o0 *= f;
-      o1 *= f;
-      o2 *= f;
-      o3 *= f;
-#pragma unroll
-      for (int k = 0; k < 8; ++k) {
-        const float w = (ml[k].x == -INFINITY) ? 0.f : fast_exp2(ml[k].x - mref);
-        Ls += w * ml[k].y;
-        o0 += w * ov[k].x;
-        o1 += w * ov[k].y;
-        o2 += w * ov[k].z;
-        o3 += w * ov[k].w;
-      }
-      M = mb;
-    }
-    const float inv = Ls > 0.f ? 1.f / Ls : 0.f;
-    uint16_t *orow = a.out + g * kD + d0;
-    const float ov4[4] = {o0 * inv, o1 * inv, o2 * inv, o3 * inv};
-    uint16_t hv[4];
-#pragma unroll
-    for (int c = 0; c < 4; ++c)
-      hv[c] = Bf16 ? f32_to_bf16_bits(ov4[c]) : __builtin_bit_cast(uint16_t, (_Float16)ov4[c]);
-    *(uint2 *)orow = uint2{(uint32_t)hv[0] | ((uint32_t)hv[1] << 16),
-                           (uint32_t)hv[2] | ((uint32_t)hv[3] << 16)};
-  }
-  if (tid == 0) __hip_atomic_store(ctr, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  const int R = 16 * wave + col;
+  if (kg == 0 && p0 + R / G < L) *(float2 *)(a.part_ml + 2 * part(R)) = make_float2(m_run, l_run);
 }
 
 // Bf16: queries (and output) are bf16.  The reference then computes the
@@ -518,7 +448,7 @@ void prefill_mfma_kernel(PrefillArgs a) {
   // ---- output: lane (col = dim 16dt + col, kg) holds rows 4kg + r ---------------
   l_run = xor32_sum(xor16_sum(l_run));
   if (a.nsplit > 1) {
-    split_epilogue<Bf16>(a, b, h, tile, split, p0, m_run, l_run, acc);
+    store_partials(a, b, h, split, p0, m_run, l_run, acc);
     return;
   }
 #pragma unroll
@@ -547,10 +477,14 @@ using namespace cq;
 namespace cq {
 namespace {
 
-// Split plan: enough key splits that the grid fills one resident generation
-// of workgroups (several per CU), at most kMaxPrefillSplits and no more than
-// the longest tile has key blocks; 1 when the workspace bounds are exceeded.
-constexpr int kMaxPrefillSplits = 16;
+// Split plan: the key splits with the least of rounds of workgroups over the CUs
+// (one per CU) x (key blocks each + a fixed part of 4 blocks' time) + the partials'
+// round trip (kernel and memory), in units of one block (2.1 us): measured on the
+// shapes above and at 32768 keys.  (Filling at least one generation instead put 160
+// workgroups of 32 blocks on 320: two rounds, 110 us against 71 for 4 sequences of
+// 2000 tokens, 300 queries; 200 queries of 200 tokens: 29 and 14.)  1 when the workspace bounds are exceeded.
+constexpr int kMaxPrefillSplits = 32;
+constexpr int64_t kMaxPartialBytes = 256 << 20;  // the workspace is kept between calls
 
 struct PrefillPlan {
   int tiles, nsplit;
@@ -564,11 +498,15 @@ PrefillPlan prefill_plan(int64_t B, int64_t H, int64_t G, int64_t n_q, int64_t T
   const int64_t groups = (int64_t)p.tiles * H * B;
   const int64_t resident = resident_workgroups(
       reinterpret_cast<const void *>(prefill_mfma_kernel<false, true>), kThreads, kSlotPrefill);
-  int64_t ns = (resident + groups - 1) / groups;
-  ns = std::min<int64_t>(ns, kMaxPrefillSplits);
-  ns = std::min<int64_t>(ns, (T + kKeys - 1) / kKeys);
-  const int64_t rows = B * H * G * n_q;
-  if (ns < 2 || B * H * p.tiles > kMaxCounters || rows * ns * kD * 4 >= ((int64_t)1 << 31)) ns = 1;
+  const int64_t rows = B * H * G * n_q, blocks = (T + kKeys - 1) / kKeys;
+  int64_t ns = 1;
+  double best = 0;
+  for (int64_t n = 1; n <= kMaxPrefillSplits && n <= blocks; ++n) {
+    if (n > 1 && rows * n * kD * 4 > kMaxPartialBytes) break;
+    const double rounds = (double)((groups * n + resident - 1) / resident);
+    const double cost = rounds * (double)((blocks + n - 1) / n + 4) + (n > 1 ? 1.5 + 1.1e-4 * rows * n : 0.);
+    if (n == 1 || cost < best) ns = n, best = cost;
+  }
   p.nsplit = (int)ns;
   p.ws_bytes = ns > 1 ? kCounterRegion + round256((size_t)rows * ns * 8) +
                             round256((size_t)rows * ns * kD * 4)
@@ -637,13 +575,11 @@ extern "C" int cq_prefill_attn(const cq_cache_desc *cache, const void *q, int32_
   a.tiles = plan.tiles;
   a.nsplit = 1;
   a.part_ml = a.part_acc = nullptr;
-  a.counters = nullptr;
   if (plan.nsplit > 1 && workspace) {  // no workspace: one split per tile
     if ((uintptr_t)workspace & 255) return CQ_ERR_ALIGN;
     if (workspace_bytes < plan.ws_bytes) return CQ_ERR_WORKSPACE;
     const int64_t rows = (int64_t)a.B * n_q_heads * n_q;
     char *w = (char *)workspace;
-    a.counters = (uint32_t *)w;
     a.part_ml = (float *)(w + kCounterRegion);
     a.part_acc = (float *)(w + kCounterRegion + round256((size_t)rows * plan.nsplit * 8));
     a.nsplit = plan.nsplit;
@@ -659,5 +595,8 @@ extern "C" int cq_prefill_attn(const cq_cache_desc *cache, const void *q, int32_
     if (pow2) prefill_mfma_kernel<false, true><<<grid, blk, 0, s>>>(a);
     else prefill_mfma_kernel<false, false><<<grid, blk, 0, s>>>(a);
   }
+  if (a.nsplit > 1)
+    launch_combine(q_dtype == CQ_BF16, a.part_ml, a.part_acc, a.out, (int64_t)a.B * a.nq * a.n_q, kD,
+                   a.nsplit, s);
   return hipGetLastError() == hipSuccess ? CQ_OK : CQ_ERR_LAUNCH;
 }

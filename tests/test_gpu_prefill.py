@@ -170,3 +170,13 @@ def test_split_keys_match_single_pass(bf16):
     tol = 8e-3 if bf16 else 2e-3
     err = np.abs(outs[0] - outs[1]) - tol * np.abs(outs[1])
     assert err.max() <= tol, err.max()
+
+
+@pytest.mark.parametrize("B,H,G,T,L", [(1, 8, 4, 2100, 64), (1, 2, 4, 4096, 1), (4, 8, 4, 700, 130),
+                                       (1, 1, 1, 2048, 33), (2, 2, 16, 333, 333)])
+def test_split_plans(B, H, G, T, L):
+    # 32 splits of one tile; as many splits as key blocks allow; more tiles than
+    # CUs (one split); a tile with most rows empty; rows of several tiles.  The
+    # second call runs on the first one's leavings in the workspace.
+    _check(B, H, G, T, L, dict(stride_k=32, stride_v=8), seed=T)
+    _check(B, H, G, T, L, dict(stride_k=32, stride_v=8), seed=T + 1)
