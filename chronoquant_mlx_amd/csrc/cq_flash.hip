@@ -54,6 +54,8 @@ struct FlashArgs {
   uint16_t *out;          // as q
   const uint8_t *mask;    // kMaskBool: element (b, h, g, i, t) at the strides below
   int64_t ms[5];
+  int32_t *blocks;        // kMaskBool: lists of visible key blocks (scan_mask_kernel); null: all
+  int planes, nblk;       // ... [planes][tiles][1 + nblk]
   int B, H, G, nq, D, L, T;
   int causal;
   float scale;
@@ -96,12 +98,109 @@ __device__ __forceinline__ int swz_v(int p, int key) {
   return p ^ (((key & 3) << 2) | ((key >> 2) & 3));
 }
 
+// Key blocks that a 256-row tile of a boolean mask sees, as a list (its length
+// first), so that the flash kernel passes over the hidden ones: a hidden key's
+// weight is exactly 0 beside any visible one.  A tile with a row that sees no key
+// lists every block (such a row weighs all keys alike).
+// scan_mask_kernel: a workgroup per 1024 keys and 64 rows of a tile, lane = 16 keys,
+// the rows dealt to its 4 waves; masks that do not depend on the q head are read once per
+// position, and once for all kv heads when they do not depend on those.  It leaves
+// a flag per block and per (row, 1024 keys), from which list_kernel makes the list.
+// (257 queries x 2 sequences under a window of 1000 of 4001 keys: the flash kernel
+// 86 -> 35 us for 4 + 3 us of scan and list.  With a tile's rows or its keys in fewer
+// workgroups the scan's loads were one after the other: 40 and 15 us.)
+constexpr int kScanKeys = 1024, kScanRows = 64, kScanGroups = kRows / kScanRows;
+
+struct MaskScan {
+  uint8_t *blk;  // [planes][tiles][kScanGroups][chunks * kScanKeys / keys]
+  uint8_t *row;  // [planes][tiles][chunks][kRows]
+  int chunks, keys;
+};
+
+__global__ __launch_bounds__(256) void scan_mask_kernel(FlashArgs a, MaskScan m) {
+  __shared__ uint64_t s_seen[4];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int chunk = blockIdx.x / kScanGroups, group = blockIdx.x % kScanGroups;
+  const int tile = blockIdx.y, plane = blockIdx.z;
+  const int b = plane / a.H, h = plane - b * a.H;  // plane 0 stands for all of them when planes == 1
+  const int row0 = tile * kRows + group * kScanRows, end = min(row0 + kScanRows, a.G * a.L);
+  const int64_t pt = (int64_t)plane * a.tiles + tile;
+  const uint8_t *base = a.mask + b * a.ms[0] + h * a.ms[1];
+  const int k0 = chunk * kScanKeys + 16 * lane;
+  const bool whole = a.ms[4] == 1 && k0 + 16 <= a.T;
+  // with one mask row per position, step over the positions' first rows (the
+  // group's first position may begin before it)
+  const int step = a.ms[2] == 0 ? a.G : 1;
+  const int first = step == 1 ? row0 : row0 / a.G * a.G;
+  uint32_t seen = 0;
+#pragma unroll 4
+  for (int r = first + step * wave; r < end; r += 4 * step) {
+    const int pos = r / a.G, head = r - pos * a.G;
+    const uint8_t *p = base + head * a.ms[2] + (int64_t)pos * a.ms[3];
+    uint32_t w[4] = {0u, 0u, 0u, 0u};
+    if (whole) {
+      __builtin_memcpy(w, p + k0, 16);
+    } else {
+      for (int e = 0; e < 16 && k0 + e < a.T; ++e) w[0] |= p[(int64_t)(k0 + e) * a.ms[4]];
+    }
+    const uint32_t any = w[0] | w[1] | w[2] | w[3];
+    seen |= any;
+    const bool row = __any(any != 0);
+    if (lane == 0)
+      m.row[(pt * m.chunks + chunk) * kRows + group * kScanRows + max(r, row0) - row0] = row;
+  }
+  const uint64_t bal = __ballot(seen != 0);
+  if (lane == 0) s_seen[wave] = bal;
+  __syncthreads();
+  const int per = kScanKeys / m.keys, lanes = m.keys / 16;  // blocks here, lanes of a block
+  if (tid < per) {
+    const uint64_t all = s_seen[0] | s_seen[1] | s_seen[2] | s_seen[3];
+    m.blk[((pt * kScanGroups + group) * m.chunks + chunk) * per + tid] = ((all >> (lanes * tid)) & ((1ull << lanes) - 1)) != 0;
+  }
+}
+
+// One wave per (tile, plane).
+__global__ __launch_bounds__(64) void list_kernel(FlashArgs a, MaskScan m) {
+  const int lane = threadIdx.x, tile = blockIdx.x, plane = blockIdx.y;
+  const int64_t pt = (int64_t)plane * a.tiles + tile;
+  const int row0 = tile * kRows, rows = min(kRows, a.G * a.L - row0);
+  const uint8_t *flags = m.row + pt * m.chunks * kRows;
+  bool blind = false;
+  for (int i = lane; i < rows; i += 64) {
+    // the row that stands for this one: the first of its position in the group
+    const int rep = a.ms[2] == 0 ? max((row0 + i) / a.G * a.G - row0, i / kScanRows * kScanRows) : i;
+    bool sees = false;
+#pragma unroll 4
+    for (int c = 0; c < m.chunks; ++c) sees |= flags[c * kRows + rep] != 0;
+    blind |= !sees;
+  }
+  const bool all = __any(blind);
+  const int nb = m.chunks * (kScanKeys / m.keys);
+  const uint8_t *blk = m.blk + pt * kScanGroups * nb;
+  int32_t *list = a.blocks + pt * (1 + a.nblk);
+  int n = 0;
+  for (int i0 = 0; i0 < a.nblk; i0 += 64) {
+    bool on = all;
+    if (i0 + lane < a.nblk) {
+#pragma unroll
+      for (int g = 0; g < kScanGroups; ++g) on |= blk[g * nb + i0 + lane] != 0;
+    }
+    on = on && i0 + lane < a.nblk;
+    const uint64_t bal = __ballot(on);
+    if (on) list[1 + n + __popcll(bal & ((1ull << lane) - 1))] = i0 + lane;
+    n += __popcll(bal);
+  }
+  if (lane == 0) list[0] = n;
+}
+
 template <int DP>
 struct alignas(16) FlashLds {
   static constexpr int kKeys = DP > 128 ? 32 : 64;  // keys per block
-  // K-steps of a wave's q' beyond the 8 that it keeps in registers: each lane's
-  // own operands (DP = 256: O^T alone takes half of the 256 registers)
-  static constexpr int kQSteps = DP > 128 ? DP / 16 - 8 : 0;
+  // K-steps of a wave's q' beyond the 6 that it keeps in registers: each lane's
+  // own operands (DP = 256: O^T alone takes half of the 256 registers; 8 steps in
+  // registers spill 49, bf16 168 us on the shape below, 6: 148, 5: 151, 4: 151)
+  static constexpr int kQSteps = DP > 128 ? DP / 16 - 6 : 0;
   uint16_t k[2][kKeys * DP], v[2][kKeys * DP];
   uint4 q[kThreads / 64][kQSteps ? kQSteps : 1][kQSteps ? 64 : 1];
 };
@@ -117,10 +216,10 @@ struct alignas(16) FlashLds {
 // whole block, 2 x KT x DP x 2 bytes for 4 x 32 x KT x DP flops: at 128 bytes a
 // clock as long as the products), then the softmax's VALU.  512 queries of 16
 // heads over 8192 keys of 4 heads, head_dim 256, bf16 (66.6 GFLOP, and half as
-// many again for the weights' low halves): 148 us here, 171 with the rebuild
+// many again for the weights' low halves): 127 us here, 150 with the rebuild
 // (11) and the merge (12), where the reconstruct fallback's products, softmax
 // and conversions took 977; fp16 110.  257 queries x 2 sequences under a
-// boolean window over 4001 keys: 86 us, 105 in all against 803.
+// boolean window over 4001 keys: 63 us in all against 803.
 //
 // Split weights (bf16 queries): the fallback holds weights in fp32, so P enters
 // as an fp16 pair hi + lo, two products per V operand.
@@ -206,7 +305,14 @@ void flash_kernel(FlashArgs a) {
   const int lim_all = a.causal ? qbase + row0 / G : T - 1;  // ... every row sees
   const int last = min(row0 + kRows, GL) - 1;
   const int key_end = a.causal ? qbase + last / G + 1 : T;
-  const int n_all = (key_end + KT - 1) / KT;
+  // blocks in the order they are taken: all up to key_end, or the tile's list
+  const int32_t *list = nullptr;
+  if constexpr (Masked) {
+    if (a.blocks)
+      list = a.blocks + ((int64_t)(a.planes == 1 ? 0 : bh) * a.tiles + tile) * (1 + a.nblk);
+  }
+  const int n_all = list ? __builtin_amdgcn_readfirstlane(list[0]) : (key_end + KT - 1) / KT;
+  auto block_id = [&](int kb) { return list ? __builtin_amdgcn_readfirstlane(list[1 + kb]) : kb; };
   const int kb_lo = (int)((int64_t)split * n_all / a.nsplit);
   const int kb_hi = (int)((int64_t)(split + 1) * n_all / a.nsplit);
 
@@ -259,10 +365,13 @@ void flash_kernel(FlashArgs a) {
   // transpose-read rows of this lane: keys 4 half + jj (+ 8), columns 16 g + 4 c
   const int jj = (lane & 15) >> 2, g1 = (lane >> 4) & 1, c4 = lane & 3;
 
+  int id = 0, id_next = 0;  // this block's place in the keys, the next one's
   auto block = [&](int kb, auto buf_c) {
     constexpr int cur = decltype(buf_c)::value;
-    const int k0 = kb * KT;
-    if (kb + 1 < kb_hi) load_block(kb + 1);  // uniform
+    const int k0 = id * KT;
+    if (kb + 1 < kb_hi) load_block(id_next);  // uniform
+    id = id_next;
+    id_next = block_id(min(kb + 2, kb_hi - 1));
 
     // mask bytes of keys k0 + 32 kt + 8 q + 4 half .. + 3 (1: visible)
     uint32_t mb[NK][4];
@@ -400,7 +509,9 @@ void flash_kernel(FlashArgs a) {
   };
 
   if (kb_lo < kb_hi) {  // uniform
-    load_block(kb_lo);
+    id = block_id(kb_lo);
+    id_next = block_id(min(kb_lo + 1, kb_hi - 1));
+    load_block(id);
     store_block(0);
   }
   __syncthreads();
@@ -490,11 +601,13 @@ int padded_dim(int D) { return D <= 64 ? 64 : D <= 96 ? 96 : D <= 128 ? 128 : 25
 
 struct FlashPlan {
   int dp, tiles, nsplit;
-  size_t kv, ml, acc;  // bytes: K (and V) rows, partial (m, l), partial o
-  size_t bytes() const { return 2 * kv + ml + acc; }
+  int nblk, chunks;
+  size_t kv, ml, acc, lists;  // bytes: K (and V) rows, partial (m, l), partial o, block lists
+  size_t bytes() const { return 2 * kv + ml + acc + lists; }
 };
 
 constexpr int kMaxFlashSplits = 32;
+constexpr size_t kMaxListBytes = 64 << 20;
 
 // Key splits: one workgroup per CU, so the grid runs in ceil(groups * ns /
 // CUs) rounds of ceil(blocks / ns) key blocks each plus a fixed part (the
@@ -516,6 +629,12 @@ FlashPlan flash_plan(int64_t B, int64_t H, int64_t G, int64_t D, int64_t L, int6
   p.nsplit = (int)best;
   const size_t rows = (size_t)(B * H * G * L);
   p.kv = round256((size_t)(B * H * T) * p.dp * 2);
+  p.nblk = (int)blocks;
+  const int64_t chunks = (T + kScanKeys - 1) / kScanKeys;
+  p.chunks = (int)chunks;
+  p.lists = (size_t)(B * H * p.tiles) *
+            ((1 + blocks) * 4 + chunks * (kScanGroups * kScanKeys / keys + kRows));  // lists, blk, row
+  p.lists = p.lists <= kMaxListBytes ? round256(p.lists) : 0;
   p.ml = best > 1 ? round256(rows * best * 8) : 0;
   p.acc = best > 1 ? round256(rows * best * D * 4) : 0;
   return p;
@@ -613,6 +732,20 @@ extern "C" int cq_flash_attn(const cq_cache_desc *cache, const void *q, int32_t 
   a.scale = scale;
   a.nsplit = p.nsplit;
   a.tiles = p.tiles;
+  a.nblk = p.nblk;
+  a.planes = a.ms[0] == 0 && a.ms[1] == 0 ? 1 : a.B * a.H;
+  a.blocks = nullptr;
+  if (mask_kind == kMaskBool && p.lists && a.planes <= 65535 && p.tiles <= 65535) {
+    a.blocks = (int32_t *)(w + 2 * p.kv + p.ml + p.acc);
+    const size_t n = (size_t)a.planes * p.tiles;
+    MaskScan m;
+    m.chunks = p.chunks;
+    m.keys = p.dp > 128 ? 32 : 64;
+    m.blk = (uint8_t *)(a.blocks + n * (1 + p.nblk));
+    m.row = m.blk + n * kScanGroups * p.chunks * (kScanKeys / m.keys);
+    scan_mask_kernel<<<dim3((unsigned)(p.chunks * kScanGroups), (unsigned)p.tiles, (unsigned)a.planes), dim3(256), 0, s>>>(a, m);
+    list_kernel<<<dim3((unsigned)p.tiles, (unsigned)a.planes), dim3(64), 0, s>>>(a, m);
+  }
   st = launch_rebuild(*cache, seq_len, p.dp, (uint16_t *)w, (uint16_t *)(w + p.kv), s);
   if (st) return st;
   const dim3 grid((unsigned)(p.tiles * a.B * a.H * p.nsplit));

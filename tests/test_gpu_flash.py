@@ -116,6 +116,31 @@ def test_flash_mask_broadcasts_like_the_fallback(shape):
     assert_close(got.float().cpu().numpy(), ref.float().cpu().numpy())
 
 
+@pytest.mark.parametrize("G,D,L,T", [(4, 128, 77, 2100), (7, 64, 40, 333), (1, 256, 300, 1025), (16, 96, 65, 1500)])
+@pytest.mark.parametrize("kind", ["window", "padded", "one key", "blind row", "per head", "per sequence"])
+def test_flash_passes_over_hidden_blocks(kind, G, D, L, T):
+    # masks that hide whole key blocks from whole row tiles, alike for every
+    # head or not; one row that sees nothing brings every block of its tile back
+    from chronoquant_mlx_amd import attention as A
+    B, H = 2, 2
+    rng = np.random.default_rng(G)
+    cache = build_gpu_cache(_stream(rng, B, H, T, D), _stream(rng, B, H, T, D), stride_k=32, stride_v=8)
+    q = to_gpu(rng.standard_normal((B, G * H, L, D)))
+    i, t = torch.arange(T - L, T, device="cuda")[:, None], torch.arange(T, device="cuda")[None]
+    window = (i >= t) & (i < t + T // 5)
+    mask = {"window": window, "padded": (t >= T // 3) & (i >= t), "one key": t == (i * 7) % T,
+            "blind row": window & (i != T - 2),
+            "per head": window & (t % G == torch.arange(G, device="cuda").view(1, 1, G, 1, 1)),
+            "per sequence": (i >= t) & (t >= 300 * torch.arange(B, device="cuda").view(B, 1, 1, 1, 1))}[kind]
+    got = A.chronoquant_sdpa(q, None, None, cache, D ** -0.5, mask)
+    A.PREFILL_KERNEL = False
+    try:
+        ref = A.chronoquant_sdpa(q, None, None, cache, D ** -0.5, mask)
+    finally:
+        A.PREFILL_KERNEL = True
+    assert_close(got.float().cpu().numpy(), ref.float().cpu().numpy())
+
+
 def test_flash_leaves_to_the_fallback():
     # additive masks, fp32 queries, head dims that are no multiple of 8, causal
     # chunks longer than the cache, and queries that autograd follows
