@@ -151,8 +151,15 @@ def require_gpu(t: torch.Tensor) -> None:
                            "(there is no CPU fallback in the product path)")
 
 
+def raw_stream(device: torch.device) -> int:
+    """The device's current stream as a hipStream_t (without the Stream object
+    that torch.cuda.current_stream builds: 2 us a call)."""
+    index = device.index
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index)
+
+
 def stream_of(t: torch.Tensor) -> int:
-    return torch.cuda.current_stream(t.device).cuda_stream
+    return raw_stream(t.device)
 
 
 _hip = None

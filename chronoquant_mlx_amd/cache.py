@@ -50,6 +50,9 @@ def _num_pframes(num_tokens: int, stride: int) -> int:
     return num_tokens - _num_keyframes(num_tokens, stride)
 
 
+# The workspace's first 1.75 MiB are the split state that has to start as zeros
+# (include/chronoquant.h); the partials behind it may hold anything.
+_ZERO_REGION = 7 << 18
 _WORKSPACES: dict = {}
 # Workspaces replaced by larger ones.  A captured HIP graph keeps the address
 # it was captured with, so a replaced workspace is never freed.
@@ -60,7 +63,7 @@ _CAPTURE_WORKSPACES: dict = {}
 
 
 def _shared_workspace(device: torch.device, nbytes: int) -> torch.Tensor:
-    """Zero-initialised split-K workspace of the decode and prefill kernels,
+    """Split-K workspace of the decode and prefill kernels, its split state zeroed,
     one per (device, stream): the caches that run on one stream share it.
 
     The kernels return its counters to zero, so it is reused without
@@ -74,15 +77,15 @@ def _shared_workspace(device: torch.device, nbytes: int) -> torch.Tensor:
     stream's eager workspace (a graph may be replayed on another stream,
     concurrently with eager calls) and eager calls never see a capture's.
     """
-    stream = torch.cuda.current_stream(device)
-    handle = stream.cuda_stream
+    handle = _lib.raw_stream(device)
     cid = _lib.stream_capture_id(handle) if torch.cuda.is_current_stream_capturing() else None
     table = _WORKSPACES if cid is None else _CAPTURE_WORKSPACES
     key = (device.index, handle) if cid is None else (device.index, handle, cid)
     ws = table.get(key)
     if ws is None or ws.numel() < nbytes:
         old = 0 if ws is None else ws.numel()
-        new = torch.zeros(max(nbytes, 1 << 20, 2 * old), dtype=torch.uint8, device=device)
+        new = torch.empty(max(nbytes, _ZERO_REGION, 2 * old), dtype=torch.uint8, device=device)
+        new[:_ZERO_REGION].zero_()
         if ws is not None:
             _RETIRED.append(ws)
         table[key] = ws = new
@@ -268,22 +271,18 @@ class ChronoQuantCache:
         return self._codec_v
 
     def _descriptor(self) -> "_lib.CqCacheDesc":
+        # (built on every call from the cache's present state, positionally: one
+        # field store at a time costs a few us)
         B, H, D = self._shape
-        d = _lib.CqCacheDesc()
-        d.batch, d.n_kv_heads, d.head_dim = B, H, D
-        codecs = {"k": self.codec_k, "v": self._get_codec_for_v()}
-        for c in ("k", "v"):
-            comp = getattr(d, c)
-            comp.keyframes = self._kf[c].data_ptr()
-            comp.packed = self._pk[c].data_ptr()
-            comp.scales = self._sc[c].data_ptr()
-            comp.cap_keyframes = self._kf[c].shape[2]
-            comp.cap_pframes = self._pk[c].shape[2]
-            comp.stride = self._stride(c)
-            comp.delta_bits = codecs[c].delta_bits
-            comp.dead_zone = float(codecs[c].dead_zone_ratio)
-            comp.packing = self._packing(c)
-        return ctypes.byref(d)
+        codec_k, codec_v = self.codec_k, self._get_codec_for_v()
+        parts = []
+        for c, stride, codec in (("k", self.stride_k, codec_k), ("v", self.stride_v, codec_v)):
+            kf, pk = self._kf[c], self._pk[c]
+            parts.append(_lib.CqComponent(kf.data_ptr(), pk.data_ptr(), self._sc[c].data_ptr(),
+                                          kf.size(2), pk.size(2), stride, codec.delta_bits,
+                                          codec.dead_zone_ratio,
+                                          self._packing(c) if self.dense_residuals else _lib.CQ_PACK_INT4))
+        return ctypes.byref(_lib.CqCacheDesc(B, H, D, 0, *parts))
 
     def _decode_workspace(self, n_q_heads: int) -> torch.Tensor:
         B, H, D = self._shape
