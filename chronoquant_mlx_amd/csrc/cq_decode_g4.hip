@@ -1304,7 +1304,12 @@ int launch_decode_g4(DecodeArgs &a, void *workspace, size_t ws_bytes, hipStream_
   // Fold records: every split waits for the others, so the grid must be one
   // resident generation; a folder's lanes hold up to 64 splits.
   const int64_t slots = (int64_t)a.B * a.H * a.nsplit;
-  if (!balanced && a.nsplit > 1 && a.nsplit <= kMaxFoldSplits && slots <= kMaxRecSplits &&
+  // One-chunk batches of per-sequence lengths fill the CUs twice as far as their
+  // balanced partition did, so they merge by tickets, which wait for nobody (the
+  // records are 0.3 us faster at 8 sequences of up to 4096 tokens).
+  const bool waits = !(one_chunk && a.seq_lens && a.B > 1);
+  if (!waits) a.flags = nullptr;
+  if (waits && !balanced && a.nsplit > 1 && a.nsplit <= kMaxFoldSplits && slots <= kMaxRecSplits &&
       (one_chunk || slots <= resident))
     a.recs = records_of(workspace);
   if (balanced) {
