@@ -330,8 +330,13 @@ static int decode_entry(const cq_cache_desc *cache, const void *q, int32_t q_dty
   if (st) return st;
   if (allow_mfma && mfma_supported(a))
     return launch_decode_mfma(a, workspace, workspace_bytes, (hipStream_t)stream);
-  if (allow_mfma && wide_supported(a))
-    return launch_decode_wide(a, workspace, workspace_bytes, (hipStream_t)stream);
+  if (allow_mfma && wide_supported(a)) {
+    // its partition splits sequences where the portable kernel's grid plan leaves a
+    // large batch whole: without room for the partials (none given, or beyond the
+    // counters or 2^31 bytes) the portable kernel serves the call
+    st = launch_decode_wide(a, workspace, workspace_bytes, (hipStream_t)stream);
+    if (st != CQ_ERR_UNSUPPORTED && st != CQ_ERR_WORKSPACE && st != CQ_ERR_ALIGN) return st;
+  }
   return launch_generic(a, workspace, workspace_bytes, (hipStream_t)stream);
 }
 

@@ -1275,9 +1275,12 @@ int launch_decode_g4(DecodeArgs &a, void *workspace, size_t ws_bytes, hipStream_
   int64_t P = std::max((int64_t)1, resident / a.H);
   P = std::min(P, (int64_t)a.B * n_max);
   const bool dense_v = a.fbits[1] == 3;  // (K rows are INT4: mfma_supported)
-  const bool one_chunk = !dense_v && !split_tokens_override() &&
-                         n_max <= kMaxFoldSplits &&
-                         (int64_t)a.B * a.H * n_max <= g4_one_chunk_resident();
+  bool one_chunk = !dense_v && !split_tokens_override() && n_max <= kMaxFoldSplits &&
+                   (int64_t)a.B * a.H * n_max <= g4_one_chunk_resident();
+  // (without room for its partials: the plans below, which may need none)
+  if (n_max > 1 && (!workspace || ((uintptr_t)workspace & 255) ||
+                    ws_bytes < workspace_bytes_for(a.B, a.nq, a.D, (int)n_max)))
+    one_chunk = false;
   bool balanced = !one_chunk && a.seq_lens && a.B > 1;
   if (one_chunk) {
     a.nsplit = (int)n_max;

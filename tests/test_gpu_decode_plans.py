@@ -41,3 +41,30 @@ def test_one_chunk_plan_edges(B, H, T, ragged):
             continue
         ck, cv = build_oracle(k[b, :, :lens[b]], v[b, :, :lens[b]], stride_k=32, stride_v=8)
         assert_tight(outs[0][b], O.sdpa_fused(q[b], ck, cv, scale), what=f"b={b} len={lens[b]}")
+
+
+@pytest.mark.parametrize("B,G,D,T", [(32, 4, 128, 1000), (256, 1, 64, 600)])
+def test_without_a_workspace(B, G, D, T):
+    # batches that fill the device with one workgroup per sequence need no
+    # partials: without a workspace they are served whole, as the portable kernel's
+    # (the same kernel at head_dim 64; at 128 its fp16 weights give the tight bar)
+    from chronoquant_mlx_amd import ChronoQuantCache, _lib
+    H, dev = 8, torch.device("cuda")
+    g = torch.Generator(device="cuda")
+    g.manual_seed(B)
+    k, v = (torch.cumsum(torch.randn(B, H, T, D, device=dev, generator=g) * 0.1, 2).half() for _ in range(2))
+    q = torch.randn(B, G * H, D, device=dev, generator=g).half()
+    cache = ChronoQuantCache(stride_k=32, stride_v=8)
+    cache.update_and_fetch(k, v)
+    need = _lib.load().cq_decode_workspace_size(B, H, G * H, D, T)
+    ws = torch.zeros(need, dtype=torch.uint8, device=dev)
+    outs = []
+    for fn, where, size in (("cq_decode_attn", None, 0), ("cq_decode_attn_generic", ws.data_ptr(), need)):
+        out = torch.empty(B, G * H, D, device=dev)
+        _lib.call(fn, cache._descriptor(), q.data_ptr(), _lib.CQ_F16, G * H, D ** -0.5, None, T, T,
+                  out.data_ptr(), _lib.CQ_F32, where, size, _lib.stream_of(q))
+        outs.append(out.cpu().numpy())
+    if D == 64:
+        assert np.array_equal(*outs)
+    else:
+        assert_tight(*outs, what="no workspace")
