@@ -8,16 +8,14 @@
 //   score_t = q'.a_g(t) + s_t * (q'.c_t)
 //   out     = sum_g P_g a_g + sum_t (p_t s_t) c_t,   P_g = sum_{t in g} p_t
 // These shapes ran on the portable kernel, whose weights and products are fp32,
-// so no operand here holds less than fp32 needs:
-// * q' is exact in fp16 (bf16 rows scaled by a power of two first), code fields
-//   enter as fp16 denormals n * 2^-24 (exact), anchors are fp16: the scores are
-//   exact products summed in fp32;
-// * P and p*s enter as fp16 pairs hi + lo (22 bits), two products each, scaled by
-//   powers of two so that the pairs stay clear of fp16's subnormals and range;
-// * the fields are not offset by a magic constant (1024 + n would leave the
-//   accumulator 14 bits for n): a chunk's code product starts at zero and is
-//   scaled into the fp32 accumulator, and the sum of the same weights times the
-//   fields' offset comes off at the end.
+// and keep that here:
+// * scores: v_mfma_f32_16x16x32_f16 of operands that are exact in fp16 (q', bf16
+//   rows scaled by a power of two first; anchors; codes -8 .. 7), summed in fp32;
+// * P, p*s and the sums P_g stay fp32 numbers of any magnitude: the weighted sums
+//   are fp32 matrix products of them with the codes and anchors as fp32.  (fp16
+//   pairs hi + lo, whose products run 16 times as fast, hold 22 bits down to a
+//   fixed step: behind a dominant token whose V is 0 the other tokens' weights were
+//   off by 5e-4 at a gap of 10 nats.)
 //
 // Layout (NS K-steps of 32 dims, 32 NS >= D; W = D / 8 words of a row): lane (c,
 // kg) of a score operand holds words NS kg .. NS kg + NS - 1 of token c (one or
@@ -26,11 +24,14 @@
 // partition of cq_plan.h, 512-token units over one resident generation.
 //
 // Bound: the chain of a chunk (loads, two products, softmax) with two waves per
-// SIMD in flight.  4 sequences of 16001 tokens, 16/4 heads x 256 dims (82 MB): 34 us,
-// 2.4 TB/s, against 370 on the portable kernel (fp32 VALU products, 8 head slots for
-// 4 heads); 16 ragged sequences of up to 4096, 32/8 x 64: 30 against 177; one of
-// 1000, 16/4 x 256: 19 against 304.  Error of the fp32 output against binary64:
-// 0.8 to 1.4e-7 relative, the portable kernel 0.6 to 1.4e-7.
+// SIMD in flight, and the fp32 products (16x16x4: 10000 clocks of a 256-dim chunk,
+// 4x4x1: 2600).  4 sequences of 16001 tokens, 16/4 heads x 256 dims (82 MB): 44 us,
+// 1.9 TB/s, against 370 on the portable kernel (fp32 VALU products, 8 head slots for
+// 4 heads), 35 with the 22-bit pairs and 57 with 16x16x4 products for 4 heads; 8
+// heads per kv head, 16/2: 39 and 28.5 with the pairs; 16 ragged sequences of up to
+// 4096, 32/8 x 64: 38 against 177; one of 1000, 16/4 x 256: 27 against 304.
+// Error of the fp32 output against binary64, mean of 8 seeds of 4000 tokens by head
+// dim: 8.0 to 9.3e-8 relative, the portable kernel 7.4 to 9.1e-8.
 #include <hip/hip_runtime.h>
 #include <math.h>
 
@@ -41,11 +42,6 @@
 namespace cq {
 
 namespace {
-
-constexpr float kTauW = 2.f;                // lazy-rescale threshold: p <= 4
-constexpr float kPScale = 16.f;             // P_g operand scale (P_g <= 64 * 4)
-constexpr float kWScale = 512.f;            // p*s operand scale (p*s <= 4 * 16, see emax)
-constexpr int kScaleExp = 4;                // log2 of the largest scale that needs no care
 
 template <int NS>
 struct WideDims {
@@ -73,7 +69,7 @@ struct alignas(16) WideMerge {
 template <int NS>
 struct WideLds {
   h8_t qn[NS][64], qc[NS][64];  // q' of K-step j, lane (head, kg): natural order, field order
-  float cs[kHeads], qsum[kHeads];
+  float cs[kHeads];
   union {
     WideWave w[kWaves];
     WideMerge<NS> mg;
@@ -98,7 +94,7 @@ __device__ __forceinline__ void bload_words(__amdgpu_buffer_rsrc_t r, uint32_t o
 }
 
 // Dense rows: the fields of dims 8 word .. 8 word + 7 (8 fb stream bits at bit 8 fb word),
-// spread to nibbles.
+// as the nibbles code + 8 of an INT4 word.
 __device__ __forceinline__ uint32_t bload_dense(__amdgpu_buffer_rsrc_t r, uint32_t row, int word, int fb) {
   const uint32_t bit = 8u * fb * word;
   const uint32_t a = bload32(r, row + 4u * (bit >> 5)), b = bload32(r, row + 4u * (bit >> 5) + 4u);
@@ -107,19 +103,41 @@ __device__ __forceinline__ uint32_t bload_dense(__amdgpu_buffer_rsrc_t r, uint32
   uint32_t w = 0;
 #pragma unroll
   for (int k = 0; k < 8; ++k) w |= ((f >> (fb * k)) & m) << (4 * k);
-  return w;
+  return w + (8u - (1u << (fb - 1))) * 0x11111111u;  // (at most 15 each: no carry)
 }
 
-// hi + lo fp16 pair of x0, x1
-__device__ __forceinline__ void split2(float x0, float x1, h2_t &hi, h2_t &lo) {
-  hi = h2_t{(_Float16)x0, (_Float16)x1};
-  lo = h2_t{(_Float16)(x0 - (float)hi.x), (_Float16)(x1 - (float)hi.y)};
-}
-__device__ __forceinline__ h8_t h8_of2(h2_t a, h2_t b, h2_t c, h2_t d) {
+// K word (8 nibbles code + 8) -> A operand: the codes in unpack_k's order of dims.
+__device__ __forceinline__ h8_t codes_k(uint32_t w) {
+  const uint32_t m = 0x000F000Fu, magic = 0x64006400u;  // fp16 1024 in both halves
+  const h2_t bias = {(_Float16)-1032.f, (_Float16)-1032.f};
+  const h2_t a = as_h2(and_or(w, m, magic)) + bias, b = as_h2(and_or(w >> 4, m, magic)) + bias;
+  const h2_t c = as_h2(and_or(w >> 8, m, magic)) + bias, d = as_h2(and_or(w >> 12, m, magic)) + bias;
   return h8_t{a.x, a.y, b.x, b.y, c.x, c.y, d.x, d.y};
 }
+// Code e of a word of two's complement nibbles (an INT4 word ^ 0x88888888).
+__device__ __forceinline__ float code_f32(uint32_t w, int e) {
+  return (float)((int)(w << (28 - 4 * e)) >> 28);
+}
+// v_mfma_f32_16x16x4_f32: lane (c, kg) holds A[row c][kg], B[kg][col c], and C as
+// mfma32's.
+__device__ __forceinline__ f4_t mfma_f32(float a, float b, f4_t c) {
+  return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+}
+// A weighted sum's step, weights a and values b by lane (c, kg).  16 heads: the
+// product above (row = head c, summed over the 4 kg).  Up to 4 heads (Few): the 16
+// blocks of v_mfma_f32_4x4x1_f32, block = 4 adjacent lanes, whose lane c holds head c %
+// 4's weight and its own column's value and receives its column's sum for heads 0 .. 3
+// over the tokens of its kg alone: 8 clocks in place of 32 for a product whose rows
+// 4 .. 15 nobody needs.
+template <bool Few>
+__device__ __forceinline__ f4_t weigh(float a, float b, f4_t c) {
+  if constexpr (Few) return __builtin_amdgcn_mfma_f32_4x4x1f32(a, b, c, 0, 0, 0);
+  else return mfma_f32(a, b, c);
+}
 
-template <int NS, bool Dense>
+// Few: at most 4 q heads per kv head.  Score column c then belongs to head c % 4, so
+// that every lane holds the weights weigh<true> wants from it.
+template <int NS, bool Dense, bool Few>
 __global__ __launch_bounds__(kThreadsMfma) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void decode_wide_kernel(DecodeArgs a) {
   using Dm = WideDims<NS>;
@@ -157,7 +175,7 @@ void decode_wide_kernel(DecodeArgs a) {
   const float isk = a.inv_stride[0], isv = a.inv_stride[1];
   const int fbk = Dense ? a.fbits[0] : 4, fbv = Dense ? a.fbits[1] : 4;
   const uint32_t krow = 4u * row_words_of(D, fbk), vrow = 4u * row_words_of(D, fbv);
-  const float biask = (float)(1 << (fbk - 1)), biasv = (float)(1 << (fbv - 1));
+  uint32_t magic;  // fp16 1024 in both halves
 
   for (int it = 0;; ++it) {
     const int tid = thread_id();
@@ -201,13 +219,14 @@ void decode_wide_kernel(DecodeArgs a) {
     // ---- q' tables: half-wave tid / 32 = head, its lane = word ----------------------
     {
       const int hh = tid >> 5, w = tid & 31;
+      const int hq = Few ? hh & 3 : hh;  // head of column hh
       float v[8];
-      float top = 0.f, sum = 0.f;
+      float top = 0.f;
 #pragma unroll
       for (int e = 0; e < 8; ++e) v[e] = 0.f;
-      if (hh < gn && w < W) {
+      if (hq < gn && w < W) {
         const uint4 raw = *(const uint4 *)((const uint16_t *)a.q +
-                                           ((int64_t)b * a.nq + h * a.G + j0 + hh) * D + 8 * w);
+                                           ((int64_t)b * a.nq + h * a.G + j0 + hq) * D + 8 * w);
         const uint32_t x[4] = {raw.x, raw.y, raw.z, raw.w};
         if (a.q_dtype == CQ_BF16) {
           const float scb = bf2f(f2bf(a.scale));
@@ -226,24 +245,15 @@ void decode_wide_kernel(DecodeArgs a) {
         }
       }
 #pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        top = fmaxf(top, fabsf(v[e]));
-        sum += v[e];
-      }
+      for (int e = 0; e < 8; ++e) top = fmaxf(top, fabsf(v[e]));
 #pragma unroll
-      for (int x = 1; x < 32; x *= 2) {
-        top = fmaxf(top, __shfl_xor(top, x, 64));
-        sum += __shfl_xor(sum, x, 64);
-      }
+      for (int x = 1; x < 32; x *= 2) top = fmaxf(top, __shfl_xor(top, x, 64));
       // bf16: a power of two brings the row's top to [2^13, 2^14), so that the
       // fp16 form is exact down to 2^-27 of it (0, infinities, NaN: as they are)
       const int ex = (int)(__float_as_uint(top) >> 23);
       const int up = (a.q_dtype != CQ_BF16 || ex == 0 || ex == 255) ? 0 : min(127 + 13 - ex, 100);
       const float f = __uint_as_float((uint32_t)(127 + up) << 23);
-      if (w == 0) {
-        lds.cs[hh] = kLog2e * __uint_as_float((uint32_t)(127 - up) << 23);
-        lds.qsum[hh] = sum * f;
-      }
+      if (w == 0) lds.cs[hh] = kLog2e * __uint_as_float((uint32_t)(127 - up) << 23);
       if (w < 4 * NS) {
         h8_t q;
 #pragma unroll
@@ -254,15 +264,13 @@ void decode_wide_kernel(DecodeArgs a) {
       }
     }
     __syncthreads();
-    const float cs = lds.cs[col], sbias = biask * lds.qsum[col];
+    const float cs = lds.cs[col];
 
-    float m_run = -INFINITY;  // per head col, log2 units
+    float m_run = -INFINITY;  // per column's head, log2 units
     float l_run = 0.f;        // sum of p over this lane's tokens
-    float w_run = 0.f;        // sum of the p*s operands (kWScale)
-    f4_t acc[NT];             // kPScale units
+    f4_t acc[NT];             // tile 8x + e: heads 4kg + r (Few: r), dim 8 (NU col + x) + e
 #pragma unroll
     for (int n = 0; n < NT; ++n) acc[n] = f4_t{0.f, 0.f, 0.f, 0.f};
-    const h2_t ones = {(_Float16)1.f, (_Float16)1.f};
     WideWave &Ws = lds.w[wave];
 
     for (int64_t c0l = t0 + (int64_t)wave * kChunk; c0l < t1; c0l += kWaves * kChunk) {
@@ -330,15 +338,13 @@ void decode_wide_kernel(DecodeArgs a) {
       uint4 va[4][NU];
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const uint32_t row = (uint32_t)min(gv_base + 4 * kg + r, gv_last) * (uint32_t)(2 * D);
+        // groups past the chunk's last: zeros (their P_g is 0, and 0 * inf is not)
+        const int g = gv_base + 4 * kg + r;
+        const uint32_t row = g <= gv_last ? (uint32_t)g * (uint32_t)(2 * D) : 0x80000000u;
 #pragma unroll
         for (int x = 0; x < NU; ++x) va[r][x] = bload128(r_kfv, row + 16u * (NU * col + x));
       }
       Ws.s16[lane] = s16;
-      // the chunk's largest V scale, in binary orders above 2^kScaleExp (fp16
-      // exponent field; 0 for every scale below): p is held down by it
-      const int ev = (int)((s16 >> 26) & 31u) - 15 - kScaleExp;
-      const float emax = wave_max((float)max(ev, 0));
 
       // ---- q'.anchor table -----------------------------------------------------------------
       {
@@ -357,7 +363,7 @@ void decode_wide_kernel(DecodeArgs a) {
       for (int j = 0; j < NS; ++j) {
         const h8_t q = lds.qc[j][lane];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) d[i] = mfma32(unpack_k(kw[i][j]), q, d[i]);
+        for (int i = 0; i < 4; ++i) d[i] = mfma32(codes_k(kw[i][j]), q, d[i]);
       }
       float sc[4][4];
       float mx = -INFINITY;
@@ -370,22 +376,20 @@ void decode_wide_kernel(DecodeArgs a) {
         const uint32_t sr[4] = {s4.x, s4.y, s4.z, s4.w};
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          const float qc = __builtin_fmaf(d[i][r], kTwo24, -sbias);  // q'.c
-          const float x = __builtin_fmaf((float)as_h2(sr[r]).x, qc, Ws.qa[gr[r]][col]) * cs;
+          const float x = __builtin_fmaf((float)as_h2(sr[r]).x, d[i][r], Ws.qa[gr[r]][col]) * cs;
           sc[i][r] = tb + r < nt ? x : -INFINITY;
           mx = fmaxf(mx, sc[i][r]);
         }
       }
       // ---- lazy running max ----------------------------------------------------------------------
-      mx = shfl_max_kg(mx) + emax;
-      if (__any(mx > m_run + kTauW)) {
+      mx = shfl_max_kg(mx);
+      if (__any(mx > m_run + kTau)) {
         const float m_new = fmaxf(m_run, mx);
         const float f = (m_run == -INFINITY) ? 0.f : fast_exp2(m_run - m_new);
         l_run *= f;
-        w_run *= f;
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          const float fr = __shfl(f, 4 * kg + r, 64);  // factor of head 4kg + r
+          const float fr = __shfl(f, Few ? r : 4 * kg + r, 64);  // factor of acc's head r
 #pragma unroll
           for (int n = 0; n < NT; ++n) acc[n][r] *= fr;
         }
@@ -393,100 +397,53 @@ void decode_wide_kernel(DecodeArgs a) {
       }
       const float mref = (m_run == -INFINITY) ? 0.f : m_run;
 
-      // ---- weights as fp16 pairs, P_g --------------------------------------------------------
-      // K index 8kg + e of the products is token 16(2P) + 4kg + e (e < 4) or
-      // 16(2P+1) + 4kg + e - 4
-      f4_t pg = {0.f, 0.f, 0.f, 0.f};  // kPScale * P_g^T: groups 4kg + r, head col
-      h8_t wh[2], wl[2];
+      // ---- weights, P_g and the code product: K index kg of step (i, r) is token
+      // 16i + 4kg + r, whose weight for head col this lane holds -----------------------
+      f4_t pg = {0.f, 0.f, 0.f, 0.f};  // groups 4kg + r, head col
 #pragma unroll
-      for (int P = 0; P < 2; ++P) {
-        h2_t ph[2][2], pl[2][2], xh[2][2], xl[2][2];
-        uint32_t ee[2][2];
+      for (int i = 0; i < 4; ++i) {
+        const int tb = 16 * i + 4 * kg;
+        const uint4 s4 = *(const uint4 *)&Ws.s16[tb];
+        const int4 g4 = *(const int4 *)&Ws.gvl[tb];
+        const uint32_t sr[4] = {s4.x, s4.y, s4.z, s4.w};
+        const int gr[4] = {g4.x, g4.y, g4.z, g4.w};
 #pragma unroll
-        for (int v = 0; v < 2; ++v) {
-          const int i = 2 * P + v, tb = 16 * i + 4 * kg;
-          const uint4 s4 = *(const uint4 *)&Ws.s16[tb];
-          const int4 g4 = *(const int4 *)&Ws.gvl[tb];
-          const uint32_t sr[4] = {s4.x, s4.y, s4.z, s4.w};
-          float p[4], w[4];
+        for (int r = 0; r < 4; ++r) {
+          const float p = fast_exp2(sc[i][r] - mref);
+          l_run += p;
+          pg = mfma_f32(gr[r] == col ? 1.f : 0.f, p, pg);
+          const float w = p * (float)as_h2(sr[r]).y;
 #pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            p[r] = fast_exp2(sc[i][r] - mref);
-            l_run += p[r];
-            w[r] = p[r] * kWScale * (float)as_h2(sr[r]).y;
-            p[r] *= kPScale;
+          for (int x = 0; x < NU; ++x) {
+            const uint32_t c = vw[i][r][x] ^ 0x88888888u;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) acc[8 * x + e] = weigh<Few>(w, code_f32(c, e), acc[8 * x + e]);
           }
-          split2(p[0], p[1], ph[v][0], pl[v][0]);
-          split2(p[2], p[3], ph[v][1], pl[v][1]);
-          split2(w[0], w[1], xh[v][0], xl[v][0]);
-          split2(w[2], w[3], xh[v][1], xl[v][1]);
-#pragma unroll
-          for (int x = 0; x < 2; ++x) {
-            w_run = __builtin_amdgcn_fdot2(xh[v][x], ones, w_run, false);
-            w_run = __builtin_amdgcn_fdot2(xl[v][x], ones, w_run, false);
-          }
-          // E^T: group col x these tokens (fp16 1.0 = 0x3c00)
-          ee[v][0] = (g4.x == col ? 0x3c00u : 0u) | (g4.y == col ? 0x3c000000u : 0u);
-          ee[v][1] = (g4.z == col ? 0x3c00u : 0u) | (g4.w == col ? 0x3c000000u : 0u);
         }
-        const h8_t e8 = h8_of(ee[0][0], ee[0][1], ee[1][0], ee[1][1]);
-        pg = mfma32(e8, h8_of2(ph[0][0], ph[0][1], ph[1][0], ph[1][1]), pg);
-        pg = mfma32(e8, h8_of2(pl[0][0], pl[0][1], pl[1][0], pl[1][1]), pg);
-        wh[P] = h8_of2(xh[0][0], xh[0][1], xh[1][0], xh[1][1]);
-        wl[P] = h8_of2(xl[0][0], xl[0][1], xl[1][0], xl[1][1]);
       }
-      h8_t pa;  // P_g hi (K index 8kg + e, e < 4: group 4kg + e) and lo (e >= 4)
-      {
-        h2_t h01, l01, h23, l23;
-        split2(pg[0], pg[1], h01, l01);
-        split2(pg[2], pg[3], h23, l23);
-        pa = h8_of2(h01, h23, l01, l23);
-      }
-      // ---- V: fields (from zero, then scaled in) and anchors -------------------------------------
-      // byte k of a word holds fields 2k (low nibble) and 2k + 1; of two tokens'
-      // words a byte permute makes one 16-bit half each, where the low nibble is
-      // the denormal n * 2^-24 and the high one 16 n * 2^-24
+      // ---- anchors: K index kg of step r is group 4kg + r ------------------------------
 #pragma unroll
-      for (int x = 0; x < NU; ++x) {
+      for (int r = 0; r < 4; ++r) {
 #pragma unroll
-        for (int k = 0; k < 4; ++k) {
-          const uint32_t sel = (uint32_t)k | (0x0cu << 8) | ((uint32_t)(4 + k) << 16) | (0x0cu << 24);
-          f4_t lo = {0.f, 0.f, 0.f, 0.f}, hi = {0.f, 0.f, 0.f, 0.f};
+        for (int x = 0; x < NU; ++x) {
+          const uint32_t a4[4] = {va[r][x].x, va[r][x].y, va[r][x].z, va[r][x].w};
 #pragma unroll
-          for (int P = 0; P < 2; ++P) {
-            const int i0 = 2 * P, i1 = 2 * P + 1;
-            const uint32_t a01 = __builtin_amdgcn_perm(vw[i0][1][x], vw[i0][0][x], sel);
-            const uint32_t a23 = __builtin_amdgcn_perm(vw[i0][3][x], vw[i0][2][x], sel);
-            const uint32_t b01 = __builtin_amdgcn_perm(vw[i1][1][x], vw[i1][0][x], sel);
-            const uint32_t b23 = __builtin_amdgcn_perm(vw[i1][3][x], vw[i1][2][x], sel);
-            const h8_t bl = h8_of(a01 & 0x000F000Fu, a23 & 0x000F000Fu, b01 & 0x000F000Fu, b23 & 0x000F000Fu);
-            const h8_t bh = h8_of(a01 & 0x00F000F0u, a23 & 0x00F000F0u, b01 & 0x00F000F0u, b23 & 0x00F000F0u);
-            lo = mfma32(wh[P], bl, lo);
-            lo = mfma32(wl[P], bl, lo);
-            hi = mfma32(wh[P], bh, hi);
-            hi = mfma32(wl[P], bh, hi);
+          for (int e = 0; e < 8; ++e) {
+            const h2_t a2 = as_h2(a4[e >> 1]);
+            acc[8 * x + e] = weigh<Few>(pg[r], (float)(e & 1 ? a2.y : a2.x), acc[8 * x + e]);
           }
-          const int n = 8 * x + 2 * k;
-          constexpr float kUp = kTwo24 * kPScale / kWScale;
-#pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            acc[n][r] = __builtin_fmaf(lo[r], kUp, acc[n][r]);
-            acc[n + 1][r] = __builtin_fmaf(hi[r], kUp / 16.f, acc[n + 1][r]);
-          }
-          const uint4 rows[4] = {va[0][x], va[1][x], va[2][x], va[3][x]};
-          const h4_t ae = rows_operand(rows, k, false), ao = rows_operand(rows, k, true);
-          acc[n] = mfma32(pa, h8_t{ae[0], ae[1], ae[2], ae[3], ae[0], ae[1], ae[2], ae[3]}, acc[n]);
-          acc[n + 1] = mfma32(pa, h8_t{ao[0], ao[1], ao[2], ao[3], ao[0], ao[1], ao[2], ao[3]}, acc[n + 1]);
         }
       }
     }
 
     // ---- totals, workgroup merge, split epilogue -------------------------------------------------
     l_run = shfl_sum_kg(l_run);
-    w_run = shfl_sum_kg(w_run) * (biasv / kWScale);
-    float off[4];
+    if constexpr (Few) {  // the four kg's tokens
 #pragma unroll
-    for (int r = 0; r < 4; ++r) off[r] = __shfl(w_run, 4 * kg + r, 64);
+      for (int n = 0; n < NT; ++n)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) acc[n][r] = shfl_sum_kg(acc[n][r]);
+    }
     WideMerge<NS> &M = lds.mg;
     constexpr int kO = WideMerge<NS>::kO;
     __syncthreads();  // wave scratch becomes the merge area
@@ -498,16 +455,12 @@ void decode_wide_kernel(DecodeArgs a) {
       const int pn = min(kMergeHeads, gn - p0);
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const int hp = 4 * kg + r - p0;
-        if (hp >= 0 && hp < pn) {
+        const int hp = (Few ? r : 4 * kg + r) - p0;
+        if (hp >= 0 && hp < pn && (!Few || r == kg)) {
           float4 *dst = (float4 *)&M.t[wave][hp][8 * NU * col];
 #pragma unroll
           for (int n = 0; n < NT; n += 4)
-            dst[n / 4] = make_float4(
-                __builtin_fmaf(acc[n][r], 1.f / kPScale, -off[r]),
-                __builtin_fmaf(acc[n + 1][r], 1.f / kPScale, -off[r]),
-                __builtin_fmaf(acc[n + 2][r], 1.f / kPScale, -off[r]),
-                __builtin_fmaf(acc[n + 3][r], 1.f / kPScale, -off[r]));
+            dst[n / 4] = make_float4(acc[n][r], acc[n + 1][r], acc[n + 2][r], acc[n + 3][r]);
         }
       }
       __syncthreads();
@@ -545,17 +498,21 @@ void decode_wide_kernel(DecodeArgs a) {
   }
 }
 
-const void *wide_kernel(int D, bool dense) {
-  auto pick = [dense](const void *plain, const void *d) { return dense ? d : plain; };
-  if (D <= 64) return pick((const void *)decode_wide_kernel<2, false>, (const void *)decode_wide_kernel<2, true>);
-  if (D <= 96) return pick((const void *)decode_wide_kernel<3, false>, (const void *)decode_wide_kernel<3, true>);
-  if (D <= 128) return pick((const void *)decode_wide_kernel<4, false>, (const void *)decode_wide_kernel<4, true>);
-  return pick((const void *)decode_wide_kernel<8, false>, (const void *)decode_wide_kernel<8, true>);
+template <int NS>
+const void *wide_kernel(bool dense, bool few) {
+  if (few) return dense ? (const void *)decode_wide_kernel<NS, true, true> : (const void *)decode_wide_kernel<NS, false, true>;
+  return dense ? (const void *)decode_wide_kernel<NS, true, false> : (const void *)decode_wide_kernel<NS, false, false>;
+}
+const void *wide_kernel(int D, bool dense, bool few) {
+  if (D <= 64) return wide_kernel<2>(dense, few);
+  if (D <= 96) return wide_kernel<3>(dense, few);
+  if (D <= 128) return wide_kernel<4>(dense, few);
+  return wide_kernel<8>(dense, few);
 }
 
 // One 8-wave workgroup per CU (two waves per SIMD of up to 256 registers)
 int64_t wide_resident() {
-  return resident_workgroups((const void *)decode_wide_kernel<8, false>, kThreadsMfma, kSlotWide);
+  return resident_workgroups(wide_kernel<8>(false, true), kThreadsMfma, kSlotWide);
 }
 
 }  // namespace
@@ -587,7 +544,7 @@ int launch_decode_wide(DecodeArgs &a, void *workspace, size_t ws_bytes, hipStrea
   if (st) return st;
   const dim3 grid((unsigned)P, (unsigned)cols), blk(kThreadsMfma);
   void *args[] = {&a};
-  const void *k = wide_kernel(a.D, a.fbits[0] != 4 || a.fbits[1] != 4);
+  const void *k = wide_kernel(a.D, a.fbits[0] != 4 || a.fbits[1] != 4, a.G <= 4);
   if (hipLaunchKernel(k, grid, blk, args, 0, stream) != hipSuccess) {
     (void)hipGetLastError();
     return CQ_ERR_LAUNCH;

@@ -13,8 +13,8 @@ from tests.cqtest import assert_close, build_oracle, to_gpu
 
 pytestmark = pytest.mark.gpu
 
-# fp32 output.  Both kernels sum exact products (or products of 22-bit weights) in
-# fp32 over up to 1300 tokens: a few 2^-22 of the terms' size, which the outputs
+# fp32 output.  Both kernels sum products of fp32 weights in fp32 over up to 1300
+# tokens: a few 2^-22 of the terms' size, which the outputs
 # (averages of values that drift to |v| ~ 4) do not cancel below a tenth of.
 ATOL, RTOL = 2e-5, 1e-5
 
@@ -84,3 +84,63 @@ def test_shapes_left_to_the_portable_kernel(D, dtype, sk):
     q = to_gpu(rng.standard_normal((1, 4, D)), torch.float32 if dtype == "f32" else torch.float16)
     out, ref = (decode(q, cache, D ** -0.5, generic=g) for g in (False, True))
     assert torch.equal(out, ref)
+
+
+def _rows64(comp, stride, T, D):
+    """The cache's rows a + c * s of one oracle component [H, T, D], in 64 bits."""
+    kf, pk, sc = comp.active()
+    t = np.arange(T)
+    x = kf.astype(np.float64)[:, t // stride]
+    x[:, t % stride != 0] += O.unpack_int4(pk, D) * sc.astype(np.float64)[..., None]
+    return x
+
+
+@pytest.mark.parametrize("D,v_scale", [(64, 1.0), (256, 1.0), (256, 300.0), (96, 1e-4)])
+@pytest.mark.parametrize("gap", [0.0, 5.0, 10.0, 15.0, 20.5, 30.0])
+def test_weights_far_below_the_largest_keep_their_bits(gap, D, v_scale):
+    # One token's score is about `gap` above all others and its V is 0, so the output is
+    # made by the others' weights alone (v_scale 300: residual scales above 32).  Bar: p =
+    # exp2(x - m) with x and m of up to 1.45 gap, each rounded twice to 2^-24 of itself,
+    # and a few 2^-24 for exp2, the products and the sums (the v are of one sign, so
+    # nothing cancels).
+    from chronoquant_mlx_amd import ChronoQuantCache
+    from chronoquant_mlx_amd.kernels import chronoquant_sdpa_cache_kernel as decode
+    rng = np.random.default_rng(int(gap) + D)
+    H, G, T, top = 2, 4, 600, 64  # (an anchor of both components: its V is 0 exactly)
+    k = np.zeros((1, H, T, D), np.float16)
+    k[..., 0] = 0.01 * rng.standard_normal((1, H, T))
+    k[:, :, top, 0] = gap
+    v = (v_scale * rng.uniform(0.5, 1.5, (1, H, T, D))).astype(np.float16)
+    v[:, :, top] = 0
+    cache = ChronoQuantCache(stride_k=32, stride_v=8, dead_zone_v=0.0)
+    cache.update_and_fetch(to_gpu(k), to_gpu(v))
+    q = np.zeros((1, G * H, D), np.float16)
+    q[..., 0] = 1.0
+    out = decode(to_gpu(q), cache, 1.0, out_dtype=torch.float32).cpu().numpy()[0]
+    ck, cv = build_oracle(k[0], v[0], stride_k=32, stride_v=8)
+    score = _rows64(ck, 32, T, D)[..., 0]
+    w = np.exp(score - score.max(-1, keepdims=True))
+    exact = np.einsum("ht,htd->hd", w, _rows64(cv, 8, T, D)) / w.sum(-1)[:, None]
+    assert_close(out, np.repeat(exact, G, axis=0), 0.0, (gap + 2) * 2.0 ** -22, what=f"gap {gap}")
+
+
+@pytest.mark.parametrize("D", [64, 256])
+@pytest.mark.parametrize("t", [3, 8])
+def test_infinite_values_like_the_portable_kernel(t, D):
+    # a value past fp16's range makes its anchor (t = 8) or its row's scale infinite:
+    # the dims it reaches are inf or NaN as there
+    from chronoquant_mlx_amd import ChronoQuantCache
+    from chronoquant_mlx_amd.kernels import chronoquant_sdpa_cache_kernel as decode
+    rng = np.random.default_rng(t)
+    k, v = (to_gpu(rng.standard_normal((1, 1, 9, D)), torch.bfloat16) for _ in range(2))
+    v[0, 0, t, 5] = 3e38
+    cache = ChronoQuantCache(stride_k=8, stride_v=8)
+    cache.update_and_fetch(k, v)
+    q = to_gpu(rng.standard_normal((1, 4, D)), torch.bfloat16)
+    out, ref = (decode(q, cache, D ** -0.5, out_dtype=torch.float32, generic=g).cpu().numpy()
+                for g in (False, True))
+    assert np.isinf(ref[..., 5]).all()
+    fin = np.isfinite(ref)
+    assert np.array_equal(out[~fin], ref[~fin], equal_nan=True)
+    if fin.any():  # (an infinite scale times a zero code: NaN in every other dim)
+        assert_close(out[fin], ref[fin], ATOL, RTOL)
