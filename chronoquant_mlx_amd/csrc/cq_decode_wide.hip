@@ -9,8 +9,11 @@
 //   out     = sum_g P_g a_g + sum_t (p_t s_t) c_t,   P_g = sum_{t in g} p_t
 // These shapes ran on the portable kernel, whose weights and products are fp32,
 // and keep that here:
-// * scores: v_mfma_f32_16x16x32_f16 of operands that are exact in fp16 (q', bf16
-//   rows scaled by a power of two first; anchors; codes -8 .. 7), summed in fp32;
+// * scores: v_mfma_f32_16x16x32_f16 of operands that are exact in fp16 (q'; anchors;
+//   codes -8 .. 7), summed in fp32.  bf16 q' rows are scaled by a power of two first,
+//   and what a row holds below fp16's last place there, if anything, goes through
+//   products of its own (kLow; the loops they make of the score products cost 1 to 3
+//   us of these times);
 // * P, p*s and the sums P_g stay fp32 numbers of any magnitude: the weighted sums
 //   are fp32 matrix products of them with the codes and anchors as fp32.  (fp16
 //   pairs hi + lo, whose products run 16 times as fast, hold 22 bits down to a
@@ -25,11 +28,11 @@
 //
 // Bound: the chain of a chunk (loads, two products, softmax) with two waves per
 // SIMD in flight, and the fp32 products (16x16x4: 10000 clocks of a 256-dim chunk,
-// 4x4x1: 2600).  4 sequences of 16001 tokens, 16/4 heads x 256 dims (82 MB): 44 us,
-// 1.9 TB/s, against 370 on the portable kernel (fp32 VALU products, 8 head slots for
+// 4x4x1: 2600).  4 sequences of 16001 tokens, 16/4 heads x 256 dims (82 MB): 45 us,
+// 1.8 TB/s, against 370 on the portable kernel (fp32 VALU products, 8 head slots for
 // 4 heads), 35 with the 22-bit pairs and 57 with 16x16x4 products for 4 heads; 8
-// heads per kv head, 16/2: 39 and 28.5 with the pairs; 16 ragged sequences of up to
-// 4096, 32/8 x 64: 38 against 177; one of 1000, 16/4 x 256: 27 against 304.
+// heads per kv head, 16/2: 41 and 28.5 with the pairs; 16 ragged sequences of up to
+// 4096, 32/8 x 64: 41 against 177; one of 1000, 16/4 x 256: 27 against 304.
 // Error of the fp32 output against binary64, mean of 8 seeds of 4000 tokens by head
 // dim: 8.0 to 9.3e-8 relative, the portable kernel 7.4 to 9.1e-8.
 #include <hip/hip_runtime.h>
@@ -42,6 +45,8 @@
 namespace cq {
 
 namespace {
+
+constexpr float kLow = 274877906944.f;  // 2^38: scale of the low parts of bf16 q'
 
 template <int NS>
 struct WideDims {
@@ -68,8 +73,10 @@ struct alignas(16) WideMerge {
 
 template <int NS>
 struct WideLds {
-  h8_t qn[NS][64], qc[NS][64];  // q' of K-step j, lane (head, kg): natural order, field order
+  // q' of K-step j, lane (head, kg): natural order, field order; [1]: the low parts
+  h8_t qn[2][NS][64], qc[2][NS][64];
   float cs[kHeads];
+  int low[kWaves];  // whether the wave's heads have low parts
   union {
     WideWave w[kWaves];
     WideMerge<NS> mg;
@@ -248,22 +255,40 @@ void decode_wide_kernel(DecodeArgs a) {
       for (int e = 0; e < 8; ++e) top = fmaxf(top, fabsf(v[e]));
 #pragma unroll
       for (int x = 1; x < 32; x *= 2) top = fmaxf(top, __shfl_xor(top, x, 64));
-      // bf16: a power of two brings the row's top to [2^13, 2^14), so that the
-      // fp16 form is exact down to 2^-27 of it (0, infinities, NaN: as they are)
+      // bf16: a power of two brings the row's top to [2^13, 2^14), so that the fp16
+      // form is exact down to 2^-31 of it (0, infinities, NaN: as they are); what it
+      // leaves is below 2^-24, scaled by kLow exact down to 2^-69 of the top
       const int ex = (int)(__float_as_uint(top) >> 23);
       const int up = (a.q_dtype != CQ_BF16 || ex == 0 || ex == 255) ? 0 : min(127 + 13 - ex, 100);
       const float f = __uint_as_float((uint32_t)(127 + up) << 23);
       if (w == 0) lds.cs[hh] = kLog2e * __uint_as_float((uint32_t)(127 - up) << 23);
+      bool some = false;
       if (w < 4 * NS) {
-        h8_t q;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) q[e] = (_Float16)(v[e] * f);
         const int qkg = w / NS, qj = w - qkg * NS;
-        lds.qn[qj][16 * qkg + hh] = q;
-        lds.qc[qj][16 * qkg + hh] = h8_t{q[0], q[4], q[1], q[5], q[2], q[6], q[3], q[7]};
+        h8_t q, l;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const float x = v[e] * f;
+          q[e] = (_Float16)x;
+          const float rest = ex == 255 ? 0.f : x - (float)q[e];
+          l[e] = (_Float16)(rest * kLow);
+          some |= rest != 0.f;
+        }
+        auto put = [&](int i, h8_t y) {
+          lds.qn[i][qj][16 * qkg + hh] = y;
+          lds.qc[i][qj][16 * qkg + hh] = h8_t{y[0], y[4], y[1], y[5], y[2], y[6], y[3], y[7]};
+        };
+        put(0, q);
+        put(1, l);
       }
+      const bool any = __any(some);
+      if (lane == 0) lds.low[wave] = any;
     }
     __syncthreads();
+    int low = 0;
+#pragma unroll
+    for (int i = 0; i < kWaves; ++i) low |= lds.low[i];
+    low = __builtin_amdgcn_readfirstlane(low);
     const float cs = lds.cs[col];
 
     float m_run = -INFINITY;  // per column's head, log2 units
@@ -349,8 +374,12 @@ void decode_wide_kernel(DecodeArgs a) {
       // ---- q'.anchor table -----------------------------------------------------------------
       {
         f4_t d = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+        for (int i = low; i >= 0; --i) {  // (low parts first, brought back to q's scale)
 #pragma unroll
-        for (int j = 0; j < NS; ++j) d = mfma32(__builtin_bit_cast(h8_t, ka[j]), lds.qn[j][lane], d);
+          for (int j = 0; j < NS; ++j) d = mfma32(__builtin_bit_cast(h8_t, ka[j]), lds.qn[i][j][lane], d);
+          if (i) d *= 1.f / kLow;
+        }
 #pragma unroll
         for (int r = 0; r < 4; ++r) Ws.qa[4 * kg + r][col] = d[r];
       }
@@ -359,11 +388,21 @@ void decode_wide_kernel(DecodeArgs a) {
       f4_t d[4];
 #pragma unroll
       for (int i = 0; i < 4; ++i) d[i] = f4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+      for (int i1 = low; i1 >= 0; --i1) {
 #pragma unroll
-      for (int j = 0; j < NS; ++j) {
-        const h8_t q = lds.qc[j][lane];
+        for (int j = 0; j < NS; ++j) {
+          const h8_t q = lds.qc[i1][j][lane];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) d[i] = mfma32(codes_k(kw[i][j]), q, d[i]);
+          for (int i = 0; i < 4; ++i) {
+            asm volatile("" : "+v"(kw[i][j]));  // (keeps the unpacked words out of registers)
+            d[i] = mfma32(codes_k(kw[i][j]), q, d[i]);
+          }
+        }
+        if (i1) {
+#pragma unroll
+          for (int i = 0; i < 4; ++i) d[i] *= 1.f / kLow;
+        }
       }
       float sc[4][4];
       float mx = -INFINITY;

@@ -144,3 +144,21 @@ def test_infinite_values_like_the_portable_kernel(t, D):
     assert np.array_equal(out[~fin], ref[~fin], equal_nan=True)
     if fin.any():  # (an infinite scale times a zero code: NaN in every other dim)
         assert_close(out[fin], ref[fin], ATOL, RTOL)
+
+
+@pytest.mark.parametrize("D,G,top", [(64, 1, 33), (80, 4, 45), (256, 4, 60), (256, 8, 33)])
+def test_bf16_queries_of_any_spread(D, G, top):
+    # an element of 2^top meets keys that are 0 there: the scores come from the others,
+    # far below fp16's range beside it
+    from chronoquant_mlx_amd import ChronoQuantCache
+    from chronoquant_mlx_amd.kernels import chronoquant_sdpa_cache_kernel as decode
+    rng = np.random.default_rng(D + top)
+    k, v = (rng.standard_normal((1, 2, 200, D)) for _ in range(2))
+    k[..., D // 2] = 0
+    cache = ChronoQuantCache(stride_k=32, stride_v=8)
+    cache.update_and_fetch(to_gpu(k), to_gpu(v))
+    q = rng.standard_normal((1, 2 * G, D))
+    q[:, ::2, D // 2] = 2.0 ** top
+    q = to_gpu(q, torch.bfloat16)
+    out, ref = (decode(q, cache, 1.0, out_dtype=torch.float32, generic=g).cpu().numpy() for g in (False, True))
+    assert_close(out, ref, ATOL, RTOL)
