@@ -41,10 +41,17 @@ typedef short s4_t __attribute__((ext_vector_type(4)));
 
 constexpr int kRows = 256;     // query rows per workgroup
 constexpr int kThreads = 512;  // 8 waves of 32 rows
-constexpr float kTau = 8.f;    // lazy-rescale threshold, log2 units
-// Weights are kept at up to 2^(kTau + kLift) = 2^14, so that the fp16 operand
-// (and the low half of the split one) stays clear of fp16's subnormals.
-constexpr float kLift = 6.f;
+// Lazy-rescale threshold and lift of the weights, log2 units: fp16 queries' weights
+// (one fp16 operand) are kept at up to 2^14 and clear of fp16's subnormals for 20
+// binary orders below the running maximum; bf16 queries' (split ones) at up to 2^15,
+// with both halves clear of them for 15 to 16.
+template <bool Bf16>
+struct Weights {
+  static constexpr float kTau = Bf16 ? 1.f : 8.f;
+  static constexpr float kLift = Bf16 ? 14.f : 6.f;
+};
+constexpr float kFull = 0.25f;         // a weight whose fp16 pair hi + lo holds 23 bits
+constexpr float kUp = 274877906944.f;  // 2^38: scale of what a pair leaves of a smaller one
 
 enum MaskKind { kMaskNone = 0, kMaskCausal = 1, kMaskBool = 2 };
 
@@ -198,8 +205,8 @@ template <int DP>
 struct alignas(16) FlashLds {
   static constexpr int kKeys = DP > 128 ? 32 : 64;  // keys per block
   // K-steps of a wave's q' beyond the 6 that it keeps in registers: each lane's
-  // own operands (DP = 256: O^T alone takes half of the 256 registers; 8 steps in
-  // registers spill 49, bf16 168 us on the shape below, 6: 148, 5: 151, 4: 151)
+  // own operands (DP = 256: O^T alone takes half of the 256 registers; with 8 steps
+  // in registers the masked bf16 instance spills)
   static constexpr int kQSteps = DP > 128 ? DP / 16 - 6 : 0;
   uint16_t k[2][kKeys * DP], v[2][kKeys * DP];
   uint4 q[kThreads / 64][kQSteps ? kQSteps : 1][kQSteps ? 64 : 1];
@@ -216,13 +223,20 @@ struct alignas(16) FlashLds {
 // whole block, 2 x KT x DP x 2 bytes for 4 x 32 x KT x DP flops: at 128 bytes a
 // clock as long as the products), then the softmax's VALU.  512 queries of 16
 // heads over 8192 keys of 4 heads, head_dim 256, bf16 (66.6 GFLOP, and half as
-// many again for the weights' low halves): 127 us here, 150 with the rebuild
-// (11) and the merge (12), where the reconstruct fallback's products, softmax
-// and conversions took 977; fp16 110.  257 queries x 2 sequences under a
-// boolean window over 4001 keys: 63 us in all against 803.
+// many again for the weights' low halves), with the rebuild (11) and the merge
+// (12): 157 us where few scores lie 11 nats below their row's maximum (below), 193
+// with outlier channels in the keys, 273 with scores of a spread of 16, where the
+// reconstruct fallback's products, softmax and conversions took 977; fp16 112.  257
+// fp16 queries x 2 sequences under a boolean window over 4001 keys: 59 us in all
+// against 803; bf16 74.
 //
 // Split weights (bf16 queries): the fallback holds weights in fp32, so P enters
-// as an fp16 pair hi + lo, two products per V operand.
+// as an fp16 pair hi + lo, two products per V operand; a pair holds 23 bits of a
+// weight of at least kFull, 2^-16 or less of the largest.  What it leaves of smaller
+// ones goes through a round of products of its own, scaled by kUp, and a second one
+// (23 bits down to 2^-92 of the largest, some down to 2^-115): tokens behind a
+// dominant one whose V is 0 are off by 9 % at a gap of 25 nats without them.  A block
+// with no score 11 nats below its row's maximum needs no round.
 template <int DP, bool Bf16, bool Masked>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void flash_kernel(FlashArgs a) {
@@ -362,8 +376,21 @@ void flash_kernel(FlashArgs a) {
 #pragma unroll
     for (int r = 0; r < 16; ++r) acc[dt][r] = 0.f;
 
-  // transpose-read rows of this lane: keys 4 half + jj (+ 8), columns 16 g + 4 c
+  // This lane's operands in a block.  K: rows 32 kt + r32, piece 2s + half.  V (transpose
+  // reads): keys 16 j + 4 half + jj (+ 8), columns 32 dt + 16 g + 4 c.  The swizzles are
+  // the same for every kt and j, and for rows of a power of two of bytes a step's place
+  // is the first one's with s or dt brought in by an exclusive or.  At 256 dims the 48
+  // places are made anew from it at each use: kept, they and the accumulators leave too
+  // few of the 256 registers for the rest (40 to 144 bytes of spills per lane, a block's
+  // loads among them).
   const int jj = (lane & 15) >> 2, g1 = (lane >> 4) & 1, c4 = lane & 3;
+  constexpr bool kPow2 = PR != 12, kAnew = DP > 128;
+  auto k_at = [&](int s) { return r32 * DP + 8 * swz_k<PR>(2 * s + half, r32); };
+  auto v_at = [&](int dt, int more) {
+    const int key = 4 * half + jj + more;
+    return key * DP + 8 * swz_v<PR>(4 * dt + 2 * g1 + (c4 >> 1), key) + 4 * (c4 & 1);
+  };
+  int k_first = k_at(0), v_first = v_at(0, 0);
 
   int id = 0, id_next = 0;  // this block's place in the keys, the next one's
   auto block = [&](int kb, auto buf_c) {
@@ -405,10 +432,10 @@ void flash_kernel(FlashArgs a) {
       f16v_t d;
 #pragma unroll
       for (int r = 0; r < 16; ++r) d[r] = 0.f;
-      const int key = 32 * kt + r32;
+      if constexpr (kAnew) asm volatile("" : "+v"(k_first));
 #pragma unroll
       for (int s = 0; s < NS; ++s) {
-        const uint4 kv = *(const uint4 *)&lds.k[cur][key * DP + 8 * swz_k<PR>(2 * s + half, key)];
+        const uint4 kv = *(const uint4 *)&lds.k[cur][32 * kt * DP + (kPow2 ? k_first ^ (16 * s) : k_at(s))];
         const h8_t q8 = s < NR ? qf[s < NR ? s : 0] : __builtin_bit_cast(h8_t, lds.q[wave][s < NR ? 0 : s - NR][Lds::kQSteps ? lane : 0]);
         d = mfma(__builtin_bit_cast(h8_t, kv), q8, d);
       }
@@ -458,7 +485,7 @@ void flash_kernel(FlashArgs a) {
     }
     mx = xor32_max(mx);
     // ---- lazy running max ----------------------------------------------------------
-    if (__any(mx > m_run + kTau)) {
+    if (__any(mx > m_run + Weights<Bf16>::kTau)) {
       const float m_new = fmaxf(m_run, mx);
       const float f = (m_run == -INFINITY) ? 0.f : fast_exp2(m_run - m_new);
       l_run *= f;
@@ -468,8 +495,48 @@ void flash_kernel(FlashArgs a) {
         for (int r = 0; r < 16; ++r) acc[dt][r] *= f;
       m_run = m_new;
     }
-    const float mref = ((m_run == -INFINITY) ? 0.f : m_run) - kLift;
+    const float mref = ((m_run == -INFINITY) ? 0.f : m_run) - Weights<Bf16>::kLift;
+    bool deep = false;  // a weight below kFull (uniform; 0s count as well)
+    if constexpr (Bf16) {
+      float mn = sc[0][0];
+#pragma unroll
+      for (int kt = 0; kt < NK; ++kt)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) mn = fminf(mn, sc[kt][r]);
+      deep = __any(mn < mref - 2.f);
+    }
     // ---- weights and P.V, 16 keys a step --------------------------------------------
+    // (tight: V operands one at a time, as the registers of a rare round allow)
+    auto product = [&](int j, const h2_t (&ph)[4], const h2_t (&pl)[4], bool tight) {
+      const h8_t bh8 = __builtin_bit_cast(h8_t, uint4{as_u(ph[0]), as_u(ph[1]), as_u(ph[2]), as_u(ph[3])});
+      h8_t bl8;
+      if constexpr (Bf16)
+        bl8 = __builtin_bit_cast(h8_t, uint4{as_u(pl[0]), as_u(pl[1]), as_u(pl[2]), as_u(pl[3])});
+      if constexpr (kAnew) asm volatile("" : "+v"(v_first));
+      const uint16_t *v16 = &lds.v[cur][16 * j * DP];
+#pragma unroll
+      for (int dt = 0; dt < ND; ++dt) {
+        const int at = kPow2 ? v_first ^ (32 * dt) : v_at(dt, 0);
+        // 8 keys on: the swizzle's third bit turns, where it has one
+        const int at2 = kAnew ? (at ^ 16) + 8 * DP : v_at(dt, 8);
+        const uint2 v1 = lds_read_tr16(v16 + at);
+        const uint2 v2 = lds_read_tr16(v16 + at2);
+        const h8_t va = __builtin_bit_cast(h8_t, uint4{v1.x, v1.y, v2.x, v2.y});
+        acc[dt] = mfma(va, bh8, acc[dt]);
+        if constexpr (Bf16) acc[dt] = mfma(va, bl8, acc[dt]);
+        if (tight) __builtin_amdgcn_sched_barrier(0);
+      }
+    };
+    // the fp16 pair of x0, x1; rest: what it leaves of those below kFull
+    auto split = [&](float &x0, float &x1, h2_t &hi, h2_t &lo, bool rest) {
+      hi = __builtin_convertvector(f2_t{x0, x1}, h2_t);
+      const float d0 = x0 - (float)hi.x, d1 = x1 - (float)hi.y;
+      lo = __builtin_convertvector(f2_t{d0, d1}, h2_t);
+      if (rest) {
+        x0 = fabsf(x0) < kFull ? d0 - (float)lo.x : 0.f;
+        x1 = fabsf(x1) < kFull ? d1 - (float)lo.y : 0.f;
+      }
+    };
     const h2_t ones = {(_Float16)1.f, (_Float16)1.f};
 #pragma unroll
     for (int j = 0; j < KT / 16; ++j) {
@@ -478,10 +545,10 @@ void flash_kernel(FlashArgs a) {
       for (int i = 0; i < 4; ++i) {
         const int kt = j >> 1, r = 8 * (j & 1) + 2 * i;
         if constexpr (Bf16) {
-          const float p0 = fast_exp2(sc[kt][r] - mref), p1 = fast_exp2(sc[kt][r + 1] - mref);
+          float p0 = fast_exp2(sc[kt][r] - mref), p1 = fast_exp2(sc[kt][r + 1] - mref);
           l_run += p0 + p1;
-          ph[i] = __builtin_convertvector(f2_t{p0, p1}, h2_t);
-          pl[i] = __builtin_convertvector(f2_t{p0 - (float)ph[i].x, p1 - (float)ph[i].y}, h2_t);
+          split(p0, p1, ph[i], pl[i], deep);
+          if (deep) sc[kt][r] = p0, sc[kt][r + 1] = p1;
         } else {
           const h2_t x = s2[kt][r >> 1];
           ph[i] = h2_t{(_Float16)fast_exp2(__builtin_fmaf((float)x.x, kLog2e, -mref)),
@@ -489,19 +556,43 @@ void flash_kernel(FlashArgs a) {
           l_run = __builtin_amdgcn_fdot2(ph[i], ones, l_run, false);
         }
       }
-      const h8_t bh8 = __builtin_bit_cast(h8_t, uint4{as_u(ph[0]), as_u(ph[1]), as_u(ph[2]), as_u(ph[3])});
-      h8_t bl8;
-      if constexpr (Bf16)
-        bl8 = __builtin_bit_cast(h8_t, uint4{as_u(pl[0]), as_u(pl[1]), as_u(pl[2]), as_u(pl[3])});
-      const int key1 = 16 * j + 4 * half + jj, key2 = key1 + 8;
+      product(j, ph, pl, false);
+    }
+    if constexpr (Bf16) {
+      // the rests, kUp larger a round, into acc as much larger: |acc| <= 2^48 (2^15 a
+      // weight, 2^16 a value, 2^17 keys) stays a number in both rounds
+      float down = 1.f;
+#pragma unroll 1
+      for (int round = deep ? 0 : 2; round < 2; ++round) {
+        float any = 0.f;
 #pragma unroll
-      for (int dt = 0; dt < ND; ++dt) {
-        const int p = 4 * dt + 2 * g1 + (c4 >> 1);
-        const uint2 v1 = lds_read_tr16(&lds.v[cur][key1 * DP + 8 * swz_v<PR>(p, key1) + 4 * (c4 & 1)]);
-        const uint2 v2 = lds_read_tr16(&lds.v[cur][key2 * DP + 8 * swz_v<PR>(p, key2) + 4 * (c4 & 1)]);
-        const h8_t va = __builtin_bit_cast(h8_t, uint4{v1.x, v1.y, v2.x, v2.y});
-        acc[dt] = mfma(va, bh8, acc[dt]);
-        if constexpr (Bf16) acc[dt] = mfma(va, bl8, acc[dt]);
+        for (int kt = 0; kt < NK; ++kt)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) any = fmaxf(any, fabsf(sc[kt][r]));
+        if (!__any(any > 0.f)) break;
+        down *= 1.f / kUp;
+#pragma unroll
+        for (int dt = 0; dt < ND; ++dt)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) acc[dt][r] *= kUp;
+#pragma unroll
+        for (int j = 0; j < KT / 16; ++j) {
+          h2_t ph[4], pl[4];
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const int kt = j >> 1, r = 8 * (j & 1) + 2 * i;
+            sc[kt][r] *= kUp;
+            sc[kt][r + 1] *= kUp;
+            split(sc[kt][r], sc[kt][r + 1], ph[i], pl[i], true);
+          }
+          product(j, ph, pl, true);
+        }
+      }
+      if (down != 1.f) {
+#pragma unroll
+        for (int dt = 0; dt < ND; ++dt)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) acc[dt][r] *= down;
       }
     }
     if (kb + 1 < kb_hi) store_block(cur ^ 1);

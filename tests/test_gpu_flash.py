@@ -76,27 +76,53 @@ def test_flash_matches_fallback(H, G, D, T, L, mask, params, dtype):
     assert_close(out.float().cpu().numpy()[0], ref.astype(np.float64), what=f"{dtype} {mask}")
 
 
-def test_flash_bf16_weights_keep_32_bits():
-    # One dominant and many small weights: with the weights rounded to fp16 the
-    # small ones (2^-16 of the top one) would be off by up to 2^-9 each; the
-    # split pair holds them to 2^-20.  V rows of the small ones share a sign, so
-    # their errors add up.  Bar: one bf16 rounding of the output (2^-9) on the
-    # part the small ones make, which the fallback in fp32 meets too.
+def _cancelling_scores(depth):
+    """(a, b): two fp16 scores about `depth` below 0 whose weights differ by 2^-5 and,
+    held in fp16 alone (the largest weight at 2^14), are off by most of half a place
+    each in opposite directions."""
+    c = -depth - np.arange(0, 2000) * 2.0 ** -10
+    c = np.unique(c.astype(np.float16).astype(np.float64))
+    p = np.exp(c)
+    if depth > 20:  # (below fp16's range beside the largest: any will do)
+        return c[-1], c[np.argmin(np.abs(c[-1] - c - 2.0 ** -5))]
+    off = (p * 2.0 ** 14).astype(np.float16).astype(np.float64) * 2.0 ** -14 / p - 1
+    for x in np.argsort(-off):
+        near = np.flatnonzero(np.abs(c[x] - c - 2.0 ** -5) < 2.0 ** -6)
+        if near.size and off[near].min() < -0.7 * off[x]:
+            return c[x], c[near[np.argmin(off[near])]]
+
+
+@pytest.mark.parametrize("depth", [2, 8, 14, 20, 40, 60])
+@pytest.mark.parametrize("D", [64, 80, 128, 256])
+def test_flash_bf16_weights_keep_32_bits(D, depth):
+    # A dominant key of V = 0, then 200 keys of V = 1 and 200 of V = -1 whose weights
+    # nearly cancel: the output is 2^-5 of what either group makes.  Bar: the output's
+    # rounding to bf16 (2^-8), and 2^5 times the weights' error in fp32 arithmetic (scores
+    # of up to 87 in binary orders, each rounded to 2^-24 of itself: 2^-17).  Weights held
+    # in fp16 miss it, and so do fp16 pairs (23 bits, down to 2^-24 beside a largest
+    # weight of 2^14) from a depth of 20 on.
     from chronoquant_mlx_amd import ChronoQuantCache, kernels
-    T, D = 4096, 64
-    rng = np.random.default_rng(3)
-    k = np.zeros((1, 1, T, D), np.float16)
-    k[..., 0] = rng.uniform(-0.25, 0.25, T)
-    v = np.ones((1, 1, T, D), np.float16)
-    k[0, 0, 0, 0], v[0, 0, 0] = 11, 0
+    n = 200
+    a, b = _cancelling_scores(depth)
+    score = np.concatenate([[0.0], np.full(n, a), np.full(n, b)])
+    value = np.concatenate([[0.0], np.ones(n), -np.ones(n)])
+    order = np.concatenate([[0], 1 + np.random.default_rng(depth).permutation(2 * n)])
+    score, value = score[order], value[order]
+    w = np.exp(score)
+    exact = (w * value).sum() / w.sum()
+    bar = (2.0 ** -8 + 2.0 ** -12) * abs(exact)
+    hi = (w * 2.0 ** 14).astype(np.float16).astype(np.float64)
+    lo = (w * 2.0 ** 14 - hi).astype(np.float16).astype(np.float64)
+    for kept, enough in ((hi, False), (hi + lo, depth < 20)):
+        assert (abs((kept * value).sum() / (w.sum() * 2.0 ** 14) - exact) < bar) == enough
+    k, v = np.zeros((1, 1, 2 * n + 1, D), np.float16), np.zeros((1, 1, 2 * n + 1, D), np.float16)
+    k[0, 0, :, 0], v[0, 0] = score, value[:, None]
     cache = ChronoQuantCache(stride_k=1, stride_v=1)
     cache.update_and_fetch(to_gpu(k), to_gpu(v))
-    q = torch.zeros(1, 1, 2, D, dtype=torch.bfloat16, device="cuda")
+    q = torch.zeros(1, 2, 2, D, dtype=torch.bfloat16, device="cuda")
     q[..., 0] = 1.0
     out = kernels.chronoquant_flash_kernel(q, cache, 1.0, None).double().cpu().numpy()
-    w = np.exp(k[0, 0, :, 0].astype(np.float64))
-    exact = w[1:].sum() / w.sum()
-    assert np.all(np.abs(out - exact) <= 2.0 ** -9 * exact), (out.ravel()[0], exact)
+    assert np.all(np.abs(out - exact) <= bar), (out.ravel()[0], exact)
 
 
 @pytest.mark.parametrize("shape", [(1, 1, 1, 9, 70), (1, 2, 1, 9, 70), (2, 2, 3, 9, 70), (9, 1), (70,)])
