@@ -263,31 +263,38 @@ void flash_kernel(FlashArgs a) {
 
   // ---- q' (B operand of the score product): dims 16s + 8 half .. + 7 ---------
   // bf16: scaled by a power of two that brings the row's largest magnitude to
-  // [2^13, 2^14), so that its fp16 form loses no bit down to 2^-27 of that;
-  // cs takes the scores back, in log2 units.
+  // [2^13, 2^14), so that its fp16 form loses no bit down to 2^-31 of that;
+  // cs takes the scores back, in log2 units.  low: a row of this wave has elements
+  // that lose bits (a block's score products then begin with theirs).
   h8_t qf[NR];
   float cs = kLog2e;
+  bool low = false;
+  auto raw_of = [&](int s) {
+    const int d0 = 16 * s + 8 * half;
+    return (valid && d0 < a.D) ? *(const uint4 *)(a.q + grow * a.D + d0) : uint4{0u, 0u, 0u, 0u};
+  };
+  // element e of 8 of a bf16 row, as q' times f; what its fp16 form loses
+  auto scaled = [&](const uint4 &u, int e, float f) {
+    const uint32_t w = e < 2 ? u.x : e < 4 ? u.y : e < 6 ? u.z : u.w;
+    const float x = __uint_as_float(e & 1 ? w & 0xffff0000u : w << 16);
+    return bf2f(f2bf(x * bf2f(f2bf(a.scale)))) * f;
+  };
+  auto lost = [](float x) {
+    const float h = (float)(_Float16)x;
+    return fabsf(h) < INFINITY ? x - h : 0.f;
+  };
   {
-    const uint16_t *qrow = a.q + grow * a.D;
-    auto raw_of = [&](int s) {
-      const int d0 = 16 * s + 8 * half;
-      return (valid && d0 < a.D) ? *(const uint4 *)(qrow + d0) : uint4{0u, 0u, 0u, 0u};
-    };
     auto keep = [&](int s, h8_t v) {
       if (s < NR) qf[s] = v;
       else lds.q[wave][s - NR][Lds::kQSteps ? lane : 0] = __builtin_bit_cast(uint4, v);
     };
     if constexpr (Bf16) {
-      const float scb = bf2f(f2bf(a.scale));
       float top = 0.f;
 #pragma unroll
       for (int s = 0; s < NS; ++s) {
         const uint4 u = raw_of(s);
-        const uint32_t w[4] = {u.x, u.y, u.z, u.w};
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
-          top = fmaxf(top, fmaxf(fabsf(bf2f(f2bf(__uint_as_float(w[i] << 16) * scb))),
-                                 fabsf(bf2f(f2bf(__uint_as_float(w[i] & 0xffff0000u) * scb)))));
+        for (int e = 0; e < 8; ++e) top = fmaxf(top, fabsf(scaled(u, e, 1.f)));
       }
       top = xor32_max(top);
       const int e = (int)(__float_as_uint(top) >> 23);  // biased exponent
@@ -295,18 +302,20 @@ void flash_kernel(FlashArgs a) {
       const int up = (e == 0 || e == 255) ? 0 : min(127 + 13 - e, 100);
       const float f = __uint_as_float((uint32_t)(127 + up) << 23);
       cs = kLog2e * __uint_as_float((uint32_t)(127 - up) << 23);
+      float left = 0.f;
 #pragma unroll
       for (int s = 0; s < NS; ++s) {
         const uint4 u = raw_of(s);  // (again: the rows are in cache, registers are not)
-        const uint32_t w[4] = {u.x, u.y, u.z, u.w};
         h8_t v;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          v[2 * i] = (_Float16)(bf2f(f2bf(__uint_as_float(w[i] << 16) * scb)) * f);
-          v[2 * i + 1] = (_Float16)(bf2f(f2bf(__uint_as_float(w[i] & 0xffff0000u) * scb)) * f);
+        for (int e = 0; e < 8; ++e) {
+          const float x = scaled(u, e, f);
+          v[e] = (_Float16)x;
+          left = fmaxf(left, fabsf(lost(x)));
         }
         keep(s, v);
       }
+      low = __any(left > 0.f);
     } else {
 #pragma unroll
       for (int s = 0; s < NS; ++s) keep(s, __builtin_bit_cast(h8_t, raw_of(s)) * (_Float16)a.scale);
@@ -432,6 +441,21 @@ void flash_kernel(FlashArgs a) {
       f16v_t d;
 #pragma unroll
       for (int r = 0; r < 16; ++r) d[r] = 0.f;
+      if constexpr (Bf16) {
+        if (low) {  // (below 2^-24; scaled by kUp exact down to 2^-69 of the row's largest)
+#pragma unroll 1
+          for (int s = 0; s < NS; ++s) {
+            const uint4 kv = *(const uint4 *)&lds.k[cur][32 * kt * DP + k_at(s)];
+            const uint4 u = raw_of(s);
+            h8_t v;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) v[e] = (_Float16)(lost(scaled(u, e, kLog2e / cs)) * kUp);
+            d = mfma(__builtin_bit_cast(h8_t, kv), v, d);
+          }
+#pragma unroll
+          for (int r = 0; r < 16; ++r) d[r] *= 1.f / kUp;
+        }
+      }
       if constexpr (kAnew) asm volatile("" : "+v"(k_first));
 #pragma unroll
       for (int s = 0; s < NS; ++s) {

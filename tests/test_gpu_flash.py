@@ -186,3 +186,26 @@ def test_flash_leaves_to_the_fallback():
         assert out.requires_grad == q.requires_grad
     q = to_gpu(rng.standard_normal((1, H, T + 1, 12)))
     assert kernels.chronoquant_flash_kernel(q, cache, 1.0, "causal") is None
+
+
+@pytest.mark.parametrize("D,top", [(64, 33), (80, 45), (128, 60), (256, 33)])
+def test_flash_bf16_queries_of_any_spread(D, top):
+    # an element of 2^top meets keys that are 0 there: the scores come from the others,
+    # far below fp16's range beside it.  Against the fallback (fp32 products), one
+    # rounding of the output to bf16 apart.
+    from chronoquant_mlx_amd import chronoquant_sdpa, kernels
+    from chronoquant_mlx_amd import attention as A
+    rng = np.random.default_rng(D + top)
+    k, v = (rng.standard_normal((1, 2, 200, D)) for _ in range(2))
+    k[..., D // 2] = 0
+    cache = build_gpu_cache(k, v, stride_k=32, stride_v=8)
+    q = rng.standard_normal((1, 8, 9, D))
+    q[:, ::2, :, D // 2] = 2.0 ** top
+    q = to_gpu(q, torch.bfloat16)
+    got = kernels.chronoquant_flash_kernel(q, cache, D ** -0.5, "causal")
+    A.PREFILL_KERNEL = False
+    try:
+        ref = chronoquant_sdpa(q, None, None, cache, D ** -0.5, "causal")
+    finally:
+        A.PREFILL_KERNEL = True
+    assert_close(got.float().cpu().numpy(), ref.float().cpu().numpy(), 1e-3, 2.0 ** -7)
