@@ -231,8 +231,8 @@ def prefill_supported(queries: torch.Tensor, cache, mask) -> bool:
 
 
 def _differentiated(t: torch.Tensor) -> bool:
-    """Whether autograd, forward-mode AD or a functorch transform follows t:
-    what is computed from it then has to stay torch ops."""
+    """Whether autograd, forward-mode AD, a functorch transform or a tensor subclass
+    follows t: what is computed from it then has to stay torch ops."""
     return ((torch.is_grad_enabled() and t.requires_grad) or type(t) is not torch.Tensor
             or torch._C._functorch.is_functorch_wrapped_tensor(t)
             or torch.autograd.forward_ad.unpack_dual(t).tangent is not None)
@@ -259,7 +259,7 @@ def chronoquant_flash_kernel(q: torch.Tensor, cache, scale: float, mask) -> torc
             return None
         kind = 1
     else:
-        if mask.dtype != torch.bool:
+        if mask.dtype != torch.bool or _differentiated(mask):
             return None
         mask = mask.to(q.device)
         try:

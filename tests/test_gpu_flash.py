@@ -209,3 +209,16 @@ def test_flash_bf16_queries_of_any_spread(D, top):
     finally:
         A.PREFILL_KERNEL = True
     assert_close(got.float().cpu().numpy(), ref.float().cpu().numpy(), 1e-3, 2.0 ** -7)
+
+
+def test_flash_masks_under_vmap():
+    # a mask that a transform follows has no storage of its own: torch ops, as before
+    from chronoquant_mlx_amd import chronoquant_sdpa
+    rng = np.random.default_rng(0)
+    cache = build_gpu_cache(_stream(rng, 1, 2, 40, 64), _stream(rng, 1, 2, 40, 64), stride_k=32, stride_v=8)
+    q = to_gpu(rng.standard_normal((1, 4, 5, 64)))
+    masks = torch.from_numpy(rng.random((3, 5, 40)) > 0.4).cuda()
+    out = torch.vmap(lambda m: chronoquant_sdpa(q, None, None, cache, 0.125, m))(masks)
+    for i in range(3):
+        ref = chronoquant_sdpa(q, None, None, cache, 0.125, masks[i])
+        assert_close(out[i].float().cpu().numpy(), ref.float().cpu().numpy())
