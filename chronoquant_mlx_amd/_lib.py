@@ -22,6 +22,7 @@ CQ_ERR_TIMEOUT = 10
 CQ_F16, CQ_BF16, CQ_F32 = 0, 1, 2
 CQ_KEYS, CQ_VALUES = 0, 1
 CQ_PACK_INT4, CQ_PACK_DENSE = 0, 1
+CQ_WORKSPACE_ZERO_BYTES = 7 << 18
 
 _DTYPES = {torch.float16: CQ_F16, torch.bfloat16: CQ_BF16, torch.float32: CQ_F32}
 

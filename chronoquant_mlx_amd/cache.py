@@ -50,9 +50,6 @@ def _num_pframes(num_tokens: int, stride: int) -> int:
     return num_tokens - _num_keyframes(num_tokens, stride)
 
 
-# The workspace's first 1.75 MiB are the split state that has to start as zeros
-# (include/chronoquant.h); the partials behind it may hold anything.
-_ZERO_REGION = 7 << 18
 _WORKSPACES: dict = {}
 # Workspaces replaced by larger ones.  A captured HIP graph keeps the address
 # it was captured with, so a replaced workspace is never freed.
@@ -84,8 +81,10 @@ def _shared_workspace(device: torch.device, nbytes: int) -> torch.Tensor:
     ws = table.get(key)
     if ws is None or ws.numel() < nbytes:
         old = 0 if ws is None else ws.numel()
-        new = torch.empty(max(nbytes, _ZERO_REGION, 2 * old), dtype=torch.uint8, device=device)
-        new[:_ZERO_REGION].zero_()
+        # the partials behind the split state may hold anything
+        zeros = _lib.CQ_WORKSPACE_ZERO_BYTES
+        new = torch.empty(max(nbytes, zeros, 2 * old), dtype=torch.uint8, device=device)
+        new[:zeros].zero_()
         if ws is not None:
             _RETIRED.append(ws)
         table[key] = ws = new

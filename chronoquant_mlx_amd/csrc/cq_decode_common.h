@@ -457,6 +457,7 @@ constexpr int kRecUnits = 64;  // 4 heads x 16 groups of 8 dims per (sequence, k
 constexpr int64_t kMaxRecSplits = 512;  // (sequence, kv head, split) triples
 constexpr size_t kRecBytes = (size_t)kMaxRecSplits * kRecUnits * kRecWords * sizeof(uint32_t);
 constexpr size_t kCounterRegion = kCounterBytes + kFlagBytes + kRecBytes;
+static_assert(kCounterRegion == CQ_WORKSPACE_ZERO_BYTES, "callers zero CQ_WORKSPACE_ZERO_BYTES");
 constexpr int64_t kMaxCounters = kCounterBytes / sizeof(uint32_t);
 // The last 256 bytes of the flag area hold the workspace's sticky status
 // word: a split wait that ran out of poll rounds sets kStatusFoldTimeout

@@ -141,13 +141,14 @@ int cq_append_lengths(const cq_cache_desc *cache, const void *keys,
 int cq_reconstruct(const cq_cache_desc *cache, int32_t component,
                    int64_t seq_len, uint16_t *out, cq_stream_t stream);
 
-/* Bytes of workspace cq_decode_attn needs for this shape.  The workspace
- * must be zero-filled once before its first use.  Its first 1.75 MiB hold the
- * split counters (one per sequence x kv head x q-head chunk, at most 16384),
- * split-ready flags and split fold records, which every call returns to
- * zero, so one workspace can be reused — also by calls of other shapes and
- * by cq_prefill_attn — without clearing.  Calls that share a workspace must
+/* Bytes of workspace cq_decode_attn needs for this shape.  Its first
+ * CQ_WORKSPACE_ZERO_BYTES must be zero-filled once before its first use; the
+ * rest may hold anything.  They are the split counters (one per sequence x kv
+ * head x q-head chunk, at most 16384), split-ready flags and split fold
+ * records, which every call returns to zero, so one workspace can be reused —
+ * also by calls of other shapes and by cq_prefill_attn — without clearing.  Calls that share a workspace must
  * be ordered on one stream.  The workspace must be 256-byte aligned. */
+#define CQ_WORKSPACE_ZERO_BYTES (7u << 18)
 size_t cq_decode_workspace_size(int32_t batch, int32_t n_kv_heads,
                                 int32_t n_q_heads, int32_t head_dim,
                                 int64_t max_seq_len);
@@ -251,11 +252,10 @@ int cq_fp16_decode_attn(const uint16_t *k, const uint16_t *v,
  * CQ_BF16 (bf16: q' = bf16(q * bf16(scale)) and fp32 scores, as the
  * reference's bf16 x fp16 promotion computes them; output bf16).
  * q, out: [B][n_q_heads][n_q][128] of q_dtype, 16-byte aligned.
- * workspace: caller-owned, zero-initialised device memory of at least
+ * workspace: caller-owned device memory of at least
  * cq_prefill_workspace_size(...) bytes, 256-byte aligned, for the split-K
- * partials (the kernels leave its counter region zeroed again, so it is
- * reused without clearing; it may be the decode workspace when large
- * enough).  NULL: the key range is not split (slower, same result). */
+ * partials (behind its first CQ_WORKSPACE_ZERO_BYTES, which are not touched:
+ * it may be the decode workspace when large enough).  NULL: the key range is not split (slower, same result). */
 int cq_prefill_attn(const cq_cache_desc *cache, const void *q, int32_t q_dtype,
                     int32_t n_q_heads, int64_t n_q, float scale, int32_t causal,
                     int64_t seq_len, void *out, void *workspace, size_t workspace_bytes,

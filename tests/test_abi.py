@@ -1,6 +1,7 @@
 """The C-ABI library loads and exports every symbol include/chronoquant.h
 declares; argument validation answers without touching a GPU — CPU only."""
 import ctypes
+import re
 import subprocess
 
 import pytest
@@ -54,3 +55,11 @@ def test_descriptor_layout_matches_header():
     assert ctypes.sizeof(_lib.CqComponent) == 56
     assert ctypes.sizeof(_lib.CqCacheDesc) == 128
     assert _lib.CqCacheDesc.k.offset == 16 and _lib.CqCacheDesc.v.offset == 72
+
+
+def test_zeroed_workspace_bytes_match_the_library():
+    # the workspace of one row of 32 dims in one split: the split state, then its (m, l)
+    # and its partial output, a 256-byte piece each
+    assert _lib.load().cq_decode_workspace_size(1, 1, 1, 32, 1) == _lib.CQ_WORKSPACE_ZERO_BYTES + 512
+    define = re.search(r"#define CQ_WORKSPACE_ZERO_BYTES \((\d+)u << (\d+)\)", open(_lib.HEADER).read())
+    assert int(define[1]) << int(define[2]) == _lib.CQ_WORKSPACE_ZERO_BYTES
