@@ -545,7 +545,8 @@ __global__ __launch_bounds__(256) void append_row4_kernel(AppendArgs a) {
 
 // ---------------------------------------------------------------------------
 // cq_append of a prompt or a chunk of one (16-bit tokens, head_dim a multiple of
-// 8, 16-byte aligned rows, at least kBulkTokens new tokens): LPR lanes per row
+// 8, 16-byte aligned rows, at least kBulkTokens new tokens and kBulkWaves waves of the
+// kernels for few rows): LPR lanes per row
 // (the power of two >= D / 8), 8 dims per lane, 64 / LPR consecutive tokens of one
 // (component, sequence, kv head) per wave and pass, kBulkPasses passes whose loads
 // are issued together.
@@ -570,7 +571,17 @@ __global__ __launch_bounds__(256) void append_row4_kernel(AppendArgs a) {
 // per lane); 64 dims 138 -> 13, 4 heads x 256 dims 105 -> 29 (one row per wave);
 // 8 x 32768 x 8 x 128: 693 -> 321 us, 4.3 TB/s.
 // ---------------------------------------------------------------------------
-constexpr int kBulkTokens = 16;
+// A pass covers up to 8 consecutive tokens of one head and a wave four passes, one
+// after the other, so few rows are done sooner by the kernels above, with a wave for
+// each four rows (head_dim 128) or each one.  2 x 8 heads x 128 dims of 96 tokens: 4.3
+// us against 4.8 here (bf16 4.7 and 5.6); the line lies at about 2560 of their waves
+// for either kernel and type (16 sequences x 8 heads x 128 dims, fp16 / bf16: 32 tokens
+// 4.6 and 5.0 / 5.4 and 5.7, 48 tokens 5.2 and 4.9 / 6.3 and 5.8; 8 heads x 64 dims: 128
+// tokens 4.5 and 4.8 / 5.0 and 5.6, 256 tokens 5.3 and 4.8 / 6.0 and 5.6).  Short
+// chunks of many sequences leave most of a workgroup's 64 to 128 tokens empty (64
+// sequences x 8 heads x 128 dims: 16 tokens 6.3 and 7.3 us, 24 tokens 7.3 and 7.1).
+constexpr int kBulkTokens = 24;
+constexpr int64_t kBulkWaves = 2560;
 constexpr int kBulkPasses = 4;
 
 typedef __bf16 bf2v_t __attribute__((ext_vector_type(2)));
@@ -1135,8 +1146,8 @@ int cq_append_lengths(const cq_cache_desc *cache, const void *keys, const int64_
   const bool low = offsets ? cache->k.cap_keyframes * cache->k.stride < (1 << 24) &&
                                  cache->v.cap_keyframes * cache->v.stride < (1 << 24)
                            : offset + n_new < (1 << 24);
-  if ((dtype == CQ_F16 || dtype == CQ_BF16) && a.D % 8 == 0 && n_new >= kBulkTokens && aligned8 &&
-      low && 2 * a.H <= 65535 && a.B <= 65535) {
+  if ((dtype == CQ_F16 || dtype == CQ_BF16) && a.D % 8 == 0 && n_new >= kBulkTokens &&
+      items >= kBulkWaves * (row4 ? 4 : 1) && aligned8 && low && 2 * a.H <= 65535 && a.B <= 65535) {
     if (dtype == CQ_F16) launch_bulk<CQ_F16>(a, s);
     else launch_bulk<CQ_BF16>(a, s);
     return launch_status();

@@ -62,7 +62,12 @@ def test_codes_match_the_oracle(dtype, bits, dz, kind):
     (2, 3, 64, 77, 0, 32, 8, 4, 4, False, False), (1, 2, 128, 130, 33, 5, 1, 3, 2, True, True),
     (2, 1, 256, 40, 20, 48, 24, 2, 3, True, False), (1, 2, 80, 65, 1, 64, 32, 4, 3, True, True),
     (1, 1, 8, 16, 0, 4, 4, 4, 4, False, False), (3, 2, 136, 100, 50, 12, 20, 4, 4, False, True),
-    (1, 2, 72, 17, 0, 16, 16, 4, 4, False, False)])
+    (1, 2, 72, 17, 0, 16, 16, 4, 4, False, False),
+    # rows enough for the chunk kernel
+    (4, 8, 64, 77, 0, 32, 8, 4, 4, False, False), (8, 16, 128, 130, 33, 5, 1, 3, 2, True, True),
+    (2, 16, 256, 60, 20, 48, 24, 2, 3, True, False), (1, 40, 80, 65, 1, 64, 32, 4, 3, True, True),
+    (4, 20, 8, 33, 0, 4, 4, 4, 4, False, False), (3, 20, 136, 100, 50, 12, 20, 4, 4, False, True),
+    (4, 20, 72, 25, 0, 16, 16, 4, 4, False, False)])
 def test_chunks_equal_short_appends(B, H, D, T, first, sk, sv, bk, bv, dense, token_major, dtype):
     from chronoquant_mlx_amd import ChronoQuantCache
     g = torch.Generator(device="cuda")
@@ -84,11 +89,12 @@ def test_chunks_equal_short_appends(B, H, D, T, first, sk, sv, bk, bv, dense, to
         assert torch.equal(a.contiguous().view(view), b.contiguous().view(view)), i
 
 
-def test_device_positions():
+@pytest.mark.parametrize("H", [2, 64])
+def test_device_positions(H):
     # a chunk at per-sequence device offsets, one of them running past the
     # capacity: its rows past the end are dropped, the others unharmed
     from chronoquant_mlx_amd import ChronoQuantCache
-    B, H, D, T, L = 3, 2, 128, 256, 32
+    B, D, T, L = 3, 128, 256, 32
     g = torch.Generator(device="cuda")
     g.manual_seed(5)
     base, new = (torch.cumsum(torch.randn(B, H, n, D, device="cuda", generator=g) * 0.2, 2).half() for n in (T, L))
@@ -114,7 +120,7 @@ def test_device_positions():
             assert torch.equal(x[b].contiguous().view(view), y[0].contiguous().view(view)), (b, i)
 
 
-@pytest.mark.parametrize("D,S,layout", [(128, 1, "plain"), (72, 1, "plain"), (128, 16, "plain"),
+@pytest.mark.parametrize("D,S,layout", [(128, 1, "plain"), (72, 1, "plain"), (128, 16, "plain"), (128, 1000, "plain"),
                                         (128, 1, "strided"), (128, 1, "beside"), (128, 1, "longer")])
 def test_lengths_stored_by_the_append(D, S, layout):
     # one-row kernels, the four-row one and the chunk one; length vectors that the
