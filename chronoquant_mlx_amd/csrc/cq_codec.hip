@@ -585,6 +585,7 @@ constexpr int64_t kBulkWaves = 2560;
 constexpr int kBulkPasses = 4;
 
 typedef __bf16 bf2v_t __attribute__((ext_vector_type(2)));
+typedef unsigned short us2_t __attribute__((ext_vector_type(2)));
 typedef float fl2_t __attribute__((ext_vector_type(2)));
 
 // maximum over the LPR lanes of a row (NaN-propagating)
@@ -862,6 +863,7 @@ struct RebuildArgs {
   uint16_t *out[2];
   float inv_stride[2];
   int BH, D, T, row_dims;
+  uint32_t *top[2];  // optional: the largest |value| of each (bh, blockIdx.x), as fp16 bits
 };
 
 // head_dim a multiple of 8, 16-byte aligned rows, T < 2^24: one thread per 8
@@ -870,44 +872,61 @@ struct RebuildArgs {
 // (One thread per 8 dims with eight 2-byte loads and stores and 64-bit
 // divisions took 17-18.5 us for one component of 8192 tokens, 4 heads x 256
 // dims; both take 11 together now, 3.7 TB/s.)
-template <int PR>
+template <int PR, bool Top>
 __global__ __launch_bounds__(256) void rebuild_kernel(RebuildArgs a) {
   const int ci = blockIdx.z;
   const cq_component &c = a.comp[ci];
   const int pr = PR ? PR : a.row_dims / 8;
-  const int i = (int)(blockIdx.x * 256 + threadIdx.x);
-  const int t = i / pr, w = i - t * pr;
-  if (t >= a.T) return;
   const int stride = c.stride;
-  int g = (int)((float)t * a.inv_stride[ci]);  // off by at most one
-  int r = t - g * stride;
-  if (r < 0) --g, r += stride;
-  else if (r >= stride) ++g, r -= stride;
   const int fb = field_bits(c), rw = row_words_of(a.D, fb);
   uint32_t magic;  // fp16 1024 in both halves
   asm volatile("v_mov_b32 %0, 0x64006400" : "=v"(magic));
   for (int bh = blockIdx.y; bh < a.BH; bh += gridDim.y) {
-    uint4 x = uint4{0u, 0u, 0u, 0u};
-    if (8 * w < a.D) {
-      x = *(const uint4 *)(c.keyframes + ((int64_t)bh * c.cap_keyframes + g) * a.D + 8 * w);
-      uint32_t word = 0x88888888u, s = 0u;  // an I-frame: + 0
-      if (r != 0) {
-        const int64_t slot = (int64_t)bh * c.cap_pframes + (t - g - 1);
-        const uint32_t *row = c.packed + slot * rw;
-        s = c.scales[slot];
-        if (fb == 4) {
-          word = row[w];
-        } else {  // dense fields to nibbles of the same codes
-          const uint32_t f8 = stream_bits(row, rw, 8 * fb * w, 8 * fb);
-          const uint32_t m = (1u << fb) - 1u, up = 8u - (1u << (fb - 1));
-          word = 0;
+    us2_t top = {0, 0};
+    for (int i = (int)(blockIdx.x * 256 + threadIdx.x); i < a.T * pr; i += (int)gridDim.x * 256) {
+      const int t = i / pr, w = i - t * pr;
+      int g = (int)((float)t * a.inv_stride[ci]);  // off by at most one
+      int r = t - g * stride;
+      if (r < 0) --g, r += stride;
+      else if (r >= stride) ++g, r -= stride;
+      uint4 x = uint4{0u, 0u, 0u, 0u};
+      if (8 * w < a.D) {
+        x = *(const uint4 *)(c.keyframes + ((int64_t)bh * c.cap_keyframes + g) * a.D + 8 * w);
+        uint32_t word = 0x88888888u, s = 0u;  // an I-frame: + 0
+        if (r != 0) {
+          const int64_t slot = (int64_t)bh * c.cap_pframes + (t - g - 1);
+          const uint32_t *row = c.packed + slot * rw;
+          s = c.scales[slot];
+          if (fb == 4) {
+            word = row[w];
+          } else {  // dense fields to nibbles of the same codes
+            const uint32_t f8 = stream_bits(row, rw, 8 * fb * w, 8 * fb);
+            const uint32_t m = (1u << fb) - 1u, up = 8u - (1u << (fb - 1));
+            word = 0;
 #pragma unroll
-          for (int k = 0; k < 8; ++k) word |= (((f8 >> (fb * k)) & m) + up) << (4 * k);
+            for (int k = 0; k < 8; ++k) word |= (((f8 >> (fb * k)) & m) + up) << (4 * k);
+          }
         }
+        x = rebuild8(word, x, s, magic);
       }
-      x = rebuild8(word, x, s, magic);
+      *(uint4 *)(a.out[ci] + ((int64_t)bh * a.T + t) * (8 * pr) + 8 * w) = x;
+      if constexpr (Top) {
+        const uint32_t v[4] = {x.x, x.y, x.z, x.w};
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+          top = __builtin_elementwise_max(top, __builtin_bit_cast(us2_t, v[k] & 0x7fff7fffu));
+      }
     }
-    *(uint4 *)(a.out[ci] + ((int64_t)bh * a.T + t) * (8 * pr) + 8 * w) = x;
+    if constexpr (Top) {
+      __shared__ float s_top[4];
+      const float m = wave_max((float)max(top.x, top.y));
+      if ((threadIdx.x & 63) == 0) s_top[threadIdx.x >> 6] = m;
+      __syncthreads();
+      if (threadIdx.x == 0)
+        a.top[ci][(int64_t)bh * gridDim.x + blockIdx.x] =
+            (uint32_t)fmaxf(fmaxf(s_top[0], s_top[1]), fmaxf(s_top[2], s_top[3]));
+      __syncthreads();
+    }
   }
 }
 
@@ -991,25 +1010,29 @@ static bool rebuild_ok(const cq_component &c, int D, int64_t T, const void *out)
   return D % 8 == 0 && T < (1 << 24) && (((uintptr_t)c.keyframes | (uintptr_t)out) & 15) == 0;
 }
 
-static void launch_rebuild(RebuildArgs &a, int components, hipStream_t s) {
+template <bool Top>
+static void launch_rebuild(RebuildArgs &a, int components, int groups, hipStream_t s) {
   for (int i = 0; i < components; ++i) a.inv_stride[i] = 1.0f / (float)a.comp[i].stride;
-  const int pr = a.row_dims / 8;
-  const dim3 grid((unsigned)(((int64_t)a.T * pr + 255) / 256), (unsigned)std::min(a.BH, 65535),
-                  (unsigned)components), blk(256);
-  switch (pr) {
-    case 8: rebuild_kernel<8><<<grid, blk, 0, s>>>(a); break;
-    case 12: rebuild_kernel<12><<<grid, blk, 0, s>>>(a); break;
-    case 16: rebuild_kernel<16><<<grid, blk, 0, s>>>(a); break;
-    case 32: rebuild_kernel<32><<<grid, blk, 0, s>>>(a); break;
-    default: rebuild_kernel<0><<<grid, blk, 0, s>>>(a); break;
+  const dim3 grid((unsigned)groups, (unsigned)std::min(a.BH, 65535), (unsigned)components), blk(256);
+  switch (a.row_dims / 8) {
+    case 8: rebuild_kernel<8, Top><<<grid, blk, 0, s>>>(a); break;
+    case 12: rebuild_kernel<12, Top><<<grid, blk, 0, s>>>(a); break;
+    case 16: rebuild_kernel<16, Top><<<grid, blk, 0, s>>>(a); break;
+    case 32: rebuild_kernel<32, Top><<<grid, blk, 0, s>>>(a); break;
+    default: rebuild_kernel<0, Top><<<grid, blk, 0, s>>>(a); break;
   }
 }
 
+// Workgroups of one (component, sequence, kv head): a token's 8 dims per thread,
+// several of them where the tops are wanted and would be more than kMaxTops.
+static int rebuild_groups(int64_t T, int row_dims) { return (int)((T * (row_dims / 8) + 255) / 256); }
+int rebuild_tops(int64_t T, int row_dims) { return std::min(rebuild_groups(T, row_dims), kMaxTops); }
+
 int launch_rebuild(const cq_cache_desc &c, int64_t T, int row_dims, uint16_t *k, uint16_t *v,
-                   hipStream_t s) {
+                   uint32_t *top_k, uint32_t *top_v, hipStream_t s) {
   if (!rebuild_ok(c.k, c.head_dim, T, k) || !rebuild_ok(c.v, c.head_dim, T, v)) return CQ_ERR_ALIGN;
-  RebuildArgs a{{c.k, c.v}, {k, v}, {}, c.batch * c.n_kv_heads, c.head_dim, (int)T, row_dims};
-  launch_rebuild(a, 2, s);
+  RebuildArgs a{{c.k, c.v}, {k, v}, {}, c.batch * c.n_kv_heads, c.head_dim, (int)T, row_dims, {top_k, top_v}};
+  launch_rebuild<true>(a, 2, rebuild_tops(T, row_dims), s);
   return launch_status();
 }
 
@@ -1241,8 +1264,8 @@ int cq_reconstruct(const cq_cache_desc *cache, int32_t component, int64_t seq_le
     return CQ_ERR_CAPACITY;
   const int D = cache->head_dim, W = (D + 7) / 8;
   if (rebuild_ok(c, D, seq_len, out)) {
-    RebuildArgs a{{c, c}, {out, out}, {}, cache->batch * cache->n_kv_heads, D, (int)seq_len, D};
-    launch_rebuild(a, 1, (hipStream_t)stream);
+    RebuildArgs a{{c, c}, {out, out}, {}, cache->batch * cache->n_kv_heads, D, (int)seq_len, D, {}};
+    launch_rebuild<false>(a, 1, rebuild_groups(seq_len, D), (hipStream_t)stream);
     return launch_status();
   }
   const int64_t total = (int64_t)cache->batch * cache->n_kv_heads * seq_len * W;

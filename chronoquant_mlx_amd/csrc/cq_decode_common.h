@@ -17,13 +17,17 @@ namespace cq {
 int validate_cache(const cq_cache_desc *c);
 // log-sum-exp merge of split partials [row][nsplit] into rows of D fp16 / bf16
 // values (cq_flash.hip)
+// (empty: the output of a row whose weights sum to 0)
 void launch_combine(bool bf16, const float *part_ml, const float *part_acc, uint16_t *out,
-                    int64_t rows, int D, int nsplit, hipStream_t s);
+                    int64_t rows, int D, int nsplit, float empty, hipStream_t s);
 int64_t num_keyframes(int64_t n, int stride);
 int64_t num_pframes(int64_t n, int stride);
-// K and V of T tokens as fp16 rows of row_dims dims (cq_codec.hip)
+// K and V of T tokens as fp16 rows of row_dims dims, and for each (sequence, kv head)
+// rebuild_tops(T, row_dims) <= kMaxTops numbers whose maximum is the largest |value|
+// of its rows as fp16 bits (cq_codec.hip)
+int rebuild_tops(int64_t T, int row_dims);
 int launch_rebuild(const cq_cache_desc &c, int64_t T, int row_dims, uint16_t *k, uint16_t *v,
-                   hipStream_t s);
+                   uint32_t *top_k, uint32_t *top_v, hipStream_t s);
 
 constexpr int kMaxSplits = 1024;
 constexpr int kThreadsMfma = 512;   // 8 waves per MFMA workgroup

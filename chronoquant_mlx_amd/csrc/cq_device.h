@@ -43,6 +43,7 @@ __device__ __forceinline__ uint32_t code_field(int code, int fb) {
 // ---------------------------------------------------------------------------
 // Rebuilt rows
 // ---------------------------------------------------------------------------
+constexpr int kMaxTops = 512;  // partial maxima of a (sequence, kv head)'s rebuilt rows
 // One code word (8 nibbles, dims 0..7 of a group) and the group's fp16
 // anchor (a01, a23, a45, a67) -> the rebuilt fp16 values in dim order:
 // fp16(a + fp16(fp16(n - 8) * s)).  The low and high nibbles of the bytes

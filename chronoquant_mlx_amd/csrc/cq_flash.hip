@@ -50,6 +50,10 @@ struct Weights {
   static constexpr float kTau = Bf16 ? 1.f : 8.f;
   static constexpr float kLift = Bf16 ? 14.f : 6.f;
 };
+// Scores of at least -kSafe leave a hidden key, at the type's lowest value, the weight
+// 0 (fp16: 104 nats and the scores' rounding above -65504).
+template <bool Bf16>
+constexpr float kSafe = Bf16 ? 1e38f : 65000.f;
 constexpr float kFull = 0.25f;         // a weight whose fp16 pair hi + lo holds 23 bits
 constexpr float kUp = 274877906944.f;  // 2^38: scale of what a pair leaves of a smaller one
 
@@ -66,6 +70,8 @@ struct FlashArgs {
   int B, H, G, nq, D, L, T;
   int causal;
   float scale;
+  const uint32_t *top_k, *top_v;  // [B * H][ntop]: largest |K| and |V| (launch_rebuild)
+  int ntop;
   int nsplit, tiles;
   float *part_ml;   // [row][nsplit][2]  (m in log2 units, l)
   float *part_acc;  // [row][nsplit][D]
@@ -107,8 +113,9 @@ __device__ __forceinline__ int swz_v(int p, int key) {
 
 // Key blocks that a 256-row tile of a boolean mask sees, as a list (its length
 // first), so that the flash kernel passes over the hidden ones: a hidden key's
-// weight is exactly 0 beside any visible one.  A tile with a row that sees no key
-// lists every block (such a row weighs all keys alike).
+// weight is exactly 0 beside any visible one whose score is not near the lowest value
+// itself (kSafe).  A tile with a row that sees no key lists every block (such a row
+// weighs all keys alike).
 // scan_mask_kernel: a workgroup per 1024 keys and 64 rows of a tile, lane = 16 keys,
 // the rows dealt to its 4 waves; masks that do not depend on the q head are read once per
 // position, and once for all kv heads when they do not depend on those.  It leaves
@@ -210,6 +217,7 @@ struct alignas(16) FlashLds {
   static constexpr int kQSteps = DP > 128 ? DP / 16 - 6 : 0;
   uint16_t k[2][kKeys * DP], v[2][kKeys * DP];
   uint4 q[kThreads / 64][kQSteps ? kQSteps : 1][kQSteps ? 64 : 1];
+  float top[3][kThreads / 64];  // largest sum of |q'|, |K| and |V| by wave
 };
 
 // Rows R = tile * 256 + 32 wave + (lane & 31) of the G * L rows of kv head
@@ -261,11 +269,21 @@ void flash_kernel(FlashArgs a) {
   const int pos = rr / G, head = rr - pos * G;
   const int64_t grow = ((int64_t)b * a.nq + h * G + head) * L + pos;
 
+  // the rows' largest |K| and |V|, wanted further down
+  const bool checked = Masked || Bf16 || a.causal;
+  float top_k = 0.f, top_v = 0.f;
+  if (checked && tid < a.ntop) {
+    top_k = (float)a.top_k[(int64_t)bh * a.ntop + tid];
+    top_v = (float)a.top_v[(int64_t)bh * a.ntop + tid];
+  }
+
   // ---- q' (B operand of the score product): dims 16s + 8 half .. + 7 ---------
   // bf16: scaled by a power of two that brings the row's largest magnitude to
   // [2^13, 2^14), so that its fp16 form loses no bit down to 2^-31 of that;
   // cs takes the scores back, in log2 units.  low: a row of this wave has elements
   // that lose bits (a block's score products then begin with theirs).
+  // sum: of the magnitudes of this half of the row.
+  float sum = 0.f;
   h8_t qf[NR];
   float cs = kLog2e;
   bool low = false;
@@ -312,26 +330,55 @@ void flash_kernel(FlashArgs a) {
           const float x = scaled(u, e, f);
           v[e] = (_Float16)x;
           left = fmaxf(left, fabsf(lost(x)));
+          sum += fabsf(x);
         }
         keep(s, v);
       }
       low = __any(left > 0.f);
+      sum *= __uint_as_float((uint32_t)(127 - up) << 23);
     } else {
 #pragma unroll
-      for (int s = 0; s < NS; ++s) keep(s, __builtin_bit_cast(h8_t, raw_of(s)) * (_Float16)a.scale);
+      for (int s = 0; s < NS; ++s) {
+        const h8_t v = __builtin_bit_cast(h8_t, raw_of(s)) * (_Float16)a.scale;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) sum += fabsf((float)v[e]);
+        keep(s, v);
+      }
     }
   }
+
+  // ---- may hidden keys be passed over? ---------------------------------------------
+  // A score is at least -sum |q'| max |K|.  Where that is not above the lowest value
+  // by enough (unsafe), or V holds an infinity or NaN (vbad; 0 times it is NaN),
+  // hidden keys are computed like any other.  (One word of each maximum per thread and
+  // a barrier: 2 us of the shapes above, and 1 us of the rebuild that leaves them.)
+  bool unsafe = false, vbad = false;
+  if (checked) {
+    sum = xor32_sum(sum);
+    const float ms = wave_max(sum == sum ? sum : INFINITY), mk = wave_max(top_k), mv = wave_max(top_v);
+    if (lane == 0) lds.top[0][wave] = ms, lds.top[1][wave] = mk, lds.top[2][wave] = mv;
+    __syncthreads();
+    float m[3] = {0.f, 0.f, 0.f};
+#pragma unroll
+    for (int i = 0; i < kThreads / 64; ++i)
+#pragma unroll
+      for (int j = 0; j < 3; ++j) m[j] = fmaxf(m[j], lds.top[j][i]);
+    vbad = __builtin_amdgcn_readfirstlane((int)m[2]) >= 0x7c00;
+    const float bound = m[0] * h2f((uint16_t)m[1]);
+    unsafe = vbad || __builtin_amdgcn_readfirstlane(!(bound < kSafe<Bf16>));  // (NaN: not safe)
+  }
+  const float low_score = Bf16 ? -1.7e38f : -65504.f;
 
   // ---- key range ----------------------------------------------------------------
   const int qbase = T - L;
   const int lim = a.causal ? qbase + pos : T - 1;           // last key this row sees
   const int lim_all = a.causal ? qbase + row0 / G : T - 1;  // ... every row sees
   const int last = min(row0 + kRows, GL) - 1;
-  const int key_end = a.causal ? qbase + last / G + 1 : T;
+  const int key_end = a.causal && !unsafe ? qbase + last / G + 1 : T;
   // blocks in the order they are taken: all up to key_end, or the tile's list
   const int32_t *list = nullptr;
   if constexpr (Masked) {
-    if (a.blocks)
+    if (a.blocks && !unsafe)
       list = a.blocks + ((int64_t)(a.planes == 1 ? 0 : bh) * a.tiles + tile) * (1 + a.nblk);
   }
   const int n_all = list ? __builtin_amdgcn_readfirstlane(list[0]) : (key_end + KT - 1) / KT;
@@ -478,20 +525,24 @@ void flash_kernel(FlashArgs a) {
     if constexpr (Masked) {
       // hidden keys take the lowest finite value (a row that sees no key
       // weighs all of them alike); -inf is for keys past the end
-      const float low = Bf16 ? -1.7e38f : -65504.f;
 #pragma unroll
       for (int kt = 0; kt < NK; ++kt)
 #pragma unroll
         for (int r = 0; r < 16; ++r)
-          if (!((mb[kt][r >> 2] >> (8 * (r & 3))) & 0xffu)) put(kt, r, low);
+          if (!((mb[kt][r >> 2] >> (8 * (r & 3))) & 0xffu)) put(kt, r, low_score);
     }
-    if (k0 + KT - 1 > lim_all) {  // uniform: only a tile's last blocks
+    auto past = [&](int end, float x) {  // keys beyond a row's end
 #pragma unroll
       for (int kt = 0; kt < NK; ++kt)
 #pragma unroll
         for (int r = 0; r < 16; ++r)
-          if (k0 + 32 * kt + 8 * (r >> 2) + 4 * half + (r & 3) > lim) put(kt, r, -INFINITY);
+          if (k0 + 32 * kt + 8 * (r >> 2) + 4 * half + (r & 3) > end) put(kt, r, x);
+    };
+    // (uniform: only a tile's last blocks)
+    if constexpr (!Masked) {
+      if (k0 + KT - 1 > lim_all) past(lim, unsafe ? low_score : -INFINITY);
     }
+    if (k0 + KT > T) past(T - 1, -INFINITY);
     float mx;
     if constexpr (Bf16) {
       mx = sc[0][0];
@@ -654,7 +705,8 @@ void flash_kernel(FlashArgs a) {
       }
     return;
   }
-  const float inv = l_run > 0.f ? 1.f / l_run : (l_run == 0.f ? 0.f : l_run);
+  // (scores of -inf alone: NaN, as the fallback's softmax gives)
+  const float inv = l_run > 0.f ? 1.f / l_run : NAN;
   uint16_t *o = a.out + grow * a.D;
 #pragma unroll
   for (int dt = 0; dt < ND; ++dt)
@@ -677,7 +729,8 @@ void flash_kernel(FlashArgs a) {
 // partials once.
 template <bool Bf16>
 __global__ __launch_bounds__(256) void combine_kernel(const float *part_ml, const float *part_acc,
-                                                      uint16_t *out, int D, int nsplit, int64_t n) {
+                                                      uint16_t *out, int D, int nsplit, float empty,
+                                                      int64_t n) {
   const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (i >= n) return;
   const int d4 = D / 4;
@@ -700,7 +753,7 @@ __global__ __launch_bounds__(256) void combine_kernel(const float *part_ml, cons
     o.z += w * v.z;
     o.w += w * v.w;
   }
-  const float inv = Ls > 0.f ? 1.f / Ls : (Ls == 0.f ? 0.f : Ls);
+  const float inv = Ls > 0.f ? 1.f / Ls : (Ls == 0.f ? empty : Ls);
   const float ov[4] = {o.x * inv, o.y * inv, o.z * inv, o.w * inv};
   uint16_t w[4];
 #pragma unroll
@@ -717,8 +770,9 @@ int padded_dim(int D) { return D <= 64 ? 64 : D <= 96 ? 96 : D <= 128 ? 128 : 25
 struct FlashPlan {
   int dp, tiles, nsplit;
   int nblk, chunks;
-  size_t kv, ml, acc, lists;  // bytes: K (and V) rows, partial (m, l), partial o, block lists
-  size_t bytes() const { return 2 * kv + ml + acc + lists; }
+  int ntop;
+  size_t kv, ml, acc, lists, tops;  // bytes: K (and V) rows, partial (m, l), partial o, block lists, tops
+  size_t bytes() const { return 2 * kv + ml + acc + lists + tops; }
 };
 
 constexpr int kMaxFlashSplits = 32;
@@ -750,6 +804,8 @@ FlashPlan flash_plan(int64_t B, int64_t H, int64_t G, int64_t D, int64_t L, int6
   p.lists = (size_t)(B * H * p.tiles) *
             ((1 + blocks) * 4 + chunks * (kScanGroups * kScanKeys / keys + kRows));  // lists, blk, row
   p.lists = p.lists <= kMaxListBytes ? round256(p.lists) : 0;
+  p.ntop = rebuild_tops(T, p.dp);
+  p.tops = round256((size_t)(2 * B * H * p.ntop) * 4);
   p.ml = best > 1 ? round256(rows * best * 8) : 0;
   p.acc = best > 1 ? round256(rows * best * D * 4) : 0;
   return p;
@@ -785,11 +841,11 @@ void launch_flash(const FlashArgs &a, int dp, bool masked, dim3 grid, hipStream_
 }  // namespace
 
 void launch_combine(bool bf16, const float *part_ml, const float *part_acc, uint16_t *out,
-                    int64_t rows, int D, int nsplit, hipStream_t s) {
+                    int64_t rows, int D, int nsplit, float empty, hipStream_t s) {
   const int64_t n = rows * (D / 4);
   const dim3 grid((unsigned)((n + 255) / 256)), blk(256);
-  if (bf16) combine_kernel<true><<<grid, blk, 0, s>>>(part_ml, part_acc, out, D, nsplit, n);
-  else combine_kernel<false><<<grid, blk, 0, s>>>(part_ml, part_acc, out, D, nsplit, n);
+  if (bf16) combine_kernel<true><<<grid, blk, 0, s>>>(part_ml, part_acc, out, D, nsplit, empty, n);
+  else combine_kernel<false><<<grid, blk, 0, s>>>(part_ml, part_acc, out, D, nsplit, empty, n);
 }
 
 }  // namespace cq
@@ -861,7 +917,12 @@ extern "C" int cq_flash_attn(const cq_cache_desc *cache, const void *q, int32_t 
     scan_mask_kernel<<<dim3((unsigned)(p.chunks * kScanGroups), (unsigned)p.tiles, (unsigned)a.planes), dim3(256), 0, s>>>(a, m);
     list_kernel<<<dim3((unsigned)p.tiles, (unsigned)a.planes), dim3(64), 0, s>>>(a, m);
   }
-  st = launch_rebuild(*cache, seq_len, p.dp, (uint16_t *)w, (uint16_t *)(w + p.kv), s);
+  uint32_t *tops = (uint32_t *)(w + 2 * p.kv + p.ml + p.acc + p.lists);
+  a.ntop = p.ntop;
+  a.top_k = tops;
+  a.top_v = tops + (int64_t)a.B * a.H * p.ntop;
+  st = launch_rebuild(*cache, seq_len, p.dp, (uint16_t *)w, (uint16_t *)(w + p.kv), tops,
+                      tops + (int64_t)a.B * a.H * p.ntop, s);
   if (st) return st;
   const dim3 grid((unsigned)(p.tiles * a.B * a.H * p.nsplit));
   const bool masked = mask_kind == kMaskBool;
@@ -869,6 +930,6 @@ extern "C" int cq_flash_attn(const cq_cache_desc *cache, const void *q, int32_t 
   else launch_flash<false>(a, p.dp, masked, grid, s);
   if (p.nsplit > 1)
     launch_combine(q_dtype == CQ_BF16, a.part_ml, a.part_acc, a.out, (int64_t)a.B * a.nq * a.L, a.D,
-                   p.nsplit, s);
+                   p.nsplit, NAN, s);
   return hipGetLastError() == hipSuccess ? CQ_OK : CQ_ERR_LAUNCH;
 }

@@ -597,6 +597,6 @@ extern "C" int cq_prefill_attn(const cq_cache_desc *cache, const void *q, int32_
   }
   if (a.nsplit > 1)
     launch_combine(q_dtype == CQ_BF16, a.part_ml, a.part_acc, a.out, (int64_t)a.B * a.nq * a.n_q, kD,
-                   a.nsplit, s);
+                   a.nsplit, 0.f, s);
   return hipGetLastError() == hipSuccess ? CQ_OK : CQ_ERR_LAUNCH;
 }

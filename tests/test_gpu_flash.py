@@ -222,3 +222,61 @@ def test_flash_masks_under_vmap():
     for i in range(3):
         ref = chronoquant_sdpa(q, None, None, cache, 0.125, masks[i])
         assert_close(out[i].float().cpu().numpy(), ref.float().cpu().numpy())
+
+
+def _both(q, cache, scale, mask):
+    from chronoquant_mlx_amd import chronoquant_sdpa, kernels
+    from chronoquant_mlx_amd import attention as A
+    got = kernels.chronoquant_flash_kernel(q, cache, scale, mask)
+    A.PREFILL_KERNEL = False
+    try:
+        ref = chronoquant_sdpa(q, None, None, cache, scale, mask)
+    finally:
+        A.PREFILL_KERNEL = True
+    return got.float().cpu().numpy(), ref.float().cpu().numpy()
+
+
+@pytest.mark.parametrize("D,T", [(64, 300), (128, 700), (256, 300)])
+@pytest.mark.parametrize("peak", [224.0, 255.8, 300.0])
+@pytest.mark.parametrize("kind", ["causal", "window", "half"])
+def test_flash_scores_at_the_lowest_value(kind, peak, D, T):
+    # fp16 scores of the visible keys about peak^2 below 0: clear of fp16's lowest
+    # value, which hidden keys' scores have, next to it, and past it (-inf), where the
+    # hidden keys take the weight.  Rows that see every key at -inf are NaN.  (window
+    # and half hide whole key blocks.)
+    L = 40
+    rng = np.random.default_rng(D)
+    k = np.zeros((1, 2, T, D))
+    k[..., 0] = peak + 0.125 * rng.integers(-1, 2, size=(1, 2, T))
+    cache = build_gpu_cache(k, _stream(rng, 1, 2, T, D), stride_k=1, stride_v=8)
+    q = torch.zeros(1, 4, L, D, dtype=torch.float16, device="cuda")
+    q[..., 0] = -peak
+    i, t = torch.arange(T - L, T, device="cuda")[:, None], torch.arange(T, device="cuda")[None]
+    mask = {"causal": "causal", "window": (i >= t) & (i < t + 90), "half": (t >= T // 2) & (i >= -t)}[kind]
+    if D == 128 and kind == "causal":
+        mask = i >= t  # (the string takes the head_dim-128 kernel in chronoquant_sdpa)
+    got, ref = _both(q, cache, 1.0, mask)
+    assert np.array_equal(np.isnan(got), np.isnan(ref))
+    assert_close(np.nan_to_num(got), np.nan_to_num(ref))
+
+
+@pytest.mark.parametrize("dtype", [torch.float16])
+@pytest.mark.parametrize("D", [64, 80, 256])
+@pytest.mark.parametrize("mask", [None, "causal", "window"])
+def test_flash_infinite_values_like_the_fallback(mask, D, dtype):
+    # V past fp16's range at an anchor (infinite) of some keys: +-inf where a row gives
+    # it weight, NaN where the weight is 0 (a hidden key) or the signs differ, and the
+    # other dims as ever.  Few keys, so that no weight rounds to 0.
+    T, L = 150, 70
+    rng = np.random.default_rng(D)
+    k, v = (to_gpu(0.3 * rng.standard_normal((1, 2, T, D)), torch.bfloat16) for _ in range(2))
+    v[0, 0, 148, 3], v[0, 0, 64, 5], v[0, 1, 4, 6], v[0, 1, 140, 6] = 3e38, -3e38, 3e38, -3e38
+    cache = build_gpu_cache(k.float().cpu().numpy(), v.float().cpu().numpy(), stride_k=4, stride_v=1,
+                            dtype=torch.bfloat16)
+    q = to_gpu(0.3 * rng.standard_normal((1, 8, L, D)), dtype)
+    i, t = torch.arange(T - L, T, device="cuda")[:, None], torch.arange(T, device="cuda")[None]
+    got, ref = _both(q, cache, D ** -0.5, (i >= t) & (i < t + 30) if mask == "window" else mask)
+    assert np.isnan(ref).any() and (mask == "window" or np.isinf(ref).any())
+    fin = np.isfinite(ref)
+    assert np.array_equal(got[~fin], ref[~fin], equal_nan=True)
+    assert_close(got[fin], ref[fin])
