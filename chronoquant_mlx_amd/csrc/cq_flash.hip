@@ -93,6 +93,14 @@ __device__ __forceinline__ uint2 lds_read_tr16(const uint16_t *p) {
   return __builtin_bit_cast(uint2, v);
 }
 
+__device__ __forceinline__ h8_t finite_or_0(h8_t v) {
+  uint4 u = __builtin_bit_cast(uint4, v);
+  auto f = [](uint32_t w) {
+    return ((w & 0x7c00u) == 0x7c00u ? 0u : w & 0xffffu) | ((w & 0x7c000000u) == 0x7c000000u ? 0u : w & 0xffff0000u);
+  };
+  return __builtin_bit_cast(h8_t, uint4{f(u.x), f(u.y), f(u.z), f(u.w)});
+}
+
 // 16-byte piece p of block row `key` sits in slot swz(p, key) of the row.  K
 // rows are read by 8 or 16 lanes of consecutive keys at one piece: the low key
 // bits spread them over the banks.  V rows are read four consecutive keys x 64
@@ -232,11 +240,11 @@ struct alignas(16) FlashLds {
 // clock as long as the products), then the softmax's VALU.  512 queries of 16
 // heads over 8192 keys of 4 heads, head_dim 256, bf16 (66.6 GFLOP, and half as
 // many again for the weights' low halves), with the rebuild (11) and the merge
-// (12): 157 us where few scores lie 11 nats below their row's maximum (below), 193
-// with outlier channels in the keys, 273 with scores of a spread of 16, where the
-// reconstruct fallback's products, softmax and conversions took 977; fp16 112.  257
-// fp16 queries x 2 sequences under a boolean window over 4001 keys: 59 us in all
-// against 803; bf16 74.
+// (12): 172 us where few scores lie 11 nats below their row's maximum (below), 201
+// with outlier channels in the keys, 280 with scores of a spread of 16, where the
+// reconstruct fallback's products, softmax and conversions took 977; fp16 120.  257
+// fp16 queries x 2 sequences under a boolean window over 4001 keys: 63 us in all
+// against 803; bf16 77.
 //
 // Split weights (bf16 queries): the fallback holds weights in fp32, so P enters
 // as an fp16 pair hi + lo, two products per V operand; a pair holds 23 bits of a
@@ -449,8 +457,12 @@ void flash_kernel(FlashArgs a) {
   int k_first = k_at(0), v_first = v_at(0, 0);
 
   int id = 0, id_next = 0;  // this block's place in the keys, the next one's
-  auto block = [&](int kb, auto buf_c) {
+  // bad_c: V holds infinities or NaN.  They meet the weights' high halves alone (a low
+  // half or a rest may be 0 or of the other sign, where the weight is neither).  (A
+  // loop of its own: 4 us of 197 on the shape above without any such value.)
+  auto block = [&](int kb, auto buf_c, auto bad_c) {
     constexpr int cur = decltype(buf_c)::value;
+    constexpr bool bad = decltype(bad_c)::value;
     const int k0 = id * KT;
     if (kb + 1 < kb_hi) load_block(id_next);  // uniform
     id = id_next;
@@ -597,14 +609,19 @@ void flash_kernel(FlashArgs a) {
         const uint2 v1 = lds_read_tr16(v16 + at);
         const uint2 v2 = lds_read_tr16(v16 + at2);
         const h8_t va = __builtin_bit_cast(h8_t, uint4{v1.x, v1.y, v2.x, v2.y});
-        acc[dt] = mfma(va, bh8, acc[dt]);
-        if constexpr (Bf16) acc[dt] = mfma(va, bl8, acc[dt]);
+        const h8_t vl = bad ? finite_or_0(va) : va;
+        acc[dt] = mfma(bad && tight ? vl : va, bh8, acc[dt]);
+        if constexpr (Bf16) acc[dt] = mfma(vl, bl8, acc[dt]);
         if (tight) __builtin_amdgcn_sched_barrier(0);
       }
     };
     // the fp16 pair of x0, x1; rest: what it leaves of those below kFull
     auto split = [&](float &x0, float &x1, h2_t &hi, h2_t &lo, bool rest) {
       hi = __builtin_convertvector(f2_t{x0, x1}, h2_t);
+      if constexpr (bad) {  // (0 for a weight of 0 alone)
+        if (hi.x == (_Float16)0.f && x0 > 0.f) hi.x = (_Float16)0x1p-24f;
+        if (hi.y == (_Float16)0.f && x1 > 0.f) hi.y = (_Float16)0x1p-24f;
+      }
       const float d0 = x0 - (float)hi.x, d1 = x1 - (float)hi.y;
       lo = __builtin_convertvector(f2_t{d0, d1}, h2_t);
       if (rest) {
@@ -681,11 +698,15 @@ void flash_kernel(FlashArgs a) {
     store_block(0);
   }
   __syncthreads();
-  for (int kb = kb_lo; kb < kb_hi;) {
-    block(kb++, std::integral_constant<int, 0>{});
-    if (kb >= kb_hi) break;
-    block(kb++, std::integral_constant<int, 1>{});
-  }
+  auto run = [&](auto bad_c) {
+    for (int kb = kb_lo; kb < kb_hi;) {
+      block(kb++, std::integral_constant<int, 0>{}, bad_c);
+      if (kb >= kb_hi) break;
+      block(kb++, std::integral_constant<int, 1>{}, bad_c);
+    }
+  };
+  if (Bf16 && vbad) run(std::integral_constant<bool, Bf16>{});
+  else run(std::false_type{});
 
   // ---- output: lane (row, half) holds dims 32 dt + 8 q + 4 half .. + 3 ---------------
   l_run = xor32_sum(l_run);

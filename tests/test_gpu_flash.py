@@ -260,7 +260,7 @@ def test_flash_scores_at_the_lowest_value(kind, peak, D, T):
     assert_close(np.nan_to_num(got), np.nan_to_num(ref))
 
 
-@pytest.mark.parametrize("dtype", [torch.float16])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("D", [64, 80, 256])
 @pytest.mark.parametrize("mask", [None, "causal", "window"])
 def test_flash_infinite_values_like_the_fallback(mask, D, dtype):
