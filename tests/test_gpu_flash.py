@@ -280,3 +280,26 @@ def test_flash_infinite_values_like_the_fallback(mask, D, dtype):
     fin = np.isfinite(ref)
     assert np.array_equal(got[~fin], ref[~fin], equal_nan=True)
     assert_close(got[fin], ref[fin])
+
+
+@pytest.mark.parametrize("dtype,mask", [(torch.float16, "causal"), (torch.bfloat16, "window")])
+def test_flash_splits_over_several_rounds(dtype, mask):
+    # more tiles than CUs and splits all the same, so that the workgroups run in
+    # several rounds; against the fallback, a kv head at a time
+    from chronoquant_mlx_amd import _lib, kernels
+    B, H, G, D, T, L = 1, 8, 4, 64, 8192, 2560
+    g = torch.Generator(device="cuda")
+    g.manual_seed(1)
+    k, v = (torch.cumsum(0.1 * torch.randn(B, H, T, D, device="cuda", generator=g), 2).half() for _ in range(2))
+    q = torch.randn(B, G * H, L, D, device="cuda", generator=g).to(dtype)
+    cache = build_gpu_cache(k.cpu().numpy(), v.cpu().numpy(), stride_k=32, stride_v=8)
+    need = _lib.load().cq_flash_scratch_size(cache._descriptor(), G * H, L, T)
+    assert G * L // 256 * H * B > torch.cuda.get_device_properties(0).multi_processor_count
+    assert need > 2 * B * H * T * D * 2 + 2 * (B * G * H * L) * D * 4  # two splits' partials
+    i, t = torch.arange(T - L, T, device="cuda")[:, None], torch.arange(T, device="cuda")[None]
+    m = (i >= t) & (i < t + 3000) if mask == "window" else mask
+    got = kernels.chronoquant_flash_kernel(q, cache, D ** -0.5, m)
+    for h in range(0, H, 7):
+        part = build_gpu_cache(k[:, h:h + 1].cpu().numpy(), v[:, h:h + 1].cpu().numpy(), stride_k=32, stride_v=8)
+        _, ref = _both(q[:, G * h:G * h + G].contiguous(), part, D ** -0.5, m)
+        assert_close(got[:, G * h:G * h + G].float().cpu().numpy(), ref)

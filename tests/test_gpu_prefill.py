@@ -175,8 +175,30 @@ def test_split_keys_match_single_pass(bf16):
 @pytest.mark.parametrize("B,H,G,T,L", [(1, 8, 4, 2100, 64), (1, 2, 4, 4096, 1), (4, 8, 4, 700, 130),
                                        (1, 1, 1, 2048, 33), (2, 2, 16, 333, 333)])
 def test_split_plans(B, H, G, T, L):
-    # 32 splits of one tile; as many splits as key blocks allow; more tiles than
-    # CUs (one split); a tile with most rows empty; rows of several tiles.  The
-    # second call runs on the first one's leavings in the workspace.
+    # 32 splits of one tile; as many splits as key blocks allow; tiles enough that
+    # splits would not pay (one); a tile with most rows empty; rows of several tiles.
+    # The second call runs on the first one's leavings in the workspace.
     _check(B, H, G, T, L, dict(stride_k=32, stride_v=8), seed=T)
     _check(B, H, G, T, L, dict(stride_k=32, stride_v=8), seed=T + 1)
+
+
+@pytest.mark.parametrize("causal", [True, False])
+def test_splits_over_several_rounds(causal):
+    # more tiles than CUs and splits all the same, so that the workgroups run in
+    # several rounds; against one pass per tile (no workspace)
+    from chronoquant_mlx_amd import _lib
+    D, B, H, G, T, L = 128, 1, 8, 4, 8192, 2560
+    k, v = _data(3, B, H, T, D)
+    cache = build_gpu_cache(k, v, stride_k=32, stride_v=8)
+    q = to_gpu(np.random.default_rng(4).standard_normal((B, G * H, L, D)))
+    tiles = G * L // 256 * H * B
+    need = _lib.load().cq_prefill_workspace_size(B, H, G * H, L, T)
+    assert tiles > torch.cuda.get_device_properties(0).multi_processor_count and need > 0
+    outs = []
+    for n in (need, 0):
+        ws = torch.zeros(n, dtype=torch.uint8, device="cuda") if n else None
+        out = torch.empty_like(q)
+        _lib.call("cq_prefill_attn", cache._descriptor(), q.data_ptr(), _lib.CQ_F16, G * H, L, D ** -0.5,
+                  int(causal), T, out.data_ptr(), _lib.ptr(ws), n, _lib.stream_of(q))
+        outs.append(out.float().cpu().numpy())
+    assert_close(outs[0], outs[1])
