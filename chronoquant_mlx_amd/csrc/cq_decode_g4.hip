@@ -1245,7 +1245,7 @@ int64_t g4_resident() {
                              kSlotG4);
 }
 
-// Residency of the one-chunk instance: with 102 VGPRs and 41 KB of LDS two of
+// Residency of the one-chunk instance: with 99 VGPRs and 41 KB of LDS two of
 // its workgroups share a CU (the pipelined instances: one).
 int64_t g4_one_chunk_resident() {
   return resident_workgroups(reinterpret_cast<const void *>(decode_g4_kernel<false, true>),

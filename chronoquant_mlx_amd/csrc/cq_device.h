@@ -194,15 +194,9 @@ __device__ __forceinline__ float wave_sum(float v) {
   return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 63));
 }
 
-// Over the 16 lanes of a row (the first four steps of wave_max / wave_sum):
-// every lane of the row gets the result, the sum with the same bits in
-// every lane (each step adds a pair of values in either order).
-__device__ __forceinline__ float row16_max(float v) {
-  v = fmaxf(v, dpp_f<kDppQuadXor1>(v));
-  v = fmaxf(v, dpp_f<kDppQuadXor2>(v));
-  v = fmaxf(v, dpp_f<kDppRowHalfMirror>(v));
-  return fmaxf(v, dpp_f<kDppRowMirror>(v));
-}
+// Over the 16 lanes of a row (the first four steps of wave_sum): every lane of
+// the row gets the sum, with the same bits (each step adds a pair of values in
+// either order).
 __device__ __forceinline__ float row16_sum(float v) {
   v += dpp_f<kDppQuadXor1>(v);
   v += dpp_f<kDppQuadXor2>(v);
