@@ -27,8 +27,9 @@
 // partition of cq_plan.h, 512-token units over one resident generation.
 //
 // Bound: the chain of a chunk (loads, two products, softmax) with two waves per
-// SIMD in flight, and the fp32 products (16x16x4: 10000 clocks of a 256-dim chunk,
-// 4x4x1: 2600).  4 sequences of 16001 tokens, 16/4 heads x 256 dims (82 MB): 45 us,
+// SIMD in flight: on the first shape below the VALU is busy for 33 % of the time, the
+// matrix cores for 12 (their fp32 products: 2600 clocks of a 256-dim chunk by 4x4x1,
+// 10000 by 16x16x4), LDS for 6, and the waves wait for 39.  4 sequences of 16001 tokens, 16/4 heads x 256 dims (82 MB): 45 us,
 // 1.8 TB/s, against 370 on the portable kernel (fp32 VALU products, 8 head slots for
 // 4 heads), 35 with the 22-bit pairs and 57 with 16x16x4 products for 4 heads; 8
 // heads per kv head, 16/2: 41 and 28.5 with the pairs; 16 ragged sequences of up to

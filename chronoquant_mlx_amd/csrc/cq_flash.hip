@@ -235,16 +235,16 @@ struct alignas(16) FlashLds {
 // weights never leave their lane; O^T = V^T P^T keeps a row in one lane (and
 // its other half), so the softmax state is per lane.
 //
-// Bound: LDS operand reads and matrix cores together (a wave's 32 rows read the
-// whole block, 2 x KT x DP x 2 bytes for 4 x 32 x KT x DP flops: at 128 bytes a
-// clock as long as the products), then the softmax's VALU.  512 queries of 16
-// heads over 8192 keys of 4 heads, head_dim 256, bf16 (66.6 GFLOP, and half as
-// many again for the weights' low halves), with the rebuild (11) and the merge
-// (12): 172 us where few scores lie 11 nats below their row's maximum (below), 201
-// with outlier channels in the keys, 280 with scores of a spread of 16, where the
-// reconstruct fallback's products, softmax and conversions took 977; fp16 120.  257
-// fp16 queries x 2 sequences under a boolean window over 4001 keys: 63 us in all
-// against 803; bf16 77.
+// Bound: a block's chain (scores, softmax, P.V, a barrier) with two waves per SIMD
+// in flight: on the first shape below the matrix cores are busy for 24 % of the
+// time, the VALU for 35, LDS for 12, without bank conflicts, and the waves wait for
+// 49.  512 queries of 16 heads over 8192 keys of 4 heads, head_dim 256, bf16 (66.6
+// GFLOP, and half as many again for the weights' low halves), with the rebuild (11)
+// and the merge (12): 172 us where few scores lie 11 nats below their row's maximum
+// (below), 201 with outlier channels in the keys, 280 with scores of a spread of 16,
+// where the reconstruct fallback's products, softmax and conversions took 977; fp16
+// 120.  257 fp16 queries x 2 sequences under a boolean window over 4001 keys: 63 us
+// in all against 803; bf16 77.
 //
 // Split weights (bf16 queries): the fallback holds weights in fp32, so P enters
 // as an fp16 pair hi + lo, two products per V operand; a pair holds 23 bits of a
