@@ -16,7 +16,7 @@
 //   us of these times);
 // * P, p*s and the sums P_g stay fp32 numbers of any magnitude: the weighted sums
 //   are fp32 matrix products of them with the codes and anchors as fp32.  (fp16
-//   pairs hi + lo, whose products run 16 times as fast, hold 22 bits down to a
+//   pairs hi + lo, whose products run 16 times as fast, hold 23 bits down to a
 //   fixed step: behind a dominant token whose V is 0 the other tokens' weights were
 //   off by 5e-4 at a gap of 10 nats.)
 //
@@ -26,14 +26,15 @@
 // NU c .. NU c + NU - 1 (NU = 2 beyond 128 dims) of 16 tokens.  Work: the balanced
 // partition of cq_plan.h, 512-token units over one resident generation.
 //
-// Bound: the chain of a chunk (loads, two products, softmax) with two waves per
-// SIMD in flight: on the first shape below the VALU is busy for 33 % of the time, the
+// Bound: the chain of a chunk (loads, two products, softmax) with two waves per SIMD
+// in flight: on the first shape below the VALU is busy for 33 % of the time, the
 // matrix cores for 12 (their fp32 products: 2600 clocks of a 256-dim chunk by 4x4x1,
-// 10000 by 16x16x4), LDS for 6, and the waves wait for 39.  4 sequences of 16001 tokens, 16/4 heads x 256 dims (82 MB): 45 us,
-// 1.8 TB/s, against 370 on the portable kernel (fp32 VALU products, 8 head slots for
-// 4 heads), 35 with the 22-bit pairs and 57 with 16x16x4 products for 4 heads; 8
-// heads per kv head, 16/2: 41 and 28.5 with the pairs; 16 ragged sequences of up to
-// 4096, 32/8 x 64: 41 against 177; one of 1000, 16/4 x 256: 27 against 304.
+// 10000 by 16x16x4), LDS for 6, and the waves wait for 39.  4 sequences of 16001
+// tokens, 16/4 heads x 256 dims (82 MB): 45 us, 1.8 TB/s, against 370 on the
+// portable kernel (fp32 VALU products, 8 head slots for 4 heads), 35 with the pairs
+// and 57 with 16x16x4 products for 4 heads; 8 heads per kv head, 16/2: 41 and 28.5
+// with the pairs; 16 ragged sequences of up to 4096, 32/8 x 64: 41 against 177; one
+// of 1000, 16/4 x 256: 27 against 304.
 // Error of the fp32 output against binary64, mean of 8 seeds of 4000 tokens by head
 // dim: 8.0 to 9.3e-8 relative, the portable kernel 7.4 to 9.1e-8.
 #include <hip/hip_runtime.h>

@@ -271,8 +271,8 @@ size_t cq_prefill_workspace_size(int32_t batch, int32_t n_kv_heads, int32_t n_q_
  * calls cq_prefill_attn declines: any head_dim that is a multiple of 8, dense
  * residual rows, and boolean masks.  The same semantics (the reconstruct
  * fallback of chronoquant_sdpa, reference attention.py:8-20, 61-74 over
- * cache.py:131-160), with bf16 queries' weights kept in 32 bits, as the
- * reference's promotion keeps them.
+ * cache.py:131-160); bf16 queries' weights, fp32 by the reference's promotion,
+ * are held to 23 bits at every size.
  * mask_kind: 0 none; 1 causal (query i sees keys <= seq_len - n_q + i, n_q <=
  * seq_len); 2 a boolean mask, one byte per element (0: hidden), element
  * (sequence, kv head, q head of the group, query, key) at the element strides
